@@ -522,7 +522,6 @@ static int ensure_chunk(fh_reconstructor *h, int n, int B)
 // Larger chunks put more slices into each work item, so fewer partial
 // bricks are written and merged per particle.
 constexpr long long AUTO_CHUNK_BYTES = 48LL << 30;
-constexpr size_t WIDE_LDS_PER_CU = 160u << 10;  // LDS of one gfx950 compute unit
 static int chunk_for(const fh_tuning &t, int P, int box, long long extra = 0)
 {
     if (t.chunk > 0) return t.chunk;
@@ -532,16 +531,17 @@ static int chunk_for(const fh_tuning &t, int P, int box, long long extra = 0)
 
 // The brick grid of an inserter mode: gauss_2 and trilinear (stencil origin
 // floor(p), origins -P/2-1 .. P/2, 8^3 origins per brick), or for the wide
-// stencils of S cells per axis 4^3 origins per brick over the origins from
-// the lowest one whose stencil reaches a cell in [-P/2, P/2] and that
-// wide_setup accepts, up to P/2 (higher origins reach no cell).
+// stencils of S cells per axis 4^3 origins per brick (3 x 3 x 5 for the
+// 6-cell Gaussians) over the origins from the lowest one whose stencil
+// reaches a cell in [-P/2, P/2] and that wide_setup accepts, up to P/2
+// (higher origins reach no cell).
 static BrickGeom brick_geom(int P, int mode)
 {
     BrickGeom g;
     const int H = P / 2, S = wide_cells(mode);
     if (S == 0) {
-        g.bs = BRICK;
-        g.halo = HALO;
+        g.bs = g.bsz = BRICK;
+        g.halo = g.haloz = HALO;
         g.ow = -H - 1;
         g.po = (float)(-H - 1);
     } else {
@@ -555,18 +555,25 @@ static BrickGeom brick_geom(int P, int mode)
         case 9: ow = -H - 7; off = 4.0f; break;  // kaiser_bessel_derived
         default: ow = -H - 4; off = 2.5f; break; // gauss_var, gauss_5, fourier_iter
         }
-        g.bs = WBS;
-        g.halo = WBS + S - 1;
+        g.bs = gauss6(mode) ? G6_BX : WBS;
+        g.bsz = gauss6(mode) ? G6_BZ : WBS;
+        g.halo = g.bs + S - 1;
+        g.haloz = g.bsz + S - 1;
         g.ow = ow;
         g.po = (float)ow + off;
     }
     g.nb = (H - g.ow + 1 + g.bs - 1) / g.bs;
-    g.part_floats = 3 * g.halo * g.halo * g.halo;
+    g.nbz = (H - g.ow + 1 + g.bsz - 1) / g.bsz;
+    g.part_floats = 3 * g.halo * g.halo * g.haloz;
     g.per_brick = S != 0;
-    g.nbricks = g.nb * g.nb * g.nb;
+    g.nbricks = g.nb * g.nb * g.nbz;
     g.nkeys = 3 * g.nbricks;
     return g;
 }
+
+// list entries a slice can take: at most 5 bricks per brick column along its
+// dominant normal axis (4 shown, see k_bin_cols)
+static long long list_per_slice(const BrickGeom &g) { return 5LL * g.nb * std::max(g.nb, g.nbz); }
 
 static int ensure_bins(fh_reconstructor *h, long long nslices)
 {
@@ -575,8 +582,7 @@ static int ensure_bins(fh_reconstructor *h, long long nslices)
     const BrickGeom g = brick_geom(h->P, h->mode);
     h->geom = g;
     BinBuffers &b = h->bins;
-    // at most 5 bricks per brick column per slice (4 shown, see k_bin_cols)
-    b.list_cap = 5LL * g.nb * g.nb * nslices;
+    b.list_cap = list_per_slice(g) * nslices;
     b.item_cap = b.list_cap / std::max(1, h->tune.slices_per_item) + g.nkeys + 1;
     FH_TRY(h, hipMalloc(&b.counts, sizeof(int) * g.nkeys));
     FH_TRY(h, hipMalloc(&b.offsets, sizeof(int) * (g.nkeys + 1)));
@@ -641,13 +647,14 @@ long long footprint_bytes_for_mode(int P, int nsym, int chunk, const char *mode_
     const long long sl = 8LL * chunk * P * (P / 2 + 1) + 4LL * chunk * P * P;
     const BrickGeom g = brick_geom(P, mode);
     const long long nslices = (long long)chunk * nsym;
-    const long long list = 5LL * g.nb * g.nb * nslices;
+    const long long list = list_per_slice(g) * nslices;
     const long long items = list / 64 + g.nkeys + 1;
     const long long bins = 4LL * list + 16LL * items + 16LL * g.nkeys + 3LL * (long long)sizeof(SliceRec) * nslices;
-    // partial bricks: about 1.1 (P/bs)^2 (slice, brick) pairs per slice, one
-    // item per 64 pairs of a key plus one per key the slices reach
-    const double pb = (double)P / g.bs;
-    const long long part_items = (long long)(1.1 * pb * pb * nslices / 64) + g.nkeys / 2;
+    // partial bricks: about 1.1 (P/bs)^2 (slice, brick) pairs per slice (P^2 times the
+    // mean width of a brick over its volume), one item per 64 pairs of a key plus one
+    // per key the slices reach
+    const double pb2 = (double)P * P * (2 * g.bs + g.bsz) / (3.0 * g.bs * g.bs * g.bsz);
+    const long long part_items = (long long)(1.1 * pb2 * nslices / 64) + g.nkeys / 2;
     const long long inter = prep_column_first(P) ? (long long)prep_inter_bytes(P, std::min(chunk, PREP_INTER_PARTICLES)) : 0;
     return v + sl + inter + bins + 4LL * g.part_floats * part_items;
 }
@@ -1308,9 +1315,8 @@ static int insert_batch_impl(fh_reconstructor *h, const float *imgs, int n, int 
     const float *df2h = df2.empty() ? nullptr : df2.data();
     // a CTF flip before a 2-D resampling stages two P x P images per particle
     const long long xbytes = xfh ? ((defocus && ctf) ? 8LL : 4LL) * h->P * h->P : 0;
-    // the brick list (at most 5 nb^2 entries per slice) is indexed with int
-    const BrickGeom bg = brick_geom(h->P, h->mode);
-    const long long max_slices = std::max(1LL, (long long)INT32_MAX / (5LL * bg.nb * bg.nb) - 1);
+    // the brick list is indexed with int
+    const long long max_slices = std::max(1LL, (long long)INT32_MAX / list_per_slice(brick_geom(h->P, h->mode)) - 1);
     const int chunk = (int)std::max(1LL, std::min({(long long)chunk_for(h->tune, h->P, box, xbytes),
                                                    (long long)std::max(n, 1), max_slices / h->nsym}));
     rc = ensure_chunk(h, chunk, box);
@@ -1373,13 +1379,8 @@ static int insert_batch_impl(fh_reconstructor *h, const float *imgs, int n, int 
         if (rc) return rc;
         FH_TRY(h, hipEventRecord(h->ev[3], h->stream));
         if (ctl[1] > 0 && wide_cells(h->mode)) {
-            // the wide stencils: one wave per item, 4 per workgroup (2 for 9-cell stencils), as
-            // many workgroups as fit the LDS of every compute unit
-            const int ww = wide_cells(h->mode) > 7 ? 2 : 4;
-            const int per_cu = std::max(1, (int)(WIDE_LDS_PER_CU / scatter_wide_lds_bytes(h->mode, ww)));
             FH_TRY(h, launch_scatter_wide(h->slices, m * h->nsym, h->nsym, h->t3d, h->wq, c, h->geom, h->bins,
-                                          h->exptab, h->rtab, rwh ? h->rw : nullptr,
-                                          std::min(h->cus * per_cu, (ctl[1] + ww - 1) / ww), ww, h->stream));
+                                          h->exptab, h->rtab, rwh ? h->rw : nullptr, ctl[1], h->cus, h->stream));
         } else if (ctl[1] > 0) {
             FH_TRY(h, launch_scatter_insert(h->slices, m * h->nsym, h->nsym, h->t3d, h->wq, c, h->geom, h->bins,
                                             h->exptab, h->rtab, rwh ? h->rw : nullptr,

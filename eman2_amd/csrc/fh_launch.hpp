@@ -86,24 +86,29 @@ constexpr int HALO_CELLS = HALO * HALO * HALO;     // cells of one partial brick
 constexpr int PART_FLOATS = 3 * HALO_CELLS;        // re, im, weight of one partial brick
 
 // Bricks over the stencil origins: brick b owns origins [ow + bs*b, ow + bs*(b+1))
-// per axis, i.e. the pixel positions p with origin(p) in that range, which is
-// p in [po + bs*b, po + bs*(b+1)) (po = ow + the origin's offset: origin(p) =
-// floor(p - off)); its partial covers the halo^3 cells [ow + bs*b, ... + halo).
+// per axis (z: bsz), i.e. the pixel positions p with origin(p) in that range,
+// which is p in [po + bs*b, po + bs*(b+1)) (po = ow + the origin's offset:
+// origin(p) = floor(p - off)); its partial covers the cells
+// [ow + bs*b, ... + halo) per axis.
 //   gauss_2 / trilinear: origin floor(p), bs 8, halo 9, ow = po = -P/2-1.
-//   wide stencils of S cells per axis: bs 4, halo 3 + S (wide_geom).
+//   the 6-cell Gaussians: bs 3 x 3 x 5, halo 8 x 8 x 10 (one lane per (x, y)
+//   column of cells).
+//   the other wide stencils of S cells per axis: bs 4, halo 3 + S.
 struct BrickGeom {
-    int nb;           // bricks per axis
-    int nbricks;      // nb^3
+    int nb, nbz;      // bricks per axis: x and y, z
+    int nbricks;      // nb nb nbz
     int nkeys;        // 3 * nbricks
-    int bs;           // brick edge, in stencil origins
-    int halo;         // cells per axis of a partial brick
+    int bs, bsz;      // brick edge, in stencil origins: x and y, z
+    int halo, haloz;  // cells per axis of a partial brick
     int ow;           // lowest stencil origin of brick 0
-    int part_floats;  // 3 * halo^3: re, im, weight of one partial brick
+    int part_floats;  // 3 * halo^2 * haloz: re, im, weight of one partial brick
     float po;         // p-space start of brick 0
     int per_brick;    // 1: work items span a brick's three axis keys (the wide-stencil scatter)
 };
 
 constexpr int WBS = 4;  // brick edge of the wide-stencil scatter
+constexpr int G6_BX = 3, G6_BZ = 5;                  // brick edges of the 6-cell Gaussians' scatter (x and y, z)
+constexpr int G6_HX = G6_BX + 5, G6_HZ = G6_BZ + 5;  // cells per axis: 8 x 8 columns, one per lane, of 10 cells
 
 // stencil cells per axis of the inserters the wide-stencil scatter takes
 // (0: not taken); modes as InsertConst::mode
@@ -112,6 +117,9 @@ __host__ __device__ constexpr int wide_cells(int mode)
     return (mode == 2 || mode == 3 || mode == 10 || mode == 11) ? 6 : mode == 5 ? 3 : (mode == 6 || mode == 7) ? 5
          : mode == 8 ? 7 : mode == 9 ? 9 : 0;
 }
+
+// the Gaussians on 6^3 cells (gauss_var, gauss_5, fourier_iter with or without a reference)
+__host__ __device__ constexpr bool gauss6(int mode) { return mode == 2 || mode == 3 || mode == 10 || mode == 11; }
 
 // ---- prep (prep_kernels.hip) ----
 hipError_t launch_edge_mean(const float *imgs, int n, int B, float *means, hipStream_t s);
@@ -177,11 +185,10 @@ hipError_t launch_scatter_insert(const float2 *slices, int nslices, int nsym, co
                                  int waves_per_block, hipStream_t s);
 hipError_t launch_merge_partials(BrickGeom g, BinBuffers b, InsertConst c, float2 *data, float *norm,
                                  hipStream_t s);
-// the wide-stencil modes (wide_cells(mode) > 0) on the bricks of wide_geom
-size_t scatter_wide_lds_bytes(int mode, int waves_per_block);
+// the wide-stencil modes (wide_cells(mode) > 0); items: the work items of the batch
 hipError_t launch_scatter_wide(const float2 *slices, int nslices, int nsym, const float *t3d, const float *wq,
                                InsertConst c, BrickGeom g, BinBuffers b, const float *exptab, const float *rtab,
-                               const float *rw, int grid, int waves_per_block, hipStream_t s);
+                               const float *rw, int items, int cus, hipStream_t s);
 int agree_blocks(int P);
 hipError_t launch_agree_batch(const float2 *slices, int nsym, const float *t3d, const float *wq, int nslices,
                               InsertConst c, float rmax, int sub, const float2 *data, const float *norm,

@@ -378,6 +378,29 @@ __device__ __forceinline__ float2 ref_get(const float2 *__restrict__ ref, int x,
     return ref[cidx(x, y < 0 ? P + y : y, z < 0 ? P + z : z, P, H)];
 }
 
+// Util::trilinear_interpolate_complex (libEM/util.h:645-654) of a reference volume at floor(p)
+__device__ __forceinline__ void ref_trilinear(const float2 *__restrict__ ref, float xx, float yy, float zz, int H,
+                                              float &re, float &im)
+{
+    const float xx0 = floorf(xx), yy0 = floorf(yy), zz0 = floorf(zz);
+    const int x0 = (int)xx0, y0 = (int)yy0, z0 = (int)zz0;
+    const float t = xx - xx0, u = yy - yy0, v = zz - zz0;
+    re = im = 0.f;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        const float2 q = ref_get(ref, x0 + (c & 1), y0 + ((c >> 1) & 1), z0 + (c >> 2), H);
+        const float a = (c & 1) ? t : 1 - t, b = (c & 2) ? u : 1 - u, e = (c & 4) ? v : 1 - v;
+        const float wc = a * b * e;
+        if (c == 0) {
+            re = wc * q.x;
+            im = wc * q.y;
+        } else {
+            re = re + wc * q.x;
+            im = im + wc * q.y;
+        }
+    }
+}
+
 // stencil range (clamped to [-P/2, P/2]) and width of one pixel; false if the
 // reference's range check rejects it (insert_wide's first half)
 __device__ __forceinline__ bool wide_setup(int mode, float xx, float yy, float zz, float w, int H,
@@ -411,27 +434,8 @@ __device__ __forceinline__ bool wide_setup(int mode, float xx, float yy, float z
             px.h = h < 0.1 ? (float)0.1 : h;
             return true;
         }
-        // Util::trilinear_interpolate_complex (libEM/util.h:645-654) at floor(p)
         px.h = 1.0f / 2.0f;
-        const float xx0 = floorf(xx), yy0 = floorf(yy), zz0 = floorf(zz);
-        const int x0 = (int)xx0, y0 = (int)yy0, z0 = (int)zz0;
-        const float t = xx - xx0, u = yy - yy0, v = zz - zz0;
-        float ar = 0.f, ai = 0.f;
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const float2 q = ref_get(ref, x0 + (c & 1), y0 + ((c >> 1) & 1), z0 + (c >> 2), H);
-            const float a = (c & 1) ? t : 1 - t, b = (c & 2) ? u : 1 - u, e = (c & 4) ? v : 1 - v;
-            const float wc = a * b * e;
-            if (c == 0) {
-                ar = wc * q.x;
-                ai = wc * q.y;
-            } else {
-                ar = ar + wc * q.x;
-                ai = ai + wc * q.y;
-            }
-        }
-        px.nre = ar;
-        px.nim = ai;
+        ref_trilinear(ref, xx, yy, zz, H, px.nre, px.nim);
         return true;
     }
     if (mode == 4) {
@@ -1619,14 +1623,15 @@ __global__ void __launch_bounds__(256) k_slice_recs(const float *__restrict__ t3
 
 // Does the slice's pixel domain (half-disk x>=0 of radius sqrt(H^2+H), or
 // the half-square with corners) come within reach of the brick?
-__device__ __forceinline__ bool brick_in_domain(const SliceRec &f, const int bc[3], int H, int BS, double po,
-                                                int corners, double rr)
+// hd: the brick's half diagonal
+__device__ __forceinline__ bool brick_in_domain(const SliceRec &f, const int bc[3], int H, const int bs[3], double hd,
+                                                double po, int corners, double rr)
 {
     double c[3];
-    for (int d = 0; d < 3; d++) c[d] = po + BS * bc[d] + 0.5 * BS;
+    for (int d = 0; d < 3; d++) c[d] = po + bs[d] * bc[d] + 0.5 * bs[d];
     const double s = c[0] * (double)f.u[0] + c[1] * (double)f.u[1] + c[2] * (double)f.u[2];
     const double t = c[0] * (double)f.v[0] + c[1] * (double)f.v[1] + c[2] * (double)f.v[2];
-    const double rh = 0.8660254037844386 * BS + 0.01;
+    const double rh = hd + 0.01;
     if (s < -rh) return false;
     if (corners) return s <= H + rh && t >= -H - rh && t <= H - 1 + rh;
     return s * s + t * t <= rr * rr;
@@ -1639,23 +1644,27 @@ template <int MODE>
 __global__ void __launch_bounds__(256) k_bin_cols(InsertConst c, BrickGeom g, BinBuffers bb)
 {
     extern __shared__ int colcnt[];
-    const int nb = g.nb, BS = g.bs, H = c.H;
+    const int nb = g.nb, H = c.H;
     const double po = g.po;
     const int col = blockIdx.x, A = blockIdx.y;
     const int c1 = col % nb, c2 = col / nb;
     const int b1 = A == 0 ? 1 : 0, b2 = A == 2 ? 1 : 2;
+    const int bs[3] = {g.bs, g.bs, g.bsz};
+    const int na = A == 2 ? g.nbz : nb;  // bricks of the column
+    if (c2 >= (b2 == 2 ? g.nbz : nb)) return;
     int bc[3];
     bc[b1] = c1;
     bc[b2] = c2;
-    for (int i = threadIdx.x; i < nb; i += blockDim.x) {
+    for (int i = threadIdx.x; i < na; i += blockDim.x) {
         bc[A] = i;
         colcnt[i] = MODE == 0 ? 0 : bb.offsets[3 * ((bc[2] * nb + bc[1]) * nb + bc[0]) + A];
     }
     __syncthreads();
     const double dlt = 1e-3;
-    const double L1 = po + BS * c1 - dlt, U1 = po + BS * c1 + BS + dlt;
-    const double L2 = po + BS * c2 - dlt, U2 = po + BS * c2 + BS + dlt;
-    const double rr = sqrt((double)c.rcut * c.rcut + c.rcut) + 0.8660254037844386 * BS + 0.01;
+    const double L1 = po + bs[b1] * c1 - dlt, U1 = po + bs[b1] * c1 + bs[b1] + dlt;
+    const double L2 = po + bs[b2] * c2 - dlt, U2 = po + bs[b2] * c2 + bs[b2] + dlt;
+    const double hd = 0.5 * sqrt((double)(2 * g.bs * g.bs + g.bsz * g.bsz));
+    const double rr = sqrt((double)c.rcut * c.rcut + c.rcut) + hd + 0.01;
     const int n = bb.ctl[4 + A];
     const SliceRec *recs = bb.recs + (size_t)A * bb.rec_cap;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
@@ -1663,13 +1672,13 @@ __global__ void __launch_bounds__(256) k_bin_cols(InsertConst c, BrickGeom g, Bi
         const double pa0 = f.r1 * L1 + f.r2 * L2, pa1 = f.r1 * U1 + f.r2 * L2;
         const double pa2 = f.r1 * L1 + f.r2 * U2, pa3 = f.r1 * U1 + f.r2 * U2;
         const double amin = fmin(fmin(pa0, pa1), fmin(pa2, pa3)), amax = fmax(fmax(pa0, pa1), fmax(pa2, pa3));
-        int lo = (int)floor((amin - dlt - po) / BS);
-        int hi = (int)floor((amax + dlt - po) / BS);
+        int lo = (int)floor((amin - dlt - po) / bs[A]);
+        int hi = (int)floor((amax + dlt - po) / bs[A]);
         if (lo < 0) lo = 0;
-        if (hi > nb - 1) hi = nb - 1;
+        if (hi > na - 1) hi = na - 1;
         for (int ca = lo; ca <= hi; ca++) {
             bc[A] = ca;
-            if (!brick_in_domain(f, bc, H, BS, po, c.corners, rr)) continue;
+            if (!brick_in_domain(f, bc, H, bs, hd, po, c.corners, rr)) continue;
             const int pos = atomicAdd(&colcnt[ca], 1);
             if (MODE == 1) {
                 if (pos < bb.list_cap) bb.list[pos] = f.q;
@@ -1679,7 +1688,7 @@ __global__ void __launch_bounds__(256) k_bin_cols(InsertConst c, BrickGeom g, Bi
     }
     if (MODE == 0) {
         __syncthreads();
-        for (int i = threadIdx.x; i < nb; i += blockDim.x) {
+        for (int i = threadIdx.x; i < na; i += blockDim.x) {
             bc[A] = i;
             bb.counts[3 * ((bc[2] * nb + bc[1]) * nb + bc[0]) + A] = colcnt[i];
         }
@@ -1859,8 +1868,8 @@ hipError_t launch_bin(const float *t3d, const float *wq, int nslices, InsertCons
     if (nslices > b.rec_cap) return hipErrorInvalidValue;
     if ((e = launch_fill_i32(b.counts, 0, g.nkeys, s)) != hipSuccess) return e;
     if ((e = launch_fill_i32(b.ctl, 0, 8, s)) != hipSuccess) return e;
-    const dim3 cgrid(g.nb * g.nb, 3);
-    const size_t clds = sizeof(int) * g.nb;
+    const dim3 cgrid(g.nb * std::max(g.nb, g.nbz), 3);
+    const size_t clds = sizeof(int) * std::max(g.nb, g.nbz);
     if (nslices > 0) {
         hipLaunchKernelGGL(k_slice_recs, dim3((nslices + 255) / 256), dim3(256), 0, s, t3d, wq, nslices, b);
         hipLaunchKernelGGL(k_bin_cols<0>, cgrid, dim3(256), clds, s, c, g, b);
@@ -2320,10 +2329,10 @@ hipError_t launch_scatter_insert(const float2 *slices, int nslices, int nsym, co
 }
 
 // ------------------------------------------------------------ wide-stencil brick scatter
-// The inserters with stencils of S = 3 to 9 cells per axis (gauss_var,
-// gauss_5, gauss_3, kaiser_bessel, kaiser_bessel_derived, gridding_5,
-// gridding_7 and fourier_iter's Gaussian) on bricks of 4^3 stencil origins,
-// binned like gauss_2's on the origin grid of the mode.  A work item's wave
+// The inserters with stencils of S = 3 to 9 cells per axis other than the
+// 6-cell Gaussians (gauss_3, kaiser_bessel, kaiser_bessel_derived,
+// gridding_5, gridding_7) on bricks of 4^3 stencil origins, binned like
+// gauss_2's on the origin grid of the mode.  A work item's wave
 // owns the brick's (3 + S)^3 cells in LDS.  For each slice of the item it
 // tests the 8 x 8 pixels around the projection of the brick's centre (a
 // pixel whose origin lies in the brick is within 2 sqrt 3 of that centre in
@@ -2349,10 +2358,6 @@ __global__ void __launch_bounds__(256) k_scatter_wide(const float2 *__restrict__
 {
     constexpr int S = wide_cells(MODE), HL = WBS + S - 1, HC = HL * HL * HL;
     constexpr int NC = S * S * S, NIT = (NC + 63) / 64;
-    // the Gaussian 6^3 stencils (gauss_var, gauss_5, fourier_iter without a reference): lanes 0..53
-    // keep one x offset oi = lane % 6 in every pass and take the (oj, ok) pair lane / 6 + 9 t in
-    // pass t, so the x distance is computed once per pixel
-    constexpr bool G6 = MODE == 2 || MODE == 3 || MODE == 10;
     extern __shared__ float lds_w[];
     float *etab = lds_w;  // the 1000 fast_exp entries
     float *acc = lds_w + 1024 + (size_t)(threadIdx.x >> 6) * 3 * HC;  // re, im, w over [z][y][x] of the cells
@@ -2362,29 +2367,13 @@ __global__ void __launch_bounds__(256) k_scatter_wide(const float2 *__restrict__
     const int H = c.H, P = c.P, nb = g.nb;
     // this lane's stencil cell in pass t: offsets oi | oj << 4 | ok << 8 (-1 past S^3) and its LDS offset
     int oc[NIT], off[NIT];
-    float fo_j[NIT], fo_k[NIT];
-    const float fo_i = (float)(lane % S);
 #pragma unroll
     for (int t = 0; t < NIT; t++) {
-        int oi, oj, ok;
-        bool in;
-        if (G6) {
-            const int pr = lane / 6 + 9 * t;
-            oi = lane % 6;
-            oj = pr % 6;
-            ok = pr / 6;
-            in = lane < 54;
-        } else {
-            const int ci = lane + 64 * t;
-            oi = ci % S;
-            oj = (ci / S) % S;
-            ok = ci / (S * S);
-            in = ci < NC;
-        }
+        const int ci = lane + 64 * t;
+        const int oi = ci % S, oj = (ci / S) % S, ok = ci / (S * S);
+        const bool in = ci < NC;
         oc[t] = in ? (oi | (oj << 4) | (ok << 8)) : -1;
         off[t] = in ? (ok * HL + oj) * HL + oi : 0;
-        fo_j[t] = (float)oj;
-        fo_k[t] = (float)ok;
     }
     const int total = bb.ctl[1];
     for (;;) {
@@ -2426,7 +2415,7 @@ __global__ void __launch_bounds__(256) k_scatter_wide(const float2 *__restrict__
                 const float weight = rw ? rw[(size_t)p * (H + 1) + hypot_int(x, y)] : wgt;
                 float xx, yy, zz;
                 pixel_coords(x, y, mm, rtab, H, c.Pf, xx, yy, zz);
-                ok = wide_setup(MODE, xx, yy, zz, weight, H, etab, px, c.ref);
+                ok = wide_setup(MODE, xx, yy, zz, weight, H, etab, px);
                 if (ok) {
 #pragma unroll
                     for (int d = 0; d < 3; d++) ok = ok && (unsigned)(px.a[d] - lo[d]) < (unsigned)WBS;
@@ -2454,10 +2443,9 @@ __global__ void __launch_bounds__(256) k_scatter_wide(const float2 *__restrict__
                 u.h = bcast_f(px.h, j);
                 u.dre = bcast_f(px.dre, j);
                 u.dim = bcast_f(px.dim, j);
-                u.nre = MODE == 11 ? bcast_f(px.nre, j) : 0.f;
-                u.nim = MODE == 11 ? bcast_f(px.nim, j) : 0.f;
+                u.nre = u.nim = 0.f;
                 u.H = H;
-                u.ref = c.ref;
+                u.ref = nullptr;
                 const int pkj = __builtin_amdgcn_readlane(pk, j);
                 bool full = true;
 #pragma unroll
@@ -2487,41 +2475,7 @@ __global__ void __launch_bounds__(256) k_scatter_wide(const float2 *__restrict__
                     const int i = u.a[0] + (o & 15), jj = u.a[1] + ((o >> 4) & 15), k = u.a[2] + ((o >> 8) & 15);
                     on[t] = o >= 0 && (full || (i >= u.lo[0] && i <= u.hi[0] && jj >= u.lo[1] && jj <= u.hi[1] &&
                                                 k >= u.lo[2] && k <= u.hi[2]));
-                    if (!G6 && on[t]) on[t] = wide_term(MODE, u, i, jj, k, etab, vr[t], vi[t], vg[t]);
-                }
-                if (G6) {
-                    // wide_term's Gaussian, pass by pass: (float)i = (float)a + (float)o exactly (small
-                    // integers), r = hypot3sq in the reference's order, fast_exp(-r h): the table entry
-                    // (int)(-(double)f * 50 + 0.5) -- f * 50 is exact in double, so one fma -- for
-                    // f >= -19.98, expf below (f = -(r h) <= 0 since h > 0).  All passes' table reads go
-                    // out before the first is used; expf runs only when a lane of the wave needs it.
-                    const float dx = ((float)u.a[0] + fo_i) - u.xx;
-                    const float dx2 = dx * dx;
-                    float fv[NIT], tv[NIT];
-                    bool big[NIT], anyb = false;
-#pragma unroll
-                    for (int t = 0; t < NIT; t++) {
-                        const float dy = ((float)u.a[1] + fo_j[t]) - u.yy, dz = ((float)u.a[2] + fo_k[t]) - u.zz;
-                        const float f = -(dx2 + dy * dy + dz * dz) * u.h;
-                        fv[t] = f;
-                        big[t] = f < -19.98f;  // the same floats as (double)f < -19.98
-                        anyb = anyb || big[t];
-                        const int gi = big[t] ? 0 : (int)__builtin_fma(-(double)f, 50.0, 0.5);
-                        tv[t] = etab[gi];
-                    }
-                    if (__ballot(anyb)) {
-#pragma unroll
-                        for (int t = 0; t < NIT; t++)
-                            if (big[t]) tv[t] = expf(fv[t]);
-                    }
-#pragma unroll
-                    for (int t = 0; t < NIT; t++) {
-                        const float gg = tv[t];
-                        vg[t] = gg * u.ww;
-                        vr[t] = u.dre * gg * u.ww;
-                        vi[t] = u.dim * gg * u.ww;
-                        on[t] = on[t] && !(fabsf(vg[t]) < FLT_MIN);
-                    }
+                    if (on[t]) on[t] = wide_term(MODE, u, i, jj, k, etab, vr[t], vi[t], vg[t]);
                 }
 #pragma unroll
                 for (int t = 0; t < NIT; t++)
@@ -2539,62 +2493,541 @@ __global__ void __launch_bounds__(256) k_scatter_wide(const float2 *__restrict__
     }
 }
 
-size_t scatter_wide_lds_bytes(int mode, int waves_per_block)
+// ------------------------------------------------------------ 6-cell Gaussian scatter
+// gauss_var (e2make3dpar's default), gauss_5 and fourier_iter with or without
+// a reference (modes 2, 3, 10, 11): 6^3 cells per pixel with weights
+// fast_exp(-r^2 h) w.  A work item is a brick of 3 x 3 x 5 stencil origins and
+// up to K slices; its 8 x 8 x 10 cells are kept in registers, lane (x, y) =
+// (lane & 7, lane >> 3) owning the column of 10 cells at (x, y).  A pixel
+// takes 6 passes, one per z plane of its stencil, over the 36 of the 64 lanes
+// whose column lies in the stencil: x and y distances are computed once per
+// pixel, the six z distances come from the lane that tested the pixel, and
+// the sums are three FMAs into fixed registers (one copy of the passes per
+// z offset of the origin).
+//
+// Bound: VALU issue (a wave64 FP32 instruction holds a SIMD for 4 cycles), 50
+// instructions per pixel in the passes that stay within the table.  The form
+// before kept the cells in LDS (54 lanes per pass, 4 passes, 6 LDS operations
+// and 28 VALU instructions each; an 8 x 8 window of candidate pixels tested
+// per slice): 142 VALU instructions per pixel, 116 ms for 8,000 x pad 384
+// gauss_var, now 41 ms; for 2,000 x pad 160 of fourier_iter with a reference
+// (its cells read from memory for every term before, kept in the lanes'
+// registers now) 37.3 ms, now 4.6 ms.  Taking the pixels' values by readlane
+// instead of through LDS: 68 ms.  At 4 waves per SIMD, without spills: 43.5.
+// The table index floor(f 50 + 1/2), f = r^2 h, which the reference takes in
+// double, is one FMA rounded toward zero with 2^21 + 1/2 added: the sum's low
+// mantissa bits are floor(4 (f 50 + 1/2)), so that its bits & 0xffc are 4
+// times the index, the byte offset of the table entry.
+#define G6_CAND 3.2838f  // half diagonal of 3 x 3 x 5 + margin for the FP32 position and origin rounding
+
+// The byte offsets of the table entries of f[0..5], or'ed with `out`: 0 on the
+// lanes of the pixel's window (f in [0, 20) there), 0xffc, the table's last
+// entry, a zero, elsewhere.  A mode switch to rounding toward zero around the
+// six FMAs.
+__device__ __forceinline__ void g6_entries(const float f[6], unsigned out, unsigned e[6])
 {
-    const int HL = WBS + wide_cells(mode) - 1;
+    float t[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) t[k] = f[k];
+    asm("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 3\n\t"
+        "v_fma_f32 %0, %0, %6, %7\n\t"
+        "v_fma_f32 %1, %1, %6, %7\n\t"
+        "v_fma_f32 %2, %2, %6, %7\n\t"
+        "v_fma_f32 %3, %3, %6, %7\n\t"
+        "v_fma_f32 %4, %4, %6, %7\n\t"
+        "v_fma_f32 %5, %5, %6, %7\n\t"
+        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0"
+        : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]), "+v"(t[4]), "+v"(t[5])
+        : "s"(50.0f), "v"(2097152.5f));
+#pragma unroll
+    for (int k = 0; k < 6; k++) e[k] = ((unsigned)__float_as_int(t[k]) & 0xffcu) | out;
+}
+
+// One pixel's values, uniform over the wave.
+struct G6Pix {
+    float xx, yy, h, re, im, w, nre, nim;  // re, im: times the weight w (mode 11: without it)
+    float dz2[6];                          // squared z distances (1e30 on clipped planes)
+};
+
+// table entry at byte offset e: the table starts the kernel's LDS (dynamic, with no static LDS before it)
+__device__ __forceinline__ float g6_table(unsigned e)
+{
+    return *(const __attribute__((address_space(3))) float *)e;
+}
+
+// The passes of a pixel whose origin lies OZ above the brick's in z; `in`: the
+// lanes of its (x, y) window.  No lane is switched off: the others add zeros.
+template <int MODE, int OZ>
+__device__ __forceinline__ void g6_add(const G6Pix &u, float cx, float cy, bool in, const float2 (&rf)[G6_HZ],
+                                       float (&ar)[G6_HZ], float (&ai)[G6_HZ], float (&aw)[G6_HZ])
+{
+    const float dx = cx - u.xx, dy = cy - u.yy;
+    const float s = dx * dx + dy * dy;
+    float f[6];
+    unsigned e[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) f[k] = (s + u.dz2[k]) * u.h;  // hypot3sq in the reference's order, times h
+    g6_entries(f, in ? 0u : 0xffcu, e);
+    float g[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) g[k] = g6_table(e[k]);
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        const int z = OZ + k;
+        if (MODE == 11) {
+            // updt = dt + ref(i, j, k) - ref~(p)
+            const float gw = g[k] * u.w;
+            ar[z] = __builtin_fmaf((u.re + rf[z].x) - u.nre, gw, ar[z]);
+            ai[z] = __builtin_fmaf((u.im + rf[z].y) - u.nim, gw, ai[z]);
+            aw[z] += gw;
+        } else {
+            ar[z] = __builtin_fmaf(u.re, g[k], ar[z]);
+            ai[z] = __builtin_fmaf(u.im, g[k], ai[z]);
+            aw[z] = __builtin_fmaf(u.w, g[k], aw[z]);
+        }
+    }
+}
+
+// The same where terms past the table (f > 19.98, by expf) can occur.  ANY:
+// also dropped ones (below FLT_MIN), cells outside fourier_iter's sphere and
+// values that are not finite: what is not added leaves the sum as it is.
+template <int MODE, int OZ, bool ANY>
+__device__ __forceinline__ void g6_add_far(const G6Pix &u, float cx, float cy, bool in, unsigned inside,
+                                           const float2 (&rf)[G6_HZ], float (&ar)[G6_HZ], float (&ai)[G6_HZ],
+                                           float (&aw)[G6_HZ])
+{
+    const float dx = cx - u.xx, dy = cy - u.yy;
+    const float s = dx * dx + dy * dy;
+    float f[6], fc[6];
+    unsigned e[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        f[k] = (s + u.dz2[k]) * u.h;
+        fc[k] = fminf(f[k], 19.98f);
+    }
+    g6_entries(fc, in ? 0u : 0xffcu, e);
+    float g[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) g[k] = g6_table(e[k]);
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        const int z = OZ + k;
+        const bool big = in && f[k] > 19.98f;  // the same floats as the reference's (double)f > 19.98
+        if (__ballot(big)) {
+            asm volatile("");  // a branch, not a select: most passes have no such lane
+            const float t = expf(-f[k]);
+            g[k] = big ? t : g[k];
+        }
+        bool on = in;
+        if (ANY) on = on && !(fabsf(g[k] * u.w) < FLT_MIN);
+        float re, im, wg;
+        if (MODE == 11) {
+            if (ANY) on = on && (inside >> z & 1u);
+            wg = g[k] * u.w;
+            re = __builtin_fmaf((u.re + rf[z].x) - u.nre, wg, ar[z]);
+            im = __builtin_fmaf((u.im + rf[z].y) - u.nim, wg, ai[z]);
+            wg += aw[z];
+        } else {
+            re = __builtin_fmaf(u.re, g[k], ar[z]);
+            im = __builtin_fmaf(u.im, g[k], ai[z]);
+            wg = __builtin_fmaf(u.w, g[k], aw[z]);
+        }
+        ar[z] = on || !ANY ? re : ar[z];
+        ai[z] = on || !ANY ? im : ai[z];
+        aw[z] = on || !ANY ? wg : aw[z];
+    }
+}
+
+// the width of the modes where it is the same for every pixel: gauss_5, fourier_iter with a reference
+template <int MODE>
+__device__ constexpr float g6_width()
+{
+    return MODE == 3 ? 1.0f / (float)(10.4 / (M_PI * M_PI)) : 1.0f / 2.0f;
+}
+
+// The lane that tests a pixel leaves its values in LDS (G6_REC float4 per
+// lane), all lanes read them back for the pixel's passes: one address for the
+// wave, no bank conflicts, where 13 readlanes cost a fifth of the passes'
+// VALU time.
+constexpr int G6_REC = 4;
+constexpr int G6_WAVE = 16 + 16 + 64 * G6_REC;  // float4 of LDS per wave
+
+template <int MODE>
+__device__ __forceinline__ void g6_put(float4 *r, const G6Pix &px)
+{
+    r[0] = make_float4(px.xx, px.yy, px.w, px.re);
+    r[1] = make_float4(px.im, MODE == 11 ? px.nre : px.h, px.dz2[0], px.dz2[1]);
+    r[2] = make_float4(px.dz2[2], px.dz2[3], px.dz2[4], px.dz2[5]);
+    if (MODE == 11) r[3].x = px.nim;
+}
+
+template <int MODE>
+__device__ __forceinline__ void g6_get(const float4 *r, G6Pix &u)
+{
+    const float4 a = r[0], b = r[1], d = r[2];
+    u.xx = a.x;
+    u.yy = a.y;
+    u.w = a.z;
+    u.re = a.w;
+    u.im = b.x;
+    u.h = MODE == 2 || MODE == 10 ? b.y : g6_width<MODE>();
+    u.nre = MODE == 11 ? b.y : 0.f;
+    u.nim = MODE == 11 ? r[3].x : 0.f;
+    u.dz2[0] = b.z;
+    u.dz2[1] = b.w;
+    u.dz2[2] = d.x;
+    u.dz2[3] = d.y;
+    u.dz2[4] = d.z;
+    u.dz2[5] = d.w;
+}
+
+// the window of lanes of the pixel tested by lane j: bits [x0, x0 + nx) of bytes [y0, y0 + ny)
+__device__ __forceinline__ bool g6_window(int pk, int j)
+{
+    const unsigned b = (unsigned)__builtin_amdgcn_readlane(pk, j);
+    const unsigned row = (((1u << (b >> 3 & 7)) - 1u) << (b & 7)) * 0x01010101u;
+    return __builtin_amdgcn_inverse_ballot_w64(((unsigned long long)row << 32 | row) &
+                                               (((1ull << (b >> 9 & 7) * 8) - 1ull) << (b >> 6 & 7) * 8));
+}
+
+// gauss_var's width of the pixel at p, (float)(1 / ((double)(|p|^2 / 4000) + 0.15)) and at least 0.1: |p|^2 / 4000
+// by the reciprocal with one exact-residual step, which rounds correctly; the double reciprocal by two Newton steps.
+__device__ __forceinline__ float g6_width_at(float x, float y, float z)
+{
+    const float n = x * x + y * y + z * z, inv = 1.0f / 4000.0f;
+    const float v = n * inv;
+    const double t = (double)__builtin_fmaf(__builtin_fmaf(-v, 4000.0f, n), inv, v) + 0.15;
+    double r = __builtin_amdgcn_rcp(t);
+    r = __builtin_fma(__builtin_fma(-t, r, 1.0), r, r);
+    r = __builtin_fma(__builtin_fma(-t, r, 1.0), r, r);
+    return fmaxf((float)r, 0.1f);  // the same floats as the reference's double comparison with 0.1
+}
+
+// The slice of lane (i, r) in a group of 8: index (-1: none), t3d rows 0 and 1, weight; loaded one group ahead.
+struct G6Slice {
+    int q;
+    float mm[6];
+    float wgt;
+};
+
+__device__ __forceinline__ void g6_fetch(G6Slice &gs, int s, int count, int qbuf, int qbase, int lane, int nslices,
+                                         const float *__restrict__ t3d, const float *__restrict__ wq)
+{
+    const int idx = s + (lane >> 3);
+    const int qi = __builtin_amdgcn_ds_bpermute((idx - qbase) << 2, qbuf);
+    const int q = idx < count ? qi : -1;
+    const bool qv = q >= 0 && q < nslices;  // never written list entries are skipped
+    gs.q = qv ? q : -1;
+#pragma unroll
+    for (int d = 0; d < 6; d++) gs.mm[d] = qv ? t3d[9 * (size_t)q + d] : 0.f;
+    gs.wgt = qv ? wq[q] : 0.f;
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 11 ? 4 : 5))) k_scatter_gauss6(const float2 *__restrict__ slices, int nslices, int nsym,
+                                                        const float *__restrict__ t3d, const float *__restrict__ wq,
+                                                        InsertConst c, BrickGeom g, BinBuffers bb,
+                                                        const float *__restrict__ exptab_g,
+                                                        const float *__restrict__ rtab_g,
+                                                        const float *__restrict__ rw)
+{
+    extern __shared__ float4 lds_g6[];
+    float *etab = reinterpret_cast<float *>(lds_g6);  // the 1000 fast_exp entries, then zeros
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // per wave: 8 slice records (2 float4 each), 64 row marks and 64 pixels
+    float4 *rec = lds_g6 + 256 + wave * G6_WAVE;
+    int *mark = reinterpret_cast<int *>(rec + 16);
+    float4 *pix = rec + 32;
+    float *rtab = reinterpret_cast<float *>(lds_g6 + 256 + (blockDim.x >> 6) * G6_WAVE);  // P + 2 entries: fl(i/P)
+    const int H = c.H, P = c.P, nb = g.nb;
+    for (int i = threadIdx.x; i < 1024; i += blockDim.x) etab[i] = i < 1000 ? exptab_g[i] : 0.f;
+    for (int i = threadIdx.x; i < P + 2; i += blockDim.x) rtab[i] = rtab_g[i];
+    __syncthreads();
+    const int n2x = MODE >= 10 ? H - 1 : H;  // stencils are clamped to [-n2, n2], fourier_iter's in x to P/2 - 1
+    const int total = bb.ctl[1];
+    for (;;) {
+        int it = 0;
+        if (lane == 0) it = atomicAdd(&bb.ctl[0], 1);
+        it = __builtin_amdgcn_readfirstlane(it);
+        if (it >= total) break;
+        const WorkItem w = bb.items[it];
+        const int brick = w.key / 3;
+        const int bc[3] = {brick % nb, (brick / nb) % nb, brick / (nb * nb)};
+        const int lo[3] = {g.ow + G6_BX * bc[0], g.ow + G6_BX * bc[1], g.ow + G6_BZ * bc[2]};
+        // p-space centre of the brick (exact: half-integers of magnitude < 2^20)
+        const float pc[3] = {g.po + (float)(G6_BX * bc[0]) + 0.5f * G6_BX, g.po + (float)(G6_BX * bc[1]) + 0.5f * G6_BX,
+                             g.po + (float)(G6_BZ * bc[2]) + 0.5f * G6_BZ};
+        const float pl[3] = {g.po + (float)(G6_BX * bc[0]), g.po + (float)(G6_BX * bc[1]), g.po + (float)(G6_BZ * bc[2])};
+        // a cell of the brick lies outside the volume: the stencils are clamped
+        const bool edge = lo[0] < -n2x || lo[0] + G6_HX - 1 > n2x || lo[1] < -H || lo[1] + G6_HX - 1 > H ||
+                          lo[2] < -H || lo[2] + G6_HZ - 1 > H;
+        // the table may end within a stencil: not for h <= 1/2 (farthest corner 3 * 3.5^2), which
+        // gauss_var's width stays below beyond |p| = 87 (the brick's pixels lie within 3.3 of its centre)
+        const bool near = MODE == 3 || (MODE != 11 && pc[0] * pc[0] + pc[1] * pc[1] + pc[2] * pc[2] < 90.5f * 90.5f);
+        const int ix = lo[0] + (lane & 7), iy = lo[1] + (lane >> 3);  // this lane's column of cells
+        const float cx = (float)ix, cy = (float)iy;
+        float ar[G6_HZ], ai[G6_HZ], aw[G6_HZ];
+        float2 rf[G6_HZ];
+        unsigned inside = 0;
+        bool cut = false;  // a cell of the brick lies outside fourier_iter's sphere, or its value is not finite
+#pragma unroll
+        for (int z = 0; z < G6_HZ; z++) {
+            ar[z] = ai[z] = aw[z] = 0.f;
+            rf[z] = make_float2(0.f, 0.f);
+            if (MODE == 11) {
+                const int iz = lo[2] + z;
+                rf[z] = ref_get(c.ref, ix, iy, iz, H);
+                if (ix * ix + iy * iy + iz * iz <= H * H) inside |= 1u << z;
+                cut = cut || !(fabsf(rf[z].x) + fabsf(rf[z].y) < FLT_MAX);
+            }
+        }
+        if (MODE == 11) cut = __ballot(cut || inside != (1u << G6_HZ) - 1u) != 0;
+        // 8 slices at a time: lane (i, r) = (lane / 8, lane % 8) sets up row r of slice i, the rows of
+        // the slice's pixels around the projection of the brick's centre (a pixel whose origin lies in the
+        // brick is within the half diagonal of that centre in p: at most 7 rows), with the range of x
+        // where p lies in the brick's box, margins as in scatter_group; the rows' pixels then form one
+        // stream of which each window gives 64 to the lanes.
+        int qbase = 0;
+        int qbuf = lane < w.count ? bb.list[w.start + lane] : -1;
+        G6Slice nxt;
+        g6_fetch(nxt, 0, w.count, qbuf, qbase, lane, nslices, t3d, wq);
+        for (int s0 = 0; s0 < w.count; s0 += 8) {
+            const G6Slice gs = nxt;
+            const int s1 = s0 + 8;
+            if (s1 < w.count) {
+                if (s1 + 8 > qbase + 64) {
+                    qbase = s1;
+                    qbuf = qbase + lane < w.count ? bb.list[w.start + qbase + lane] : -1;
+                }
+                g6_fetch(nxt, s1, w.count, qbuf, qbase, lane, nslices, t3d, wq);
+            }
+            if ((lane & 7) == 0) {
+                rec[2 * (lane >> 3)] = make_float4(gs.mm[0], gs.mm[1], gs.mm[2], gs.mm[3]);
+                rec[2 * (lane >> 3) + 1] = make_float4(gs.mm[4], gs.mm[5], gs.wgt,
+                                                       __int_as_float(gs.q >= 0 ? gs.q / nsym : 0));  // particle
+            }
+            int cnt = 0, xs = 0, y = 0;
+            {
+                const float sc = pc[0] * gs.mm[0] + pc[1] * gs.mm[1] + pc[2] * gs.mm[2];
+                const float tc = pc[0] * gs.mm[3] + pc[1] * gs.mm[4] + pc[2] * gs.mm[5];
+                const int xc0 = (int)rintf(sc), yc0 = (int)rintf(tc);
+                const float fs = sc - (float)xc0, ft = tc - (float)yc0;
+                const int dy = (int)ceilf(ft - G6_CAND) + (lane & 7);
+                y = yc0 + dy;
+                if (gs.q >= 0 && gs.wgt != 0.0f && (float)dy <= ft + G6_CAND && y >= -H && y <= H - 1) {
+                    float xl = fs - G6_CAND, xh = fs + G6_CAND;
+#pragma unroll
+                    for (int d = 0; d < 3; d++) {
+                        const float ud = gs.mm[d], vd = gs.mm[3 + d];
+                        if (fabsf(ud) >= 0.05f) {
+                            const float b0 = pl[d] - ((float)xc0 * ud + (float)yc0 * vd) - (float)dy * vd;
+                            const float iu = __builtin_amdgcn_rcpf(ud);
+                            const float t0 = (b0 - SC_DLT) * iu;
+                            const float t1 = (b0 + (float)(d == 2 ? G6_BZ : G6_BX) + SC_DLT) * iu;
+                            xl = fmaxf(xl, fminf(t0, t1));
+                            xh = fminf(xh, fmaxf(t0, t1));
+                        }
+                    }
+                    const int a = max((int)ceilf(xl - SC_EPS), -xc0);
+                    int b = min((int)floorf(xh + SC_EPS), H - xc0);
+                    // hypot_fast_int(x, y) <= rcut
+                    if (!c.corners) b = min(b, isqrt24(c.rcut * c.rcut + c.rcut - y * y) - xc0);
+                    xs = xc0 + a;
+                    cnt = max(0, b - a + 1);
+                }
+            }
+            const int incl = wave_scan_add(cnt);
+            const int rows = __builtin_amdgcn_readlane(incl, 63);
+            const int excl = incl - cnt;
+            // row record read by the slots of this row: (x - slot, y) as two int16
+            const int rowrec = (int)(((unsigned)(xs - excl) & 0xffffu) | ((unsigned)y << 16));
+            for (int next = 0; next < rows; next += 64) {
+                // row of slot next + lane: the last non-empty row starting at or before it
+                mark[lane] = -1;
+                wave_sync_lds();
+                if (cnt > 0 && excl >= next && excl < next + 64) mark[excl - next] = lane;
+                if (cnt > 0 && excl < next && excl + cnt > next) mark[0] = lane;
+                wave_sync_lds();
+                const int rl = wave_scan_max(mark[lane]) & 63;
+                const int rr = __builtin_amdgcn_ds_bpermute(rl << 2, rowrec);
+                const int slot = next + lane;
+                bool ok = slot < rows, med = false, any = false;
+                G6Pix px;
+                px.xx = px.yy = px.h = px.re = px.im = px.w = px.nre = px.nim = 0.f;
+#pragma unroll
+                for (int k = 0; k < 6; k++) px.dz2[k] = 0.f;
+                int pk = 0, oz = 0;
+                if (ok) {
+                    const float4 ra = rec[2 * (rl >> 3)], rb = rec[2 * (rl >> 3) + 1];
+                    const int x = (int)(short)(rr & 0xffff) + slot, ry = rr >> 16;
+                    const float pm[6] = {ra.x, ra.y, ra.z, ra.w, rb.x, rb.y};
+                    float pp[3];
+                    pixel_coords(x, ry, pm, rtab, H, c.Pf, pp[0], pp[1], pp[2]);
+                    int a[3];
+                    ok = (unsigned)x <= (unsigned)H;
+#pragma unroll
+                    for (int d = 0; d < 3; d++) {
+                        // floor((double)p - 2.5): the fraction p - floor(p) is below 1/2 or not
+                        const float fl = floorf(pp[d]);
+                        a[d] = (int)fl - (pp[d] - fl >= 0.5f ? 2 : 3);
+                        ok = ok && (unsigned)(a[d] - lo[d]) < (unsigned)(d == 2 ? G6_BZ : G6_BX);
+                    }
+                    pk = (a[0] - lo[0]) | 6 << 3 | (a[1] - lo[1]) << 6 | 6 << 9;
+                    oz = a[2] - lo[2];
+#pragma unroll
+                    for (int k = 0; k < 6; k++) {
+                        const float dz = (float)(a[2] + k) - pp[2];
+                        px.dz2[k] = dz * dz;
+                    }
+                    if (edge) {
+                        // the stencil clamped to the volume: window of columns and planes of the cells inside
+                        int l[3], n[3];
+#pragma unroll
+                        for (int d = 0; d < 3; d++) {
+                            const int n2 = d == 0 ? n2x : H;
+                            l[d] = max(a[d], -n2);
+                            n[d] = min(a[d] + 5, n2) - l[d] + 1;
+                            ok = ok && a[d] >= -n2 - 4 && a[d] <= n2 + 3 && n[d] > 0;
+                        }
+                        pk = (l[0] - lo[0]) | n[0] << 3 | (l[1] - lo[1]) << 6 | n[1] << 9;
+#pragma unroll
+                        for (int k = 0; k < 6; k++)
+                            if (a[2] + k < l[2] || a[2] + k >= l[2] + n[2]) {
+                                px.dz2[k] = 1e30f;  // weight 0
+                                any = true;
+                            }
+                    }
+                    if (ok) {
+                        const unsigned p = (unsigned)__float_as_int(rb.w);
+                        const float2 dt = slice_value(slices + (size_t)p * P * (H + 1), x, ry, P, H);
+                        const float wt = rw ? rw[(size_t)p * (H + 1) + hypot_int(x, ry)] : rb.z;
+                        px.xx = pp[0];
+                        px.yy = pp[1];
+                        px.w = wt;
+                        px.h = MODE == 2 || MODE == 10 ? g6_width_at(pp[0], pp[1], pp[2]) : g6_width<MODE>();
+                        if (MODE == 11) ref_trilinear(c.ref, pp[0], pp[1], pp[2], H, px.nre, px.nim);
+                        px.re = MODE == 11 ? dt.x : dt.x * wt;
+                        px.im = MODE == 11 ? dt.y : dt.y * wt;
+                        any = any || cut || !(fabsf(wt) > 1e-25f) ||
+                              !(fabsf(px.re) + fabsf(px.im) + fabsf(px.nre) + fabsf(px.nim) + fabsf(wt) < FLT_MAX);
+                        if (near) {
+                            float far = 0.f;  // squared distance of the stencil's farthest corner
+#pragma unroll
+                            for (int d = 0; d < 3; d++) {
+                                const float e = fmaxf(pp[d] - (float)a[d], (float)(a[d] + 5) - pp[d]);
+                                far += e * e;
+                            }
+                            med = far * px.h > 19.9f;
+                            // exp(-80) / 100 is above FLT_MIN
+                            any = any || far * px.h > 80.f || (med && !(fabsf(wt) > 1e-2f));
+                        }
+                    }
+                }
+                if (ok) g6_put<MODE>(pix + G6_REC * lane, px);
+                wave_sync_lds();
+                // the pixels one after another, by the z offset of their origin: each offset's loop adds
+                // into registers of its own choice
+#define G6_LOOP(Z, COND, ADD)                                                              \
+    for (unsigned long long left = __ballot((COND) && oz == Z); left; left &= left - 1) {   \
+        const int j = (int)__builtin_ctzll(left);                                           \
+        G6Pix u;                                                                            \
+        g6_get<MODE>(pix + G6_REC * j, u);                                                  \
+        const bool in = g6_window(pk, j);                                                   \
+        ADD;                                                                                \
+    }
+#define G6_LOOPS(COND, ADD) \
+    G6_LOOP(0, COND, ADD(0)) G6_LOOP(1, COND, ADD(1)) G6_LOOP(2, COND, ADD(2)) G6_LOOP(3, COND, ADD(3)) G6_LOOP(4, COND, ADD(4))
+#define G6_NEAR(Z) g6_add<MODE, Z>(u, cx, cy, in, rf, ar, ai, aw)
+#define G6_FAR(Z) g6_add_far<MODE, Z, false>(u, cx, cy, in, inside, rf, ar, ai, aw)
+#define G6_ANY(Z) g6_add_far<MODE, Z, true>(u, cx, cy, in, inside, rf, ar, ai, aw)
+                G6_LOOPS(ok && !med && !any, G6_NEAR)
+                if (MODE != 11 && __ballot(ok && med && !any)) { G6_LOOPS(ok && med && !any, G6_FAR) }
+                if (__ballot(ok && any)) { G6_LOOPS(ok && any, G6_ANY) }
+#undef G6_LOOP
+#undef G6_LOOPS
+#undef G6_NEAR
+#undef G6_FAR
+#undef G6_ANY
+                wave_sync_lds();  // the pixels' and slices' records are read before the next ones are written
+            }
+        }
+        float *out = bb.part + (size_t)it * g.part_floats + lane;  // [field][z][y][x]
+#pragma unroll
+        for (int z = 0; z < G6_HZ; z++) {
+            out[64 * z] = ar[z];
+            out[64 * (G6_HZ + z)] = ai[z];
+            out[64 * (2 * G6_HZ + z)] = aw[z];
+        }
+    }
+}
+
+static size_t scatter_wide_lds_bytes(InsertConst c, int waves_per_block)
+{
+    if (gauss6(c.mode)) return sizeof(float) * (1024 + 4 * G6_WAVE * (size_t)waves_per_block + c.P + 2);
+    const int HL = WBS + wide_cells(c.mode) - 1;
     return sizeof(float) * (1024 + (size_t)waves_per_block * 3 * HL * HL * HL);
 }
 
 hipError_t launch_scatter_wide(const float2 *slices, int nslices, int nsym, const float *t3d, const float *wq,
                                InsertConst c, BrickGeom g, BinBuffers b, const float *exptab, const float *rtab,
-                               const float *rw, int grid, int waves_per_block, hipStream_t s)
+                               const float *rw, int items, int cus, hipStream_t s)
 {
     const int S = wide_cells(c.mode);
-    if (S == 0 || waves_per_block < 1 || waves_per_block > 4 || g.bs != WBS || g.halo != WBS + S - 1)
+    const bool g6 = gauss6(c.mode);
+    if (S == 0 || g.bs != (g6 ? G6_BX : WBS) || g.bsz != (g6 ? G6_BZ : WBS) || g.halo != g.bs + S - 1 ||
+        g.haloz != g.bsz + S - 1)
         return hipErrorInvalidValue;
-    const size_t lds = scatter_wide_lds_bytes(c.mode, waves_per_block);
+    // one wave per item: 4 waves per workgroup (2 for 9-cell stencils), as many workgroups as fit
+    // the compute units
+    const int ww = S > 7 ? 2 : 4;
+    const size_t lds = scatter_wide_lds_bytes(c, ww);
     if (lds > 65536) return hipErrorInvalidValue;
-    const dim3 gr(grid), bl(64 * waves_per_block);
-#define FH_WIDE(M) \
-    case M: hipLaunchKernelGGL(k_scatter_wide<M>, gr, bl, lds, s, slices, nslices, nsym, t3d, wq, c, g, b, exptab, rtab, rw); break;
+#define FH_WIDE(KERNEL)                                                                                                  \
+    {                                                                                                                    \
+        int per = 0;                                                                                                     \
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, KERNEL, 64 * ww, lds) != hipSuccess || per < 1) per = 1;   \
+        hipLaunchKernelGGL((KERNEL), dim3(std::min(cus * per, (items + ww - 1) / ww)), dim3(64 * ww), lds, s, slices,     \
+                           nslices, nsym, t3d, wq, c, g, b, exptab, rtab, rw);                                           \
+        return hipGetLastError();                                                                                        \
+    }
     switch (c.mode) {
-        FH_WIDE(2)
-        FH_WIDE(3)
-        FH_WIDE(5)
-        FH_WIDE(6)
-        FH_WIDE(7)
-        FH_WIDE(8)
-        FH_WIDE(9)
-        FH_WIDE(10)
-        FH_WIDE(11)
-    default:
-        return hipErrorInvalidValue;
+    case 2: FH_WIDE(k_scatter_gauss6<2>)
+    case 3: FH_WIDE(k_scatter_gauss6<3>)
+    case 5: FH_WIDE(k_scatter_wide<5>)
+    case 6: FH_WIDE(k_scatter_wide<6>)
+    case 7: FH_WIDE(k_scatter_wide<7>)
+    case 8: FH_WIDE(k_scatter_wide<8>)
+    case 9: FH_WIDE(k_scatter_wide<9>)
+    case 10: FH_WIDE(k_scatter_gauss6<10>)
+    case 11: FH_WIDE(k_scatter_gauss6<11>)
+    default: return hipErrorInvalidValue;
     }
 #undef FH_WIDE
-    return hipGetLastError();
 }
 
 // ------------------------------------------------------------ merge of partial bricks
 // Sum over the work items of the bricks whose cells include unfolded cell
-// (i, j, k): brick b covers cells [ow + BS*b, ow + BS*b + HL) per axis, so a
-// cell lies in the bricks floor(u / BS) down to ceil((u - HL + 1) / BS),
-// u = cell - ow (for gauss_2, BS 8 and HL 9: the brick owning the origin and,
-// on each axis where the cell is a brick's first, also the previous brick).
-template <int BS, int HL>
+// (i, j, k): brick b covers cells [ow + BS*b, ow + BS*b + HL) per axis (z:
+// BZ, HZ), so a cell lies in the bricks floor(u / BS) down to
+// ceil((u - HL + 1) / BS), u = cell - ow (for gauss_2, BS 8 and HL 9: the
+// brick owning the origin and, on each axis where the cell is a brick's
+// first, also the previous brick).
+template <int BS, int HL, int BZ, int HZ>
 __device__ __forceinline__ void partial_sum(const float *__restrict__ part, const int *__restrict__ item_off, int nb,
-                                            int ow, int pf, int i, int j, int k, float &re, float &im, float &w)
+                                            int nbz, int ow, int pf, int i, int j, int k, float &re, float &im,
+                                            float &w)
 {
-    constexpr int HC = HL * HL * HL;
+    constexpr int HC = HL * HL * HZ;
     const int ui = i - ow, uj = j - ow, uk = k - ow;  // >= 0 for cells >= -H
-    const int bi1 = min(ui / BS, nb - 1), bj1 = min(uj / BS, nb - 1), bk1 = min(uk / BS, nb - 1);
+    const int bi1 = min(ui / BS, nb - 1), bj1 = min(uj / BS, nb - 1), bk1 = min(uk / BZ, nbz - 1);
     const int bi0 = ui < HL ? 0 : (ui - HL + BS) / BS, bj0 = uj < HL ? 0 : (uj - HL + BS) / BS;
-    const int bk0 = uk < HL ? 0 : (uk - HL + BS) / BS;
+    const int bk0 = uk < HZ ? 0 : (uk - HZ + BZ) / BZ;
     re = im = w = 0.f;
     for (int bk = bk1; bk >= bk0; bk--)
         for (int bj = bj1; bj >= bj0; bj--)
             for (int bi = bi1; bi >= bi0; bi--) {
                 const int b = (bk * nb + bj) * nb + bi;
-                const int cc = ((uk - BS * bk) * HL + (uj - BS * bj)) * HL + (ui - BS * bi);
+                const int cc = ((uk - BZ * bk) * HL + (uj - BS * bj)) * HL + (ui - BS * bi);
                 const int i0 = item_off[3 * b], i1 = item_off[3 * b + 3];
                 for (int it = i0; it < i1; it++) {
                     const float *p = part + (size_t)it * pf + cc;
@@ -2612,11 +3045,11 @@ __device__ __forceinline__ void partial_sum(const float *__restrict__ part, cons
 // conjugate copies of the double insertion (value only) and, at x = P/2,
 // the x = -P/2 cells added twice with their weight once; at (0,0,0) and
 // (P/2,0,0) the real part and weight with the imaginary part set to 0.
-template <int BS, int HL>
+template <int BS, int HL, int BZ, int HZ>
 __global__ void __launch_bounds__(256) k_merge_partials(const float *__restrict__ part, const int *__restrict__ item_off,
                                                         BrickGeom g, InsertConst c, float2 *data, float *norm)
 {
-    const int H = c.H, P = c.P, nb = g.nb, ow = g.ow, pf = g.part_floats;
+    const int H = c.H, P = c.P, nb = g.nb, nbz = g.nbz, ow = g.ow, pf = g.part_floats;
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (long long)P * P * (H + 1)) return;
     const int xs = (int)(idx % (H + 1));
@@ -2624,10 +3057,10 @@ __global__ void __launch_bounds__(256) k_merge_partials(const float *__restrict_
     const int ys = (int)(rest % P), zs = (int)(rest / P);
     float r, i, w;
     if (ys == 0 && zs == 0 && (xs == 0 || xs == H)) {
-        partial_sum<BS, HL>(part, item_off, nb, ow, pf, xs, 0, 0, r, i, w);
+        partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, xs, 0, 0, r, i, w);
         if (xs == H) {
             float r2, i2, w2;
-            partial_sum<BS, HL>(part, item_off, nb, ow, pf, -H, 0, 0, r2, i2, w2);
+            partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, -H, 0, 0, r2, i2, w2);
             r += r2;
             i += i2;
             w += w2;
@@ -2652,7 +3085,7 @@ __global__ void __launch_bounds__(256) k_merge_partials(const float *__restrict_
     float dre = 0.f, dim = 0.f, dw = 0.f;
     for (int a = 0; a < njd; a++)
         for (int b = 0; b < nkd; b++) {
-            partial_sum<BS, HL>(part, item_off, nb, ow, pf, xs, jd[a], kd[b], r, i, w);
+            partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, xs, jd[a], kd[b], r, i, w);
             dre += r;
             dim += i;
             dw += w;
@@ -2660,17 +3093,17 @@ __global__ void __launch_bounds__(256) k_merge_partials(const float *__restrict_
     for (int a = 0; a < njn; a++)
         for (int b = 0; b < nkn; b++) {
             if (xs == 0 || xs == H) {
-                partial_sum<BS, HL>(part, item_off, nb, ow, pf, xs, jn[a], kn[b], r, i, w);
+                partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, xs, jn[a], kn[b], r, i, w);
                 dre += r;
                 dim -= i;
                 if (xs == H) {
-                    partial_sum<BS, HL>(part, item_off, nb, ow, pf, -H, jn[a], kn[b], r, i, w);
+                    partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, -H, jn[a], kn[b], r, i, w);
                     dre += 2.f * r;
                     dim -= 2.f * i;
                     dw += w;
                 }
             } else {
-                partial_sum<BS, HL>(part, item_off, nb, ow, pf, -xs, jn[a], kn[b], r, i, w);
+                partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, -xs, jn[a], kn[b], r, i, w);
                 dre += r;
                 dim -= i;
                 dw += w;
@@ -2688,21 +3121,20 @@ hipError_t launch_merge_partials(BrickGeom g, BinBuffers b, InsertConst c, float
 {
     const long long n = (long long)c.P * c.P * (c.H + 1);
     const dim3 grid((unsigned)((n + 255) / 256));
-    if (g.bs == BRICK && g.halo == HALO)
-        hipLaunchKernelGGL((k_merge_partials<BRICK, HALO>), grid, dim3(256), 0, s, b.part, b.item_off, g, c, data, norm);
-    else if (g.bs == WBS && g.halo == WBS + 2)
-        hipLaunchKernelGGL((k_merge_partials<WBS, WBS + 2>), grid, dim3(256), 0, s, b.part, b.item_off, g, c, data, norm);
-    else if (g.bs == WBS && g.halo == WBS + 4)
-        hipLaunchKernelGGL((k_merge_partials<WBS, WBS + 4>), grid, dim3(256), 0, s, b.part, b.item_off, g, c, data, norm);
-    else if (g.bs == WBS && g.halo == WBS + 5)
-        hipLaunchKernelGGL((k_merge_partials<WBS, WBS + 5>), grid, dim3(256), 0, s, b.part, b.item_off, g, c, data, norm);
-    else if (g.bs == WBS && g.halo == WBS + 6)
-        hipLaunchKernelGGL((k_merge_partials<WBS, WBS + 6>), grid, dim3(256), 0, s, b.part, b.item_off, g, c, data, norm);
-    else if (g.bs == WBS && g.halo == WBS + 8)
-        hipLaunchKernelGGL((k_merge_partials<WBS, WBS + 8>), grid, dim3(256), 0, s, b.part, b.item_off, g, c, data, norm);
-    else
-        return hipErrorInvalidValue;
-    return hipGetLastError();
+#define FH_MERGE(BS, HL, BZ, HZ)                                                                                       \
+    if (g.bs == BS && g.halo == HL && g.bsz == BZ && g.haloz == HZ) {                                                  \
+        hipLaunchKernelGGL((k_merge_partials<BS, HL, BZ, HZ>), grid, dim3(256), 0, s, b.part, b.item_off, g, c, data,  \
+                           norm);                                                                                      \
+        return hipGetLastError();                                                                                      \
+    }
+    FH_MERGE(BRICK, HALO, BRICK, HALO)
+    FH_MERGE(G6_BX, G6_HX, G6_BZ, G6_HZ)
+    FH_MERGE(WBS, WBS + 2, WBS, WBS + 2)
+    FH_MERGE(WBS, WBS + 4, WBS, WBS + 4)
+    FH_MERGE(WBS, WBS + 6, WBS, WBS + 6)
+    FH_MERGE(WBS, WBS + 8, WBS, WBS + 8)
+#undef FH_MERGE
+    return hipErrorInvalidValue;
 }
 
 }  // namespace fh
