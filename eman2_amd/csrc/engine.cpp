@@ -575,6 +575,26 @@ static BrickGeom brick_geom(int P, int mode)
 // dominant normal axis (4 shown, see k_bin_cols)
 static long long list_per_slice(const BrickGeom &g) { return 5LL * g.nb * std::max(g.nb, g.nbz); }
 
+// Slices per work item of a batch of nslices slices (at most the tuned value).
+// A work item is one wave's serial chain and ends in one partial brick: with
+// many slices per item the bricks at the volume's centre, which every slice
+// crosses, outlast the rest of a small batch; with few, the partial bricks
+// outweigh the slices added.  The two costs grow as K and as pairs / K, so the
+// best K goes with the square root of the (slice, brick) pairs per resident
+// wave.  Measured insertion of K = 1024 against this rule: pad 96, 2,000
+// slices 1.38 -> 0.37 ms; pad 192, 5,000 slices 2.66 -> 1.45 ms; pad 384,
+// 24,000 slices (K = 757) 19.85 -> 19.9 ms; gauss_var at pad 96, 3,000 slices
+// 6.8 -> 3.6 ms, at pad 192, 1,000 slices 8.2 -> 3.3 ms.
+static int item_slices(const fh_reconstructor *h, long long nslices)
+{
+    const BrickGeom &g = h->geom;
+    // about 0.63 of (P + brick)^2 times the brick's mean width over its volume
+    const double pb2 = (double)(h->P + 8) * (h->P + 8) * (2 * g.bs + g.bsz) / (3.0 * g.bs * g.bs * g.bsz);
+    const double per_wave = 0.63 * pb2 * (double)nslices / (16.0 * h->cus);
+    const double k = (wide_cells(h->mode) ? 6.0 : 8.0) * sqrt(per_wave);
+    return (int)std::min((double)h->tune.slices_per_item, std::max(16.0, k));
+}
+
 static int ensure_bins(fh_reconstructor *h, long long nslices)
 {
     if (nslices <= h->bins_cap_slices) return FH_OK;
@@ -583,7 +603,9 @@ static int ensure_bins(fh_reconstructor *h, long long nslices)
     h->geom = g;
     BinBuffers &b = h->bins;
     b.list_cap = list_per_slice(g) * nslices;
-    b.item_cap = b.list_cap / std::max(1, h->tune.slices_per_item) + g.nkeys + 1;
+    // smaller batches have fewer items: pairs over K grows with the slices, up to K's rounding
+    const int K = item_slices(h, nslices);
+    b.item_cap = b.list_cap / K * (K < h->tune.slices_per_item ? 5 : 4) / 4 + g.nkeys + 1;
     FH_TRY(h, hipMalloc(&b.counts, sizeof(int) * g.nkeys));
     FH_TRY(h, hipMalloc(&b.offsets, sizeof(int) * (g.nkeys + 1)));
     FH_TRY(h, hipMalloc(&b.item_off, sizeof(int) * (g.nkeys + 1)));
@@ -1071,7 +1093,8 @@ static int insert_batch_graph(fh_reconstructor *h, const float *imgs, int n, int
         hipError_t e = prep_kernels(h, m, box, dimgs, dfd, cc, xf_host ? h->xfd : nullptr, dfd2);
         if (e == hipSuccess) e = launch_compose(h->rots, h->wts, m, h->syms_d, h->nsym, h->t3d, h->wq, h->stream);
         if (e == hipSuccess)
-            e = launch_bin(h->t3d, h->wq, m * h->nsym, c, h->geom, h->bins, h->tune.slices_per_item, h->stream);
+            e = launch_bin(h->t3d, h->wq, m * h->nsym, c, h->geom, h->bins, item_slices(h, (long long)m * h->nsym),
+                           h->stream);
         if (e == hipSuccess)
             e = launch_scatter_insert(h->slices, m * h->nsym, h->nsym, h->t3d, h->wq, c, h->geom, h->bins, h->exptab,
                                       h->rtab, rw_host ? h->rw : nullptr, grid, wpb, h->stream);
@@ -1368,7 +1391,8 @@ static int insert_batch_impl(fh_reconstructor *h, const float *imgs, int n, int 
             st.chunks += 1;
             continue;
         }
-        FH_TRY(h, launch_bin(h->t3d, h->wq, m * h->nsym, c, h->geom, h->bins, h->tune.slices_per_item, h->stream));
+        FH_TRY(h, launch_bin(h->t3d, h->wq, m * h->nsym, c, h->geom, h->bins, item_slices(h, (long long)m * h->nsym),
+                             h->stream));
         FH_TRY(h, hipEventRecord(h->ev[2], h->stream));
         // the work item count sizes the partial-brick buffer
         int ctl[4];

@@ -85,7 +85,7 @@ typedef struct {
  * normal axis. */
 typedef struct {
     int waves_per_block; /* independent item workers per workgroup: 1 to 4 */
-    int slices_per_item; /* slices a work item adds before writing its partial brick */
+    int slices_per_item; /* most slices a work item adds before writing its partial brick (small batches take fewer) */
     int chunk;           /* particles per batched launch; 0 = as many as fit in 48 GiB of staging */
     int blocks_per_cu;   /* persistent grid: workgroups per compute unit */
     int graph;           /* 1: device-resident batches run each chunk as one captured hipGraph */
