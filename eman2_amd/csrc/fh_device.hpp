@@ -36,6 +36,14 @@ __device__ __forceinline__ float sqrt_int_rn(int n)
     r = __fmaf_rn(-su, s, x) > 0.f ? su : r;
     return n == 0 ? 0.f : r;
 }
+// orders a wave's LDS accesses before and after it
+__device__ __forceinline__ void wave_sync_lds()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // multiply by -i
 __device__ __forceinline__ float2 mul_mi(float2 a) { return make_float2(a.y, -a.x); }
 

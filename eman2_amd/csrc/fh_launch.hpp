@@ -192,7 +192,10 @@ hipError_t launch_scatter_wide(const float2 *slices, int nslices, int nsym, cons
 int agree_blocks(int P);
 hipError_t launch_agree_batch(const float2 *slices, int nsym, const float *t3d, const float *wq, int nslices,
                               InsertConst c, float rmax, int sub, const float2 *data, const float *norm,
-                              const float *exptab, const float *rtab, double *acc, hipStream_t s);
+                              const float4 *vol, const float *exptab, const float *rtab, double *acc, hipStream_t s);
+// vol: (re, im, weight, 0) per voxel, pack_elems(P) of them, in cubes of 2^3 voxels
+size_t pack_elems(int P);
+hipError_t launch_pack_volume(const float2 *data, const float *norm, int P, float4 *vol, hipStream_t s);
 hipError_t launch_agree(const float2 *slices, int nsym, const float *t3d, int nslices, InsertConst c, float rmax,
                         const float2 *data, const float *norm, const float *rtab, double *partial, hipStream_t s);
 

@@ -887,24 +887,27 @@ __device__ void own_contribution(const float2 *S, const float *t3dp, int nsym, i
         }
 }
 
-// Tiles of compare pixels: each workgroup takes a 32 x 16 tile of one
-// (particle, symmetry op) slice and stages the slice around it (2-pixel
-// halo: the sources of a compare pixel's nearest cell lie within 2 pixels
-// of it) in LDS -- pixel positions, values and the insertion loop's pixel
-// filters -- so that the own-contribution gather of the slice's own plane
-// reads LDS; the other symmetry planes, the conjugate cells and windows
-// that leave the patch take the global gather.  Same arithmetic and order
-// as gather_cell.
-constexpr int AT_X = 32, AT_Y = 16, AT_HALO = 2;
-constexpr int AT_PX = AT_X + 2 * AT_HALO, AT_PY = AT_Y + 2 * AT_HALO;
-constexpr int AT_PATCH = AT_PX * AT_PY;
-// Mirror patch of the x = 0 tiles: pixels x in [-4, 2], y in
-// [-ty0 - AT_Y - 1, -ty0 + 2], the sources of the mirrored cells of compare
-// pixels x < 3 (around (-x, -y)).
-constexpr int AT_MX = 7, AT_MY = AT_Y + 4, AT_MPATCH = AT_MX * AT_MY;
+// Tiles of compare pixels: each workgroup takes a tile of one (particle,
+// symmetry op) slice, 32 x 32 pixels without symmetry and 32 x 16 with it, and
+// stages the slice around it (2-pixel halo: the sources of a compare pixel's
+// nearest cell lie within 2 pixels of it) in LDS -- pixel positions, values
+// and the insertion loop's pixel filters -- so that the own-contribution
+// gather of the slice's own plane reads LDS; the other symmetry planes and
+// windows that leave the patch take the global gather.
+constexpr int AT_X = 32, AT_HALO = 2;
+constexpr int AT_PX = AT_X + 2 * AT_HALO;
+constexpr int AT_MX = 7;
+// Sizes for tiles of AY rows.  Mirror patch of the x = 0 tiles: pixels x in
+// [-4, 2], y in [-ty0 - AY - 1, -ty0 + 2], the sources of the mirrored cells of
+// compare pixels x < 3 (around (-x, -y)).
+template <int AY>
+struct AgreeTile {
+    static constexpr int PY = AY + 2 * AT_HALO, PATCH = AT_PX * PY, MY = AY + 4, MPATCH = AT_MX * MY;
+    static constexpr int THREADS = 16 * AY, WAVES = THREADS / 64;
+};
 
 // Patch entries carry the floors of their position packed as
-// (x0 + 512) | (y0 + 512) << 10 | (z0 + 512) << 20 in the .w bits, or
+// (x0 + 512) | (y0 + 512) << 10 | (z0 + 512) << 20, or
 // AP_NOKEY for pixels the insertion loop skips (radius cut, origin range).
 // For a cell key kc, kc - key has every 10-bit digit in {0, 1} exactly when
 // the cell is a corner of the pixel's 2x2x2 stencil; the digits are
@@ -914,13 +917,21 @@ constexpr int AP_NOKEY = (int)0x80000000u;
 constexpr unsigned AP_DIGITS = 0x100401u;
 __device__ __forceinline__ int ap_key(int x0, int y0, int z0)
 {
-    return (x0 + 512) | ((y0 + 512) << 10) | ((z0 + 512) << 20);
+    return x0 + (y0 << 10) + (z0 << 20) + (512 + (512 << 10) + (512 << 20));  // digits of 10 bits, none negative
 }
 
+// A patch entry: pixel position, packed floors (AP_NOKEY: skipped by the
+// insertion loop) and slice_value.
+struct AgreePx {
+    float x, y, z;
+    int key;
+    float2 v;
+};
+
 struct AgreePatch {
-    const float4 *pos;   // xx, yy, zz, packed floors (AP_NOKEY: skipped by the insertion loop)
-    const float2 *val;   // slice_value
+    const AgreePx *px;
     int x0, y0;          // pixel of patch entry 0
+    int py;              // patch rows
 };
 
 __device__ __forceinline__ void gather_cell_patch(const float2 *__restrict__ S, const float *m, const AgreePatch &pt,
@@ -936,63 +947,81 @@ __device__ __forceinline__ void gather_cell_patch(const float2 *__restrict__ S, 
     const float t = m[3] * ci + m[4] * cj + m[5] * ck;
     const int xa = max(0, (int)ceilf(s - 1.7330f)), xb = min(H, (int)floorf(s + 1.7330f));
     const int ya = max(-H, (int)ceilf(t - 1.7330f)), yb = min(H - 1, (int)floorf(t + 1.7330f));
-    if (xa < pt.x0 || xb >= pt.x0 + AT_PX || ya < pt.y0 || yb >= pt.y0 + AT_PY) {
+    if (xa < pt.x0 || xb >= pt.x0 + AT_PX || ya < pt.y0 || yb >= pt.y0 + pt.py) {
         gather_cell(S, m, ci, cj, ck, c, weight, etab, rtab, re, im, w);
         return;
     }
     for (int y = ya; y <= yb; y++)
         for (int x = xa; x <= xb; x++) {
             const int e = (y - pt.y0) * AT_PX + (x - pt.x0);
-            const float4 q = pt.pos[e];
-            if (__float_as_int(q.w) == AP_NOKEY) continue;  // radius cut / origin out of range
+            const AgreePx q = pt.px[e];
+            if (q.key == AP_NOKEY) continue;  // radius cut / origin out of range
             const int x0 = (int)floorf(q.x), y0 = (int)floorf(q.y), z0 = (int)floorf(q.z);
             if ((unsigned)(ci - x0) > 1u || (unsigned)(cj - y0) > 1u || (unsigned)(ck - z0) > 1u) continue;
             const float gg = corner_weight(c.mode, ci, cj, ck, q.x, q.y, q.z, c.h, weight, etab);
-            const float2 dt = pt.val[e];
-            re += dt.x * gg;
-            im += dt.y * gg;
+            re += q.v.x * gg;
+            im += q.v.y * gg;
             w += gg;
         }
 }
 
 // Own-plane contributions to unfolded cell (ci, cj, ck), the nearest cell of
-// patch entry e (row pitch PITCH), or its mirror -(ci, cj, ck) gathered
-// around the mirrored pixel.  A stencil that holds the cell starts within 1 of it on every
-// axis, and the cell lies within 0.5 of entry e's position, so the source
-// pixel sits less than 1.5 from that position on every axis: only the
-// in-plane offsets (ox, oy) in [-2, 2]^2 flagged in omask (bit
-// (oy + 2) * 5 + ox + 2, uniform over the slice) can hold it.  Same terms, in
-// the same y-then-x order, as gather_cell_patch.
-template <int PITCH>
-__device__ __forceinline__ void gather_own_offsets(const float4 *pos, const float2 *val, int e, unsigned omask, int ci,
-                                                   int cj, int ck, const InsertConst &c, float weight,
-                                                   const float *etab, float &re, float &im, float &w)
+// patch entry e, or its mirror -(ci, cj, ck) gathered around the mirrored
+// pixel.  A stencil that holds the cell starts
+// within 1 of it on every axis, and the cell lies within 0.5 of entry e's
+// position, so the source pixel sits less than 1.5 from that position on
+// every axis: only the in-plane offsets (ox, oy) in [-2, 2]^2 of
+// own_offset_mask can hold it.  Lane k of `list` holds the k-th of the n
+// offsets, in patch entries times 24 bytes; taken four at a time, so that
+// their reads are in flight together.
+// gauss_2's table index (int)((double)f 50 + 0.5) is read off the sum's bits:
+// with 2^18 added the double's high word ends in the index and two fraction
+// bits, so that word & 0xffc is the entry's byte offset (the sum is exact
+// wherever it could reach the next integer: f 50 is a multiple of 2^-29 from
+// f = 2^-7 on).  Misses read the table too, up to byte 0xffc of the LDS, which
+// the table starts.
+template <int MODE, int N>
+__device__ __forceinline__ void gather_some_offsets(const AgreePx *px, int list, int k0, int kc, float cx, float cy, float cz,
+                                                    float h, float weight, float &re, float &im, float &w)
 {
-    const int kc = ap_key(ci, cj, ck);
-    for (unsigned mm = omask; mm != 0u; mm &= mm - 1u) {  // set bits in increasing order
-        const int k = __builtin_ctz(mm);
-        const int o = e + (k / 5 - 2) * PITCH + (k % 5 - 2);
-        // position, key and value read together; the weight is corner_weight()'s
-        // arithmetic with the table index clamped for the misses it is computed for
-        const float4 q = pos[o];
-        const float2 dt = val[o];
-        const bool hit = ((unsigned)(kc - __float_as_int(q.w)) & ~AP_DIGITS) == 0u;
-        const float dx = (float)ci - q.x, dy = (float)cj - q.y, dz = (float)ck - q.z;
-        float gg;
-        if (c.mode == 0) {
-            const float r = dx * dx + dy * dy + dz * dz;
-            const float f = r * c.h;
-            gg = etab[min((int)__builtin_fma((double)f, 50.0, 0.5), EXPN - 1)] * weight;
+    AgreePx q[N];
+    float g[N];
+#pragma unroll
+    for (int k = 0; k < N; k++)
+        q[k] = *reinterpret_cast<const AgreePx *>(reinterpret_cast<const char *>(px) +
+                                                  __builtin_amdgcn_readlane(list, k0 + k));
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const float dx = cx - q[k].x, dy = cy - q[k].y, dz = cz - q[k].z;
+        if (MODE == 0) {
+            const float f = (dx * dx + dy * dy + dz * dz) * h;
+            const unsigned b = (unsigned)__double2hiint(__builtin_fma((double)f, 50.0, 262144.5)) & 0xffcu;
+            g[k] = *(const __attribute__((address_space(3))) float *)b * weight;
         } else {
-            gg = (float)((1.0 - (double)fabsf(dx)) * (1.0 - (double)fabsf(dy)) * (1.0 - (double)fabsf(dz)) *
-                         (double)weight);
-        }
-        if (hit) {
-            re += dt.x * gg;
-            im += dt.y * gg;
-            w += gg;
+            g[k] = (float)((1.0 - (double)fabsf(dx)) * (1.0 - (double)fabsf(dy)) * (1.0 - (double)fabsf(dz)) *
+                           (double)weight);
         }
     }
+    // each term as the insertion adds it, so that a voxel only this particle reached cancels to 0
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const float gg = ((unsigned)(kc - q[k].key) & ~AP_DIGITS) == 0u ? g[k] : 0.f;
+        re += q[k].v.x * gg;
+        im += q[k].v.y * gg;
+        w += gg;
+    }
+}
+
+template <int MODE>
+__device__ __forceinline__ void gather_own_offsets(const AgreePx *px, int list, int n, int ci, int cj, int ck, float h,
+                                                   float weight, float &re, float &im, float &w)
+{
+    const int kc = ap_key(ci, cj, ck);
+    const float cx = (float)ci, cy = (float)cj, cz = (float)ck;
+    int k = 0;
+    for (; k + 4 <= n; k += 4) gather_some_offsets<MODE, 4>(px, list, k, kc, cx, cy, cz, h, weight, re, im, w);
+    if (n & 2) gather_some_offsets<MODE, 2>(px, list, k, kc, cx, cy, cz, h, weight, re, im, w);
+    if (n & 1) gather_some_offsets<MODE, 1>(px, list, n - 1, kc, cx, cy, cz, h, weight, re, im, w);
 }
 
 // Offsets (ox, oy) in [-2, 2]^2 whose step ox * row0 + oy * row1 of slice
@@ -1008,6 +1037,16 @@ __device__ __forceinline__ unsigned own_offset_mask(const float *m)
         ok = fmaxf(fabsf(d0), fmaxf(fabsf(d1), fabsf(d2))) < 1.51f;
     }
     return (unsigned)__ballot(ok);
+}
+
+// Lane k: the k-th set bit's offset in patch entries of row pitch `pitch`, times 24 bytes.
+__device__ __forceinline__ int own_offset_list(unsigned mask, int pitch)
+{
+    const int b = threadIdx.x & 63;
+    const int o = (int)sizeof(AgreePx) * ((b / 5 - 2) * pitch + (b % 5 - 2));
+    // lane b < 25 with its bit set sends its offset to lane (bits below b), the others to lane 63
+    const int to = b < 25 && (mask >> b & 1u) ? __popc(mask & ((1u << b) - 1u)) : 63;
+    return __builtin_amdgcn_ds_permute(to << 2, o);
 }
 
 // own_contribution() with the slice's own plane gathered from the patch.
@@ -1072,79 +1111,139 @@ __device__ void own_contribution_tile(const float2 *S, const float *t3dp, int ns
         }
 }
 
-// One workgroup per (32 x 16 compare-pixel tile, particle x symmetry op
-// slice); eight double sums per particle accumulated with float64 atomics
-// into acc[p][8].
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_agree_batch(const float2 *__restrict__ slices, int nsym,
-                                                     const float *__restrict__ t3d, const float *__restrict__ wq,
-                                                     InsertConst c, float rmax, int sub,
-                                                     const float2 *__restrict__ data, const float *__restrict__ norm,
-                                                     const float *__restrict__ exptab, const float *__restrict__ rtab_g,
-                                                     double *__restrict__ acc_out)
+// Voxel (x, y, z) of the packed volume: cubes of 2^3 voxels, 128 bytes, so that the nearest voxels of a
+// slice's plane fall in few cache lines.  (P even; fewer than 2^30 entries for P <= 1024.)
+__device__ __forceinline__ unsigned pack_index(unsigned x, unsigned y, unsigned z, int P)
 {
+    const unsigned H = P / 2;
+    return (((z >> 1) * H + (y >> 1)) * (H / 2 + 1) + (x >> 1)) * 8 + ((z & 1) << 2 | (y & 1) << 1 | (x & 1));
+}
+
+// One workgroup per (compare-pixel tile, particle x symmetry op slice); eight
+// double sums per particle accumulated with float64 atomics into acc[p][8].
+// vol: the volume as float4 (re, im, weight, 0) per voxel, or null, then data
+// and norm are read.  n3: the low-resolution band is 9 < x^2 + y^2 < n3.
+// Bound: VALU issue (92 % at pad 600), then the volume's cache lines.  8,000
+// slices at pad 600: 36.5 ms before, 23.8 now.  What it took: the voxels read
+// before the patch is staged and at most 80 registers (3 workgroups of 8 waves
+// per CU; 34 ms with 2), the packed volume in 2^3 cubes (0.60 G instead of
+// 0.92 G line misses; data and weights read apart: 33.4 ms), offsets in groups
+// of four so that their LDS reads overlap, 32 x 32 tiles (halo 1.27 instead of
+// 1.41).  1,500 particles of d2 at pad 192: 7.1 -> 5.6 ms, the other planes'
+// gather by full waves (with the volume as it is 5.7).
+template <int MODE, bool SYM, bool PACKED>
+__global__ void __launch_bounds__(AgreeTile<SYM ? 16 : 32>::THREADS) __attribute__((amdgpu_waves_per_eu(SYM ? 5 : 6)))
+    k_agree_batch(const float2 *__restrict__ slices, int nsym, const float *__restrict__ t3d, const float *__restrict__ wq,
+                  InsertConst c, int n3, int sub, const float2 *__restrict__ data, const float *__restrict__ norm,
+                  const float4 *__restrict__ vol, const float *__restrict__ exptab, const float *__restrict__ rtab_g,
+                  double *__restrict__ acc_out)
+{
+    constexpr int AY = SYM ? 16 : 32;
+    using AT = AgreeTile<AY>;
     const int H = c.H, P = c.P;
     const int q = blockIdx.y, p = q / nsym, own = q - p * nsym;
     const int W = H + 2;
     const int ntx = (W + AT_X - 1) / AT_X;
-    const int tx0 = (blockIdx.x % ntx) * AT_X, ty0 = (int)(blockIdx.x / ntx) * AT_Y - H;
+    const int tx0 = (blockIdx.x % ntx) * AT_X, ty0 = (int)(blockIdx.x / ntx) * AY - H;
     const float2 *S = slices + (size_t)p * P * (H + 1);
     const float *t3dp = t3d + 9 * (size_t)p * nsym;
     const float *m = t3d + 9 * (size_t)q;
     const float weight = wq[q];
-    // LDS: patch positions and values, mirror patch positions and values,
-    // fast_exp and fl(i/P) tables
+    // dynamic LDS, from address 0: fast_exp table, patch, mirror patch, queued compare pixels, near planes;
+    // with symmetry each wave's queue and sums of the other planes
     extern __shared__ float4 agree_lds[];
-    float4 *ppos = agree_lds;
-    float2 *pval = reinterpret_cast<float2 *>(ppos + AT_PATCH);
-    float *etab = reinterpret_cast<float *>(ppos + AT_PATCH + AT_PATCH / 2 + AT_MPATCH + AT_MPATCH / 2);
-    float *rtab = etab + EXPN;
-    for (int i = threadIdx.x; i < EXPN; i += blockDim.x) etab[i] = exptab[i];
-    for (int i = threadIdx.x; i < P + 2; i += blockDim.x) rtab[i] = rtab_g[i];
-    __syncthreads();
-    AgreePatch pt{ppos, pval, tx0 - AT_HALO, ty0 - AT_HALO};
-    __shared__ unsigned short dq[AT_X * AT_Y];  // queued compare pixels (tile index)
-    __shared__ int dn;
-    if (threadIdx.x == 0) dn = 0;
+    float *etab = reinterpret_cast<float *>(agree_lds);
+    AgreePx *ppx = reinterpret_cast<AgreePx *>(etab + EXPN);
+    AgreePx *mpx = ppx + AT::PATCH;
+    unsigned long long *near_ops = reinterpret_cast<unsigned long long *>(mpx + AT::MPATCH);  // 64 words
+    int *dn = reinterpret_cast<int *>(near_ops + 64);
+    unsigned short *dq = reinterpret_cast<unsigned short *>(dn + 2);  // AT_X * AY queued compare pixels (tile index)
+    // with symmetry: fl(i/P), the pixels' cells (keys), the sums and the queue of the other planes
+    constexpr int NPX = AT_X * AY, QUEUE = 3 * NPX;
+    float *rtab_l = reinterpret_cast<float *>(dq + NPX);
+    int *cell = reinterpret_cast<int *>(rtab_l + P + 2);
+    float *osum = reinterpret_cast<float *>(cell + NPX);
+    int *queue = reinterpret_cast<int *>(osum + 3 * NPX);
+    const float *rtab = SYM ? rtab_l : rtab_g;
+    if (SYM) {
+        for (int i = threadIdx.x; i < P + 2; i += AT::THREADS) rtab_l[i] = rtab_g[i];
+        for (int i = threadIdx.x; i < 3 * NPX; i += AT::THREADS) osum[i] = 0.f;
+    }
+    for (int i = threadIdx.x; i < EXPN; i += AT::THREADS) etab[i] = exptab[i];
+    AgreePatch pt{ppx, tx0 - AT_HALO, ty0 - AT_HALO, AT::PY};
+    if (threadIdx.x == 0) dn[0] = dn[1] = 0;
     // packed floor keys need |x0|, |y0|, |z0| <= 511
     const bool fastkeys = sub && H <= 510;
     const unsigned omask = fastkeys ? own_offset_mask(m) : 0u;
-    auto stage = [&](int x, int y, float4 &pos, float2 &val) {
-        pos = make_float4(0.f, 0.f, 0.f, __int_as_float(AP_NOKEY));
-        val = make_float2(0.f, 0.f);
-        // the insertion loop's pixels: x in [0, P/2], y in [-P/2, P/2), radius cut (corners off here)
-        if (x >= 0 && x <= H && y >= -H && y <= H - 1 && x * x + y * y <= H * H + H) {
-            float xx, yy, zz;
-            pixel_coords(x, y, m, rtab, H, c.Pf, xx, yy, zz);
-            const int x0 = (int)floorf(xx), y0 = (int)floorf(yy), z0 = (int)floorf(zz);
-            const bool in = !(x0 < -H - 1 || y0 < -H - 1 || z0 < -H - 1 || x0 > H || y0 > H || z0 > H);
-            pos = make_float4(xx, yy, zz, __int_as_float(in ? ap_key(x0, y0, z0) : AP_NOKEY));
-            if (in) val = slice_value(S, x, y, P, H);
+    const int olist = own_offset_list(omask, AT_PX), on = __popc(omask);
+    auto stage = [&](int x, int y, AgreePx &e) {
+        AgreePx o{0.f, 0.f, 0.f, AP_NOKEY, make_float2(0.f, 0.f)};
+        // the insertion loop's pixels: x in [0, P/2], y in [-P/2, P/2), radius cut (corners off here; it
+        // bounds |x| and |y| by P/2)
+        if (x >= 0 && y < H && x * x + y * y <= H * H + H) {
+            pixel_coords(x, y, m, rtab_g, H, c.Pf, o.x, o.y, o.z);
+            // origins in [-P/2 - 1, P/2]
+            if (fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z))) < (float)(H + 1)) {
+                o.key = ap_key((int)floorf(o.x), (int)floorf(o.y), (int)floorf(o.z));
+                const bool cj = x == 0 && y < 0;  // slice_value
+                o.v = S[(unsigned)(cj ? -y : (y < 0 ? P + y : y)) * (unsigned)(H + 1) + (unsigned)x];
+                if (cj) o.v.y = -o.v.y;
+            }
         }
+        e = o;
     };
-    for (int e = threadIdx.x; e < AT_PATCH; e += blockDim.x)
-        stage(pt.x0 + e % AT_PX, pt.y0 + e / AT_PX, ppos[e], pval[e]);
-    float4 *mpos = ppos + AT_PATCH + AT_PATCH / 2;  // after pval
-    float2 *mval = reinterpret_cast<float2 *>(mpos + AT_MPATCH);
-    const int my0 = -ty0 - AT_Y - 1;
+    // own contributions reach compare pixels within the insertion radius plus sqrt(3) (a stencil) plus
+    // sqrt(3) / 2 (the nearest cell): beyond, the tile's patch is not needed
+    const int rown2 = (H + 4) * (H + 4);
+    const int ny0 = ty0 > 0 ? ty0 : (ty0 + AY - 1 < 0 ? ty0 + AY - 1 : 0);  // the tile's row nearest 0
+    const bool inner = sub && tx0 * tx0 + ny0 * ny0 <= rown2;
+    const int my0 = -ty0 - AY - 1;
     const bool mirror = fastkeys && tx0 == 0;
-    if (mirror)
-        for (int e = threadIdx.x; e < AT_MPATCH; e += blockDim.x)
-            stage(e % AT_MX - 4, my0 + e / AT_MX, mpos[e], mval[e]);
-    __syncthreads();
-    double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    // One compare pixel.  Outside the general pass a pixel whose voxel needs
-    // the general own-contribution enumeration returns false untouched, to be
-    // queued: the few such pixels of a tile (x < 3, voxels on the x = 0,
-    // x = P/2 and y, z = P/2 planes) then share waves instead of holding back
-    // every wave they fall in.
-    auto pixel = [&](int x, int y, bool general) -> bool {
-        const float rx = rtab[x + H], ry = rtab[y + H];
+    // the other symmetry planes that pass within reach of the tile's nearest cells: |n . p| <= sqrt(3)
+    // (gather_cell's bound) + sqrt(3) / 2
+    const int lane = threadIdx.x & 63;
+    const int nwords = (nsym + 63) / 64;  // symmetries of more than 4096 operators take every plane
+    if (SYM && fastkeys && nwords <= 64) {
+        for (int wd = threadIdx.x >> 6; wd < nwords; wd += AT::WAVES) {
+            const int sop = 64 * wd + lane;
+            bool hit = false;
+            if (sop < nsym && sop != own) {
+                const float *o = t3dp + 9 * sop;
+                const float n0 = o[1] * o[5] - o[2] * o[4], n1 = o[2] * o[3] - o[0] * o[5], n2 = o[0] * o[4] - o[1] * o[3];
+                const float a = n0 * m[0] + n1 * m[1] + n2 * m[2], b = n0 * m[3] + n1 * m[4] + n2 * m[5];
+                const float xa = a * (float)tx0, xb = a * (float)(tx0 + AT_X - 1);
+                const float ya = b * (float)ty0, yb = b * (float)(ty0 + AY - 1);
+                hit = fminf(xa, xb) + fminf(ya, yb) <= 2.62f && fmaxf(xa, xb) + fmaxf(ya, yb) >= -2.62f;
+            }
+            const unsigned long long hm = __ballot(hit);
+            if (lane == 0) near_ops[wd] = hm;
+        }
+    }
+    double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+    int nval = 0;
+    // One compare pixel: load() takes its voxel and slice value, compare() its own contribution and the
+    // sums.  Outside the general pass a pixel whose voxel needs the general own-contribution enumeration is
+    // left for later (the few such pixels of a tile, voxels on the x = P/2 and y, z = P/2 planes, then share
+    // waves instead of holding back every wave they fall in).
+    struct Pixel {
+        int l, x, y, x0, y0, z0;
+        bool now, later;
+        float vr, vi, nv;
+        float2 d;
+    };
+    auto load = [&](Pixel &a, bool valid, int x, int y, bool general) {
+        a.x = x;
+        a.y = y;
+        const float rx = valid ? rtab_g[x + H] : 0.f, ry = valid ? rtab_g[y + H] : 0.f;
         const float c0 = rx * m[0] + ry * m[3];
         const float c1 = rx * m[1] + ry * m[4];
         const float c2 = rx * m[2] + ry * m[5];
-        if (fabsf(c0) > 0.5f || fabsf(c1) >= 0.5f || fabsf(c2) >= 0.5f) return true;
-        const float xx = c0 * c.Pf, yy = c1 * c.Pf, zz = c2 * c.Pf;
-        const int x0 = round_ref(xx), y0 = round_ref(yy), z0 = round_ref(zz);
+        valid = valid && !(fabsf(c0) > 0.5f || fabsf(c1) >= 0.5f || fabsf(c2) >= 0.5f);
+        // Util::round: half away from zero
+        a.x0 = (int)(c0 * c.Pf + copysignf(0.5f, c0));
+        a.y0 = (int)(c1 * c.Pf + copysignf(0.5f, c1));
+        a.z0 = (int)(c2 * c.Pf + copysignf(0.5f, c2));
+        const int x0 = a.x0, y0 = a.y0, z0 = a.z0;
         // Common voxel: |x0|, |y0|, |z0| < P/2 leave one direct and one
         // mirrored source cell, +-(x0, y0, z0) (on x0 = 0 the mirrored one
         // through the double insertion's conjugate copy, value only).  From
@@ -1152,143 +1251,266 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
         // cell, whose in-plane distance exceeds sqrt(3) + sqrt(3)/2; below,
         // its sources lie around (-x, -y), in the mirror patch.
         const bool common = fastkeys && (x >= 3 || mirror) && abs(x0) < H && abs(y0) < H && abs(z0) < H;
-        if (sub && !general && !common) return false;
-        const float *Sf = reinterpret_cast<const float *>(S);
-        const int slen = (P + 2) * P;
-        const int fidx = 2 * x + (P + 2) * (y < 0 ? P + y : y);
-        const float d20 = fidx < slen ? Sf[fidx] : 0.f;
-        const float d21 = fidx + 1 < slen ? Sf[fidx + 1] : 0.f;
-        int xs, ysn, zsn;
-        if (x0 < 0) {
-            xs = -x0;
-            ysn = y0 <= 0 ? -y0 : P - y0;
-            zsn = z0 <= 0 ? -z0 : P - z0;
-        } else {
-            xs = x0;
-            ysn = y0 < 0 ? P + y0 : y0;
-            zsn = z0 < 0 ? P + z0 : z0;
-        }
-        const size_t ci = cidx(xs, ysn, zsn, P, H);
-        float vr = 0.f, vi = 0.f;
-        const bool inb = !(abs(x0) >= H + 1 || abs(y0) > H || abs(z0) > H);
-        if (inb) {
-            const float2 v = data[ci];
-            vr = v.x;
-            vi = v.y;
-        }
-        float nv = norm[ci];
-        if (sub) {
-            float ore, oim, ow;
-            if (general) {
-                own_contribution_tile(S, t3dp, nsym, own, pt, xs, ysn, zsn, c, weight, etab, rtab, ore, oim, ow);
+        a.later = valid && sub && !general && !common;
+        a.now = valid && !a.later;
+        a.vr = a.vi = a.nv = 0.f;
+        a.d = make_float2(0.f, 0.f);
+        if (a.now) {
+            // the slice's floats 2x, 2x + 1 of row y; x = P/2 + 1 reads the next row's first, past the last row 0
+            const unsigned fidx = (unsigned)(y < 0 ? P + y : y) * (unsigned)(H + 1) + (unsigned)x;
+            if (fidx < (unsigned)P * (unsigned)(H + 1)) a.d = S[fidx];
+            const int sg = x0 < 0 ? -1 : 1;
+            const int ys = sg * y0, zs = sg * z0;
+            const unsigned zi = (unsigned)(zs < 0 ? P + zs : zs), yi = (unsigned)(ys < 0 ? P + ys : ys);
+            const unsigned xi = (unsigned)(sg * x0);
+            if (PACKED) {
+                const float4 v = vol[pack_index(xi, yi, zi, P)];
+                a.vr = v.x;
+                a.vi = v.y;
+                a.nv = v.z;
             } else {
-                const int e = (y - pt.y0) * AT_PX + (x - pt.x0);
-                float r = 0.f, i = 0.f, w = 0.f, r2 = 0.f, i2 = 0.f, w2 = 0.f;
-                for (int sop = 0; sop < nsym; sop++) {
-                    if (sop == own) {
-                        gather_own_offsets<AT_PX>(ppos, pval, e, omask, x0, y0, z0, c, weight, etab, r, i, w);
-                        if (x < 3)  // mirror patch entry of (-x, -y)
-                            gather_own_offsets<AT_MX>(mpos, mval, 4 - x + (-y - my0) * AT_MX, omask, -x0, -y0, -z0,
-                                                      c, weight, etab, r2, i2, w2);
-                    } else {
-                        gather_cell(S, t3dp + 9 * sop, x0, y0, z0, c, weight, etab, rtab, r, i, w);
-                        gather_cell(S, t3dp + 9 * sop, -x0, -y0, -z0, c, weight, etab, rtab, r2, i2, w2);
-                    }
-                }
-                if (x0 >= 0) {  // direct cell (x0, y0, z0), mirrored -(x0, y0, z0)
-                    ore = r + r2;
-                    oim = i - i2;
-                    ow = x0 == 0 ? w : w + w2;
-                } else {
-                    ore = r2 + r;
-                    oim = i2 - i;
-                    ow = w2 + w;
-                }
+                const unsigned ci = (zi * P + yi) * (unsigned)(H + 1) + xi;  // P^2 (P/2 + 1) < 2^30
+                const float2 v = data[ci];
+                a.vr = v.x;
+                a.vi = v.y;
+                a.nv = norm[ci];
             }
-            if (inb) {
-                vr = vr - ore;
-                vi = vi - oim;
-            }
-            nv = nv - ow;
         }
-        if (x0 < 0) vi = -vi;  // get_complex_at conjugate for x<0
-        if (nv != 0.f) {
-            const float dt0 = __fdiv_rn(vr, nv), dt1 = __fdiv_rn(vi, nv), dt2 = nv;
-            const float r = sqrt_int_rn(x * x + y * y);  // Util::hypot_fast
-            const float dotv = (dt0 * d20 + dt1 * d21) * dt2;
-            const float pw = (dt0 * dt0 + dt1 * dt1) * dt2;
-            const float pw2 = (d20 * d20 + d21 * d21) * dt2;
-            if (r > 3 && r < rmax) {
+    };
+    auto compare = [&](Pixel &a, bool general) {
+        const int x0 = a.x0, y0 = a.y0, z0 = a.z0, r2d = a.x * a.x + a.y * a.y;
+        const bool reach = a.now && r2d <= rown2;
+        if (sub) {
+            float ore = 0.f, oim = 0.f, ow = 0.f;
+            if (general) {
+                if (reach) {
+                    const int sg = x0 < 0 ? -1 : 1, ys = sg * y0, zs = sg * z0;
+                    own_contribution_tile(S, t3dp, nsym, own, pt, sg * x0, ys < 0 ? P + ys : ys, zs < 0 ? P + zs : zs, c,
+                                          weight, etab, rtab, ore, oim, ow);
+                }
+            } else {
+                float r = 0.f, i = 0.f, w = 0.f, r2 = 0.f, i2 = 0.f, w2 = 0.f;
+                if (__ballot(reach)) {
+                    // lanes without a pixel in reach gather around entry 0, in bounds, and drop the sums
+                    const int e = reach ? (a.y - pt.y0) * AT_PX + (a.x - pt.x0) : 2 * AT_PX + 2;
+                    gather_own_offsets<MODE>(ppx + e, olist, on, x0, y0, z0, c.h, weight, r, i, w);
+                    const bool low = reach && a.x < 3;
+                    if (__ballot(low)) {  // mirror patch entry of (-x, -y)
+                        const int e2 = low ? 4 - a.x + (-a.y - my0) * AT_MX : 2 * AT_MX + 2;
+                        gather_own_offsets<MODE>(mpx + e2, own_offset_list(omask, AT_MX), on, -x0, -y0, -z0, c.h, weight, r2, i2,
+                                                 w2);
+                    }
+                    if (!reach) r = i = w = 0.f;
+                    if (!low) r2 = i2 = w2 = 0.f;
+                }
+                // direct cell (x0, y0, z0) and mirrored -(x0, y0, z0), the volume's voxel being the mirrored
+                // one of a cell with x0 < 0
+                ore = r + r2;
+                oim = i - i2;
+                ow = x0 == 0 ? w : w + w2;
+                if (SYM && reach) {
+                    ore += osum[a.l];
+                    oim += osum[NPX + a.l];
+                    ow += osum[2 * NPX + a.l];
+                }
+                oim = x0 >= 0 ? oim : -oim;
+            }
+            a.vr = a.vr - ore;
+            a.vi = a.vi - oim;
+            a.nv = a.nv - ow;
+        }
+        const float vr = a.vr, vi = x0 < 0 ? -a.vi : a.vi, nv = a.nv;  // get_complex_at conjugate for x<0
+        if (a.now && nv != 0.f) {
+            // value v over weight nv against d: dot and powers weighted by nv, nv cancelled once
+            const float dotv = vr * a.d.x + vi * a.d.y;
+            const float pw = __fdiv_rn(vr * vr + vi * vi, nv);
+            const float pw2 = (a.d.x * a.d.x + a.d.y * a.d.y) * nv;
+            if (r2d > 9 && r2d < n3) {  // 3 < hypot_fast(x, y) < rmax
                 acc[4] += dotv;
                 acc[5] += pw;
                 acc[6] += pw2;
             }
-            acc[1] += dt2;
+            acc[1] += nv;
             acc[0] += dotv;
             acc[2] += pw;
             acc[3] += pw2;
-            acc[7] += 1.0;
+            nval++;
         }
-        return true;
     };
-    // tile slot l -> pixel; in the x = 0 tiles the first 48 slots are the
-    // columns x < 3 of all 16 rows, so that only one wave runs their mirrored
-    // gather
+    // tile slot l -> pixel; in the x = 0 tiles the first slots are the columns
+    // x < 3 of all rows, so that few waves run their mirrored gather
     auto slot = [&](int l, int &x, int &y) {
         if (tx0 == 0) {
-            if (l < 3 * AT_Y) {
+            if (l < 3 * AY) {
                 x = l % 3;
                 y = ty0 + l / 3;
             } else {
-                x = 3 + (l - 3 * AT_Y) % (AT_X - 3);
-                y = ty0 + (l - 3 * AT_Y) / (AT_X - 3);
+                x = 3 + (l - 3 * AY) % (AT_X - 3);
+                y = ty0 + (l - 3 * AY) / (AT_X - 3);
             }
         } else {
             x = tx0 + l % AT_X;
             y = ty0 + l / AT_X;
         }
     };
-    for (int it = 0; it < AT_Y * AT_X / 256; it++) {
-        const int l = threadIdx.x + it * 256;
+    // the voxels are read before the patch is staged: their latency runs beside it
+    constexpr int NP = AY * AT_X / AT::THREADS;
+    Pixel px[NP];
+#pragma unroll
+    for (int it = 0; it < NP; it++) {
         int x, y;
-        slot(l, x, y);
-        if (x >= W || y >= H || (x == 0 && y == 0)) continue;
-        if (!pixel(x, y, false)) dq[atomicAdd(&dn, 1)] = (unsigned short)l;
+        slot(threadIdx.x + it * AT::THREADS, x, y);
+        px[it].l = threadIdx.x + it * AT::THREADS;
+        load(px[it], x < W && y < H && !(x == 0 && y == 0), x, y, false);
+        if (SYM) cell[px[it].l] = ap_key(px[it].x0, px[it].y0, px[it].z0);
+    }
+    if (inner)
+        for (int e = threadIdx.x; e < AT::PATCH; e += AT::THREADS)
+            stage(pt.x0 + e % AT_PX, pt.y0 + e / AT_PX, ppx[e]);
+    if (mirror && inner)
+        for (int e = threadIdx.x; e < AT::MPATCH; e += AT::THREADS)
+            stage(e % AT_MX - 4, my0 + e / AT_MX, mpx[e]);
+    __syncthreads();
+    if (SYM && fastkeys && inner) {
+        // The other planes' contributions to the pixels' nearest cells and their mirrors: the (pixel, plane,
+        // sign) triples whose cell lies within the plane's reach are queued, so that full waves run the
+        // gather for the few pixels along the planes' intersections, and summed per pixel: value of the
+        // cell minus the conjugate of its mirror's, weights (the mirror's not on x0 = 0).  What the queue
+        // does not hold is gathered at once.
+        auto gather = [&](int e) {
+            const int l = e & (NPX - 1), kc = cell[l], is = e >> 10 & 1 ? -1 : 1;
+            const int x0 = (kc & 1023) - 512, y0 = (kc >> 10 & 1023) - 512, z0 = (kc >> 20) - 512;
+            float a = 0.f, b = 0.f, g = 0.f;
+            gather_cell(S, t3dp + 9 * (e >> 11), is * x0, is * y0, is * z0, c, weight, etab, rtab, a, b, g);
+            if (a != 0.f || b != 0.f || g != 0.f) {
+                atomicAdd(&osum[l], a);
+                atomicAdd(&osum[NPX + l], is < 0 ? -b : b);
+                if (is > 0 || x0 != 0) atomicAdd(&osum[2 * NPX + l], g);
+            }
+        };
+        for (int wd = 0; wd < nwords; wd++) {
+            for (unsigned long long ops = nwords <= 64 ? near_ops[wd] : ~0ull; ops; ops &= ops - 1) {
+                const int sop = 64 * wd + __builtin_ctzll(ops);
+                if (sop >= nsym) break;
+                if (sop == own) continue;
+                const float *o = t3dp + 9 * sop;
+                const float n0 = o[1] * o[5] - o[2] * o[4], n1 = o[2] * o[3] - o[0] * o[5], n2 = o[0] * o[4] - o[1] * o[3];
+#pragma unroll
+                for (int it = 0; it < NP; it++) {
+                    const Pixel &a = px[it];
+                    const bool slab = a.now && a.x * a.x + a.y * a.y <= rown2 &&
+                                      !(fabsf(n0 * a.x0 + n1 * a.y0 + n2 * a.z0) > 1.7330f);
+                    const float s = o[0] * a.x0 + o[1] * a.y0 + o[2] * a.z0;  // gather_cell's x range is not empty
+#pragma unroll
+                    for (int sgn = 0; sgn < 2; sgn++) {
+                        const bool hit = slab && (sgn ? s <= 1.74f : s >= -1.74f);
+                        const unsigned long long hm = __ballot(hit);
+                        if (!hm) continue;
+                        int base = 0;
+                        if (lane == 0) base = atomicAdd(&dn[1], __popcll(hm));
+                        base = __builtin_amdgcn_readfirstlane(base) + __popcll(hm & ((1ull << lane) - 1ull));
+                        if (hit) {
+                            const int e = a.l | sgn << 10 | sop << 11;
+                            if (base < QUEUE) queue[base] = e;
+                            else gather(e);
+                        }
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        const int n = min(dn[1], QUEUE);
+        for (int k = threadIdx.x; k < n; k += AT::THREADS) gather(queue[k]);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int it = 0; it < NP; it++) {
+        compare(px[it], false);
+        if (px[it].later) dq[atomicAdd(dn, 1)] = (unsigned short)(threadIdx.x + it * AT::THREADS);
     }
     __syncthreads();
-    for (int j = threadIdx.x; j < dn; j += blockDim.x) {
+    for (int j = threadIdx.x; j < *dn; j += AT::THREADS) {
         int x, y;
         slot(dq[j], x, y);
-        pixel(x, y, true);
+        Pixel a;
+        load(a, true, x, y, true);
+        compare(a, true);
     }
-    // block sums through LDS (the patch's space, no longer read): 32 threads
-    // per sum add 8 of the 256 partials each, then a 32-lane butterfly
+    // block sums through LDS (the patch's space, no longer read): a wave per sum, or two sums per wave
     __syncthreads();
-    static_assert((sizeof(float4) + sizeof(float2)) * AT_PATCH >= 8 * 256 * sizeof(double), "block sums");
-    double *red = reinterpret_cast<double *>(agree_lds);  // 8 x 256 doubles within the patch's bytes
+    static_assert(sizeof(AgreePx) * (AT::PATCH + AT::MPATCH) >= 8 * AT::THREADS * sizeof(double), "block sums");
+    double *red = reinterpret_cast<double *>(ppx);  // 8 x THREADS doubles within the patches' bytes
 #pragma unroll
-    for (int k = 0; k < 8; k++) red[k * 256 + threadIdx.x] = acc[k];
+    for (int k = 0; k < 7; k++) red[k * AT::THREADS + threadIdx.x] = acc[k];
+    red[7 * AT::THREADS + threadIdx.x] = (double)nval;
     __syncthreads();
-    const int k = threadIdx.x >> 5, l = threadIdx.x & 31;
+    constexpr int PER = AT::THREADS / 8;  // threads per sum: 64 or 32
+    const int k = threadIdx.x / PER, l = threadIdx.x % PER;
     double v = 0.0;
 #pragma unroll
-    for (int i = 0; i < 8; i++) v += red[k * 256 + l + 32 * i];
+    for (int i = 0; i < 8; i++) v += red[k * AT::THREADS + l + PER * i];
 #pragma unroll
-    for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    for (int o = PER / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if (l == 0) unsafeAtomicAdd(&acc_out[(size_t)p * 8 + k], v);
+}
+
+// One thread per entry, the 8 of a cube consecutive; cubes past x = P/2 (P/2 even) are half filled.
+__global__ void __launch_bounds__(256) k_pack_volume(const float2 *__restrict__ data, const float *__restrict__ norm, int P,
+                                                     float4 *__restrict__ vol)
+{
+    const unsigned H = P / 2, nbx = H / 2 + 1, n = nbx * H * H * 8;
+    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const unsigned b = i >> 3, x = 2 * (b % nbx) + (i & 1), yz = b / nbx;
+        const unsigned y = 2 * (yz % H) + (i >> 1 & 1), z = 2 * (yz / H) + (i >> 2 & 1);
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (x <= H) {
+            const unsigned ci = (z * P + y) * (H + 1) + x;
+            const float2 d = data[ci];
+            v = make_float4(d.x, d.y, norm[ci], 0.f);
+        }
+        vol[i] = v;
+    }
+}
+
+size_t pack_elems(int P) { return (size_t)(P / 4 + 1) * (P / 2) * (P / 2) * 8; }
+
+hipError_t launch_pack_volume(const float2 *data, const float *norm, int P, float4 *vol, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_pack_volume, dim3(8192), dim3(256), 0, s, data, norm, P, vol);
+    return hipGetLastError();
 }
 
 hipError_t launch_agree_batch(const float2 *slices, int nsym, const float *t3d, const float *wq, int nslices,
                               InsertConst c, float rmax, int sub, const float2 *data, const float *norm,
-                              const float *exptab, const float *rtab, double *acc, hipStream_t s)
+                              const float4 *vol, const float *exptab, const float *rtab, double *acc, hipStream_t s)
 {
     if (nslices <= 0) return hipSuccess;
     c.corners = 0;
-    const int ntx = (c.P / 2 + 2 + AT_X - 1) / AT_X, nty = (c.P + AT_Y - 1) / AT_Y;
-    const size_t lds = (sizeof(float4) + sizeof(float2)) * (AT_PATCH + AT_MPATCH) + sizeof(float) * (EXPN + c.P + 2);
-    hipLaunchKernelGGL(k_agree_batch, dim3(ntx * nty, nslices), dim3(256), lds, s, slices, nsym, t3d, wq, c, rmax, sub,
-                       data, norm, exptab, rtab, acc);
-    return hipGetLastError();
+    // the first n whose root, rounded to float, is not below rmax
+    int n3 = std::max(0, (int)((double)rmax * rmax) - 2);
+    while ((float)sqrt((double)n3) < rmax) n3++;
+    const bool sym = nsym > 1;
+    const int AY = sym ? 16 : 32;
+    const int ntx = (c.P / 2 + 2 + AT_X - 1) / AT_X, nty = (c.P + AY - 1) / AY;
+    const size_t patch = sym ? AgreeTile<16>::PATCH + AgreeTile<16>::MPATCH : AgreeTile<32>::PATCH + AgreeTile<32>::MPATCH;
+    const size_t lds = sizeof(float) * EXPN + sizeof(AgreePx) * patch + 8 * 64 + 8 + sizeof(short) * AT_X * AY +
+                       (sym ? sizeof(float) * (c.P + 2 + (1 + 3 + 3) * AT_X * AY) : 0);
+#define FH_AGREE(M, S, K)                                                                                               \
+    if (c.mode == M && sym == S && (vol != nullptr) == K) {                                                             \
+        hipLaunchKernelGGL((k_agree_batch<M, S, K>), dim3(ntx * nty, nslices), dim3(16 * AY), lds, s, slices, nsym, t3d, \
+                           wq, c, n3, sub, data, norm, vol, exptab, rtab, acc);                                         \
+        return hipGetLastError();                                                                                       \
+    }
+    FH_AGREE(0, false, false)
+    FH_AGREE(0, false, true)
+    FH_AGREE(0, true, false)
+    FH_AGREE(0, true, true)
+    FH_AGREE(1, false, false)
+    FH_AGREE(1, false, true)
+    FH_AGREE(1, true, false)
+    FH_AGREE(1, true, true)
+#undef FH_AGREE
+    return hipErrorInvalidValue;
 }
 
 // ------------------------------------------------------------ projection
@@ -1921,13 +2143,6 @@ template <int A>
 __device__ __forceinline__ int acc_slot(int i, int j, int k)
 {
     return A == 0 ? (i * HALO + k) * HALO + j : (A == 1 ? (j * HALO + k) * HALO + i : (k * HALO + j) * HALO + i);
-}
-
-__device__ __forceinline__ void wave_sync_lds()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Wave64 inclusive scans on DPP (GFX9 row shifts and row broadcasts): no
