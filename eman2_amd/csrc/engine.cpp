@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "fh_launch.hpp"
+#include "host_pool.hpp"
 
 using namespace fh;
 
@@ -343,9 +344,10 @@ struct fh_reconstructor {
     fh_tuning tune{2, 1024, 0, 8, 0};
     fh_stats stats{};
     hipEvent_t ev[6] = {};
-    // pinned staging for large device-to-host copies (two buffers, one event each)
-    float *pin[2] = {nullptr, nullptr};
-    hipEvent_t pin_ev[2] = {};
+    // blocks, streams, pinned staging and copy threads shared with other handles
+    HostPool::Ref pool = HostPool::get();
+    char *pin = nullptr;                              // staging ring
+    hipEvent_t pin_ev[HostPool::PIN_SLOTS] = {};      // the last copy through each slot
 };
 
 #define FH_TRY(h, expr)                                                                    \
@@ -365,73 +367,79 @@ static int fail(fh_reconstructor *h, int code, const std::string &msg)
 
 static size_t vol_elems(int P) { return (size_t)P * P * (P / 2 + 1); }
 
-// Device-to-host copy of `bytes` into caller (pageable) memory: through two
-// pinned staging buffers, the DMA of one chunk running while several host
-// threads copy the previous chunk out; small copies go directly.
-constexpr size_t PIN_CHUNK = 64ull << 20;
-static void par_memcpy(char *dst, const char *src, size_t len)
+// Device memory of a handle, from blocks kept by earlier handles where one fits.
+template <typename T>
+static hipError_t dmalloc(fh_reconstructor *h, T **p, size_t bytes)
 {
-    const int nt = (int)std::min<size_t>(8, std::max<size_t>(1, len >> 23));
-    if (nt == 1) {
-        memcpy(dst, src, len);
-        return;
-    }
-    std::vector<std::thread> th;
-    const size_t per = (len + nt - 1) / nt;
-    for (int t = 0; t < nt; t++) {
-        const size_t a = t * per, b = std::min(len, a + per);
-        if (a < b) th.emplace_back([=] { memcpy(dst + a, src + a, b - a); });
-    }
-    for (auto &x : th) x.join();
+    return h->pool->alloc(h->device, reinterpret_cast<void **>(p), bytes);
+}
+// Given back for any handle's use: the work queued on this handle's stream, the only one that uses it, is
+// waited for first.
+static void dfree(fh_reconstructor *h, void *p)
+{
+    (void)hipStreamSynchronize(h->stream);
+    h->pool->free(h->device, p);
 }
 
-// the two staging buffers and their events (recorded once, so that a first
-// wait on them returns at once)
+// Copies between the device and caller (pageable) memory run through a ring
+// of pinned slots, the DMA of some chunks beside the host copy of another by
+// several threads.  A pageable copy of the runtime takes longer from some
+// tens of KB on: 1 MB to the host 0.45 ms against 0.15, 4 MB 1.7 against
+// 0.25 (first touch of the target's pages included); below that it is as
+// quick as the staging.  340 MB: 8.8 ms through two 64 MB buffers and threads
+// started per chunk.
+constexpr size_t STAGE_MIN = 64u << 10;
+static size_t stage_chunk(size_t bytes)
+{
+    // a few chunks for overlap, none so small that its DMA's start outweighs it
+    return std::min(HostPool::PIN_SLOT, std::max<size_t>(512u << 10, (bytes / 4 + 4095) & ~(size_t)4095));
+}
+
+// the staging ring and its events (recorded once, so that a first wait on
+// them returns at once)
 static hipError_t ensure_pinned(fh_reconstructor *h)
 {
     hipError_t e;
-    for (int i = 0; i < 2; i++) {
-        if (!h->pin[i] && (e = hipHostMalloc((void **)&h->pin[i], PIN_CHUNK, hipHostMallocDefault)) != hipSuccess)
-            return e;
-        if (!h->pin_ev[i]) {
-            if ((e = hipEventCreateWithFlags(&h->pin_ev[i], hipEventDisableTiming)) != hipSuccess) return e;
-            if ((e = hipEventRecord(h->pin_ev[i], h->stream)) != hipSuccess) return e;
+    if (!h->pin && (e = h->pool->pinned(&h->pin)) != hipSuccess) return e;
+    for (auto &ev : h->pin_ev)
+        if (!ev) {
+            if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
+            if ((e = hipEventRecord(ev, h->stream)) != hipSuccess) return e;
         }
-    }
     return hipSuccess;
 }
 
 static hipError_t d2h_staged(fh_reconstructor *h, void *dst, const void *src, size_t bytes)
 {
     hipError_t e;
-    if (bytes < (16ull << 20)) {
+    if (bytes < STAGE_MIN) {
         if ((e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream)) != hipSuccess) return e;
         return hipStreamSynchronize(h->stream);
     }
     if ((e = ensure_pinned(h)) != hipSuccess) return e;
     const char *s = static_cast<const char *>(src);
     char *d = static_cast<char *>(dst);
-    const size_t nchunk = (bytes + PIN_CHUNK - 1) / PIN_CHUNK;
-    for (size_t c = 0; c <= nchunk; c++) {
-        if (c < nchunk) {  // the DMA of chunk c into buffer c % 2 (free: chunk c-2 was copied out)
-            const size_t off = c * PIN_CHUNK, len = std::min(PIN_CHUNK, bytes - off);
-            if ((e = hipMemcpyAsync(h->pin[c & 1], s + off, len, hipMemcpyDeviceToHost, h->stream)) != hipSuccess)
+    const size_t chunk = stage_chunk(bytes), n = (bytes + chunk - 1) / chunk, ahead = HostPool::PIN_SLOTS - 1;
+    for (size_t c = 0; c < n + ahead; c++) {
+        if (c < n) {  // the DMA of chunk c into its slot (free: chunk c - 4 was copied out)
+            const size_t off = c * chunk, len = std::min(chunk, bytes - off), k = c % HostPool::PIN_SLOTS;
+            if ((e = hipMemcpyAsync(h->pin + k * HostPool::PIN_SLOT, s + off, len, hipMemcpyDeviceToHost, h->stream)) !=
+                hipSuccess)
                 return e;
-            if ((e = hipEventRecord(h->pin_ev[c & 1], h->stream)) != hipSuccess) return e;
+            if ((e = hipEventRecord(h->pin_ev[k], h->stream)) != hipSuccess) return e;
         }
-        if (c > 0) {  // chunk c-1 out of its buffer while chunk c is in flight
-            const size_t p = c - 1, off = p * PIN_CHUNK, len = std::min(PIN_CHUNK, bytes - off);
-            if ((e = hipEventSynchronize(h->pin_ev[p & 1])) != hipSuccess) return e;
-            par_memcpy(d + off, reinterpret_cast<const char *>(h->pin[p & 1]), len);
+        if (c >= ahead && c - ahead < n) {  // chunk c - 3 out of its slot while the next ones are in flight
+            const size_t q = c - ahead, off = q * chunk, len = std::min(chunk, bytes - off), k = q % HostPool::PIN_SLOTS;
+            if ((e = hipEventSynchronize(h->pin_ev[k])) != hipSuccess) return e;
+            h->pool->copies.copy(d + off, h->pin + k * HostPool::PIN_SLOT, len);
         }
     }
     return hipSuccess;
 }
 
-// Host-to-device copy of `bytes` from caller (pageable) memory, the mirror
-// image: host threads copy chunk c into a pinned buffer (once the DMA that
-// last read that buffer is done) while the DMA of chunk c-1 runs.  Queued on
-// the handle's stream, so kernels queued after it see the data.
+// The mirror image: host threads copy chunk c into its slot (once the DMA
+// that last read the slot is done) while the DMA of the chunks before runs.
+// Queued on the handle's stream, so kernels queued after it see the data.
 static hipError_t h2d_staged(fh_reconstructor *h, void *dst, const void *src, size_t bytes)
 {
     hipError_t e;
@@ -439,13 +447,14 @@ static hipError_t h2d_staged(fh_reconstructor *h, void *dst, const void *src, si
     if ((e = ensure_pinned(h)) != hipSuccess) return e;
     const char *s = static_cast<const char *>(src);
     char *d = static_cast<char *>(dst);
-    const size_t nchunk = (bytes + PIN_CHUNK - 1) / PIN_CHUNK;
-    for (size_t c = 0; c < nchunk; c++) {
-        const size_t off = c * PIN_CHUNK, len = std::min(PIN_CHUNK, bytes - off);
-        if ((e = hipEventSynchronize(h->pin_ev[c & 1])) != hipSuccess) return e;  // buffer free
-        par_memcpy(reinterpret_cast<char *>(h->pin[c & 1]), s + off, len);
-        if ((e = hipMemcpyAsync(d + off, h->pin[c & 1], len, hipMemcpyHostToDevice, h->stream)) != hipSuccess) return e;
-        if ((e = hipEventRecord(h->pin_ev[c & 1], h->stream)) != hipSuccess) return e;
+    const size_t chunk = stage_chunk(bytes), n = (bytes + chunk - 1) / chunk;
+    for (size_t c = 0; c < n; c++) {
+        const size_t off = c * chunk, len = std::min(chunk, bytes - off), k = c % HostPool::PIN_SLOTS;
+        char *slot = h->pin + k * HostPool::PIN_SLOT;
+        if ((e = hipEventSynchronize(h->pin_ev[k])) != hipSuccess) return e;  // slot free
+        h->pool->copies.copy(slot, s + off, len);
+        if ((e = hipMemcpyAsync(d + off, slot, len, hipMemcpyHostToDevice, h->stream)) != hipSuccess) return e;
+        if ((e = hipEventRecord(h->pin_ev[k], h->stream)) != hipSuccess) return e;
     }
     return hipSuccess;
 }
@@ -453,9 +462,9 @@ static hipError_t h2d_staged(fh_reconstructor *h, void *dst, const void *src, si
 static void free_chunk(fh_reconstructor *h)
 {
     for (float **p : {&h->imgs, &h->means, &h->rots, &h->wts, &h->dfs, &h->dfs2, &h->t3d, &h->wq, &h->rw})
-        if (*p) { (void)hipFree(*p); *p = nullptr; }
-    if (h->slices) { (void)hipFree(h->slices); h->slices = nullptr; }
-    if (h->inter) { (void)hipFree(h->inter); h->inter = nullptr; }
+        if (*p) { dfree(h, *p); *p = nullptr; }
+    if (h->slices) { dfree(h, h->slices); h->slices = nullptr; }
+    if (h->inter) { dfree(h, h->inter); h->inter = nullptr; }
     h->inter_n = 0;
     h->cap_n = h->cap_B = 0;
 }
@@ -464,25 +473,25 @@ static void free_bins(fh_reconstructor *h)
 {
     BinBuffers &b = h->bins;
     for (int **p : {&b.counts, &b.offsets, &b.item_off, &b.tile, &b.list, &b.ctl})
-        if (*p) { (void)hipFree(*p); *p = nullptr; }
-    if (b.items) { (void)hipFree(b.items); b.items = nullptr; }
-    if (b.recs) { (void)hipFree(b.recs); b.recs = nullptr; }
+        if (*p) { dfree(h, *p); *p = nullptr; }
+    if (b.items) { dfree(h, b.items); b.items = nullptr; }
+    if (b.recs) { dfree(h, b.recs); b.recs = nullptr; }
     b.rec_cap = 0;
-    if (b.part) { (void)hipFree(b.part); b.part = nullptr; }
+    if (b.part) { dfree(h, b.part); b.part = nullptr; }
     b.part_cap = 0;
     h->bins_cap_slices = 0;
 }
 
 static void free_ref(fh_reconstructor *h)
 {
-    if (h->ref) { (void)hipFree(h->ref); h->ref = nullptr; }
+    if (h->ref) { dfree(h, h->ref); h->ref = nullptr; }
 }
 
 static void free_volume(fh_reconstructor *h)
 {
-    if (h->data) { (void)hipFree(h->data); h->data = nullptr; }
-    if (h->norm) { (void)hipFree(h->norm); h->norm = nullptr; }
-    if (h->pack) { (void)hipFree(h->pack); h->pack = nullptr; }
+    if (h->data) { dfree(h, h->data); h->data = nullptr; }
+    if (h->norm) { dfree(h, h->norm); h->norm = nullptr; }
+    if (h->pack) { dfree(h, h->pack); h->pack = nullptr; }
     h->ready = false;
 }
 
@@ -500,20 +509,20 @@ static int ensure_chunk(fh_reconstructor *h, int n, int B)
     free_chunk(h);
     const int P = h->P, H = h->H;
     const size_t ns = (size_t)n * h->nsym;
-    FH_TRY(h, hipMalloc(&h->imgs, sizeof(float) * (size_t)n * B * B));
-    FH_TRY(h, hipMalloc(&h->means, sizeof(float) * n));
-    FH_TRY(h, hipMalloc(&h->rots, sizeof(float) * 9 * (size_t)n));
-    FH_TRY(h, hipMalloc(&h->wts, sizeof(float) * n));
-    FH_TRY(h, hipMalloc(&h->dfs, sizeof(float) * n));
-    FH_TRY(h, hipMalloc(&h->dfs2, sizeof(float) * n));
-    FH_TRY(h, hipMalloc(&h->slices, sizeof(float2) * (size_t)n * P * (H + 1)));
+    FH_TRY(h, dmalloc(h, &h->imgs, sizeof(float) * (size_t)n * B * B));
+    FH_TRY(h, dmalloc(h, &h->means, sizeof(float) * n));
+    FH_TRY(h, dmalloc(h, &h->rots, sizeof(float) * 9 * (size_t)n));
+    FH_TRY(h, dmalloc(h, &h->wts, sizeof(float) * n));
+    FH_TRY(h, dmalloc(h, &h->dfs, sizeof(float) * n));
+    FH_TRY(h, dmalloc(h, &h->dfs2, sizeof(float) * n));
+    FH_TRY(h, dmalloc(h, &h->slices, sizeof(float2) * (size_t)n * P * (H + 1)));
     if (prep_column_first(P)) {
         h->inter_n = std::min(n, PREP_INTER_PARTICLES);
-        FH_TRY(h, hipMalloc(&h->inter, prep_inter_bytes(P, h->inter_n)));
+        FH_TRY(h, dmalloc(h, &h->inter, prep_inter_bytes(P, h->inter_n)));
     }
-    FH_TRY(h, hipMalloc(&h->t3d, sizeof(float) * 9 * ns));
-    FH_TRY(h, hipMalloc(&h->wq, sizeof(float) * ns));
-    if (h->usessnr) FH_TRY(h, hipMalloc(&h->rw, sizeof(float) * (size_t)n * (H + 1)));
+    FH_TRY(h, dmalloc(h, &h->t3d, sizeof(float) * 9 * ns));
+    FH_TRY(h, dmalloc(h, &h->wq, sizeof(float) * ns));
+    if (h->usessnr) FH_TRY(h, dmalloc(h, &h->rw, sizeof(float) * (size_t)n * (H + 1)));
     h->cap_n = n;
     h->cap_B = B;
     return FH_OK;
@@ -608,14 +617,14 @@ static int ensure_bins(fh_reconstructor *h, long long nslices)
     // smaller batches have fewer items: pairs over K grows with the slices, up to K's rounding
     const int K = item_slices(h, nslices);
     b.item_cap = b.list_cap / K * (K < h->tune.slices_per_item ? 5 : 4) / 4 + g.nkeys + 1;
-    FH_TRY(h, hipMalloc(&b.counts, sizeof(int) * g.nkeys));
-    FH_TRY(h, hipMalloc(&b.offsets, sizeof(int) * (g.nkeys + 1)));
-    FH_TRY(h, hipMalloc(&b.item_off, sizeof(int) * (g.nkeys + 1)));
-    FH_TRY(h, hipMalloc(&b.tile, sizeof(int) * 2 * scan_tiles(g)));
-    FH_TRY(h, hipMalloc(&b.list, sizeof(int) * b.list_cap));
-    FH_TRY(h, hipMalloc(&b.items, sizeof(WorkItem) * b.item_cap));
-    FH_TRY(h, hipMalloc(&b.ctl, sizeof(int) * 8));
-    FH_TRY(h, hipMalloc(&b.recs, sizeof(SliceRec) * 3 * (size_t)nslices));
+    FH_TRY(h, dmalloc(h, &b.counts, sizeof(int) * g.nkeys));
+    FH_TRY(h, dmalloc(h, &b.offsets, sizeof(int) * (g.nkeys + 1)));
+    FH_TRY(h, dmalloc(h, &b.item_off, sizeof(int) * (g.nkeys + 1)));
+    FH_TRY(h, dmalloc(h, &b.tile, sizeof(int) * 2 * scan_tiles(g)));
+    FH_TRY(h, dmalloc(h, &b.list, sizeof(int) * b.list_cap));
+    FH_TRY(h, dmalloc(h, &b.items, sizeof(WorkItem) * b.item_cap));
+    FH_TRY(h, dmalloc(h, &b.ctl, sizeof(int) * 8));
+    FH_TRY(h, dmalloc(h, &b.recs, sizeof(SliceRec) * 3 * (size_t)nslices));
     b.rec_cap = nslices;
     h->bins_cap_slices = nslices;
     return FH_OK;
@@ -627,10 +636,10 @@ static int ensure_partials(fh_reconstructor *h, long long items)
 {
     BinBuffers &b = h->bins;
     if (items <= b.part_cap) return FH_OK;
-    if (b.part) { (void)hipFree(b.part); b.part = nullptr; }
+    if (b.part) { dfree(h, b.part); b.part = nullptr; }
     b.part_cap = 0;
     const long long cap = items + items / 4 + 1024;
-    FH_TRY(h, hipMalloc(&b.part, sizeof(float) * h->geom.part_floats * (size_t)cap));
+    FH_TRY(h, dmalloc(h, &b.part, sizeof(float) * h->geom.part_floats * (size_t)cap));
     b.part_cap = cap;
     return FH_OK;
 }
@@ -768,7 +777,7 @@ int fh_create(const fh_params *p, fh_reconstructor **out)
     h->syms = ops;
     h->nsym = (int)ops.size() / 9;
     hipError_t e;
-    if ((e = hipSetDevice(h->device)) != hipSuccess || (e = hipStreamCreate(&h->stream)) != hipSuccess) {
+    if ((e = hipSetDevice(h->device)) != hipSuccess || (e = h->pool->stream(h->device, &h->stream)) != hipSuccess) {
         g_create_error = std::string("device error: ") + hipGetErrorString(e);
         delete h;
         return FH_ERR_DEVICE;
@@ -788,10 +797,10 @@ int fh_create(const fh_params *p, fh_reconstructor **out)
     }
     make_plan(P, &h->plan);
     h->scale = (float)sqrt((double)(1.0f / (float)P * (float)(P + 2)));
-    if ((e = hipMalloc(&h->exptab, sizeof(float) * 1000)) != hipSuccess ||
-        (e = hipMalloc(&h->rtab, sizeof(float) * (P + 2))) != hipSuccess ||
-        (e = hipMalloc(&h->tw, sizeof(float2) * P)) != hipSuccess ||
-        (e = hipMalloc(&h->syms_d, sizeof(float) * ops.size())) != hipSuccess ||
+    if ((e = dmalloc(h, &h->exptab, sizeof(float) * 1000)) != hipSuccess ||
+        (e = dmalloc(h, &h->rtab, sizeof(float) * (P + 2))) != hipSuccess ||
+        (e = dmalloc(h, &h->tw, sizeof(float2) * P)) != hipSuccess ||
+        (e = dmalloc(h, &h->syms_d, sizeof(float) * ops.size())) != hipSuccess ||
         (e = hipMemcpy(h->exptab, et.data(), sizeof(float) * 1000, hipMemcpyHostToDevice)) != hipSuccess ||
         (e = hipMemcpy(h->rtab, rt.data(), sizeof(float) * (P + 2), hipMemcpyHostToDevice)) != hipSuccess ||
         (e = hipMemcpy(h->tw, tw.data(), sizeof(float2) * P, hipMemcpyHostToDevice)) != hipSuccess ||
@@ -815,22 +824,21 @@ int fh_destroy(fh_reconstructor *h)
         free_bins(h);
         free_volume(h);
         free_ref(h);
-        if (h->pvol) (void)hipFree(h->pvol);
-        if (h->ximgs) (void)hipFree(h->ximgs);
-        if (h->ximgs2) (void)hipFree(h->ximgs2);
-        if (h->xfd) (void)hipFree(h->xfd);
-        for (int i = 0; i < 2; i++) {
-            if (h->pin[i]) (void)hipHostFree(h->pin[i]);
-            if (h->pin_ev[i]) (void)hipEventDestroy(h->pin_ev[i]);
-        }
-        if (h->partial) (void)hipFree(h->partial);
-        if (h->rw1) (void)hipFree(h->rw1);
-        if (h->acc8) (void)hipFree(h->acc8);
+        if (h->pvol) dfree(h, h->pvol);
+        if (h->ximgs) dfree(h, h->ximgs);
+        if (h->ximgs2) dfree(h, h->ximgs2);
+        if (h->xfd) dfree(h, h->xfd);
+        if (h->pin) h->pool->give_pinned(h->pin);
+        for (auto &ev : h->pin_ev)
+            if (ev) (void)hipEventDestroy(ev);
+        if (h->partial) dfree(h, h->partial);
+        if (h->rw1) dfree(h, h->rw1);
+        if (h->acc8) dfree(h, h->acc8);
         for (void *p : {(void *)h->exptab, (void *)h->rtab, (void *)h->tw, (void *)h->syms_d})
-            if (p) (void)hipFree(p);
+            if (p) dfree(h, p);
         for (auto &ev : h->ev)
             if (ev) (void)hipEventDestroy(ev);
-        if (h->stream) (void)hipStreamDestroy(h->stream);
+        if (h->stream) h->pool->give_stream(h->device, h->stream);
     }
     delete h;
     return FH_OK;
@@ -842,11 +850,11 @@ static int setup_locked(fh_reconstructor *h)
     free_ref(h);  // fourier_iter's setup() drops the reference volume (reconstructor.cpp:462-464)
     const size_t n = vol_elems(h->P);
     if (!h->data) {
-        hipError_t e = hipMalloc(&h->data, sizeof(float2) * n);
+        hipError_t e = dmalloc(h, &h->data, sizeof(float2) * n);
         if (e != hipSuccess) return fail(h, FH_ERR_NOMEM, std::string("volume allocation: ") + hipGetErrorString(e));
-        e = hipMalloc(&h->norm, sizeof(float) * n);
+        e = dmalloc(h, &h->norm, sizeof(float) * n);
         if (e != hipSuccess) {
-            (void)hipFree(h->data);
+            dfree(h, h->data);
             h->data = nullptr;
             return fail(h, FH_ERR_NOMEM, std::string("weight allocation: ") + hipGetErrorString(e));
         }
@@ -875,7 +883,7 @@ static int iter_seed_complex(fh_reconstructor *h, const float *seed)
     int rc = setup_locked(h);
     if (rc) return rc;
     const size_t n = vol_elems(h->P);
-    FH_TRY(h, hipMalloc(&h->ref, sizeof(float2) * n));
+    FH_TRY(h, dmalloc(h, &h->ref, sizeof(float2) * n));
     FH_TRY(h, hipMemcpyAsync(h->ref, seed, sizeof(float2) * n, hipMemcpyHostToDevice, h->stream));
     FH_TRY(h, hipStreamSynchronize(h->stream));
     return FH_OK;
@@ -893,7 +901,7 @@ int fh_setup_seed_map(fh_reconstructor *h, const float *map)
     const int P = h->P;
     // the map goes through the particle staging (P images of P x P) and the prep's FFT passes
     if ((rc = ensure_chunk(h, std::max(P, h->cap_n), std::max(P, h->cap_B)))) return rc;
-    FH_TRY(h, hipMalloc(&h->ref, sizeof(float2) * vol_elems(P)));
+    FH_TRY(h, dmalloc(h, &h->ref, sizeof(float2) * vol_elems(P)));
     FH_TRY(h, h2d_staged(h, h->imgs, map, sizeof(float) * (size_t)P * P * P));
     FH_TRY(h, launch_fill_f32(h->means, 0.f, P, h->stream));
     FH_TRY(h, launch_fft3d_forward_corner(h->imgs, P, h->means, h->ref, h->plan, h->tw, h->stream));
@@ -985,20 +993,20 @@ static hipError_t prep_kernels(fh_reconstructor *h, int n, int B, const float *d
 static int ensure_ximgs(fh_reconstructor *h, int n, bool two = false)
 {
     if (two && n > h->ximgs2_cap) {
-        if (h->ximgs2) (void)hipFree(h->ximgs2);
+        if (h->ximgs2) dfree(h, h->ximgs2);
         h->ximgs2 = nullptr;
         h->ximgs2_cap = 0;
-        FH_TRY(h, hipMalloc(&h->ximgs2, sizeof(float) * (size_t)n * h->P * h->P));
+        FH_TRY(h, dmalloc(h, &h->ximgs2, sizeof(float) * (size_t)n * h->P * h->P));
         h->ximgs2_cap = n;
     }
     if (n <= h->ximgs_cap) return FH_OK;
-    if (h->ximgs) (void)hipFree(h->ximgs);
-    if (h->xfd) (void)hipFree(h->xfd);
+    if (h->ximgs) dfree(h, h->ximgs);
+    if (h->xfd) dfree(h, h->xfd);
     h->ximgs = nullptr;
     h->xfd = nullptr;
     h->ximgs_cap = 0;
-    FH_TRY(h, hipMalloc(&h->ximgs, sizeof(float) * (size_t)n * h->P * h->P));
-    FH_TRY(h, hipMalloc(&h->xfd, sizeof(float) * 6 * (size_t)n));
+    FH_TRY(h, dmalloc(h, &h->ximgs, sizeof(float) * (size_t)n * h->P * h->P));
+    FH_TRY(h, dmalloc(h, &h->xfd, sizeof(float) * 6 * (size_t)n));
     h->ximgs_cap = n;
     return FH_OK;
 }
@@ -1189,8 +1197,7 @@ int fh_preprocess_slice_xform(fh_reconstructor *h, const float *img, const float
     FH_TRY(h, hipMemcpyAsync(h->imgs, img, sizeof(float) * P * P, hipMemcpyHostToDevice, h->stream));
     // preprocess_slice has no edge-mean step
     if ((rc = prep_single_raw(h, xf6.empty() ? nullptr : xf6.data()))) return rc;
-    FH_TRY(h, hipMemcpyAsync(slice_out, h->slices, sizeof(float2) * P * (H + 1), hipMemcpyDeviceToHost, h->stream));
-    FH_TRY(h, hipStreamSynchronize(h->stream));
+    FH_TRY(h, d2h_staged(h, slice_out, h->slices, sizeof(float2) * P * (H + 1)));
     return FH_OK;
 }
 
@@ -1479,9 +1486,14 @@ int fh_prep_batch(fh_reconstructor *h, const float *imgs, int n, int box, const 
         rc = prep_chunk(h, m, box, dimgs, defocus ? defocus + c0 : nullptr, ctf, nullptr,
                         df2.empty() ? nullptr : df2.data() + c0);
         if (rc) return rc;
-        FH_TRY(h, hipMemcpyAsync(slices_out + (size_t)c0 * P * (P + 2), h->slices, sizeof(float2) * (size_t)m * P * (H + 1),
-                                 where == FH_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, h->stream));
-        FH_TRY(h, hipStreamSynchronize(h->stream));
+        const size_t bytes = sizeof(float2) * (size_t)m * P * (H + 1);
+        float *dst = slices_out + (size_t)c0 * P * (P + 2);
+        if (where == FH_DEVICE) {
+            FH_TRY(h, hipMemcpyAsync(dst, h->slices, bytes, hipMemcpyDeviceToDevice, h->stream));
+            FH_TRY(h, hipStreamSynchronize(h->stream));
+        } else {
+            FH_TRY(h, d2h_staged(h, dst, h->slices, bytes));
+        }
     }
     return FH_OK;
 }
@@ -1558,10 +1570,10 @@ int fh_projection(fh_reconstructor *h, const float xform[12], int ret_fourier, f
     const InsertConst c = iconst(h);
     FH_TRY(h, launch_project(h->data, h->norm, c, rot9, h->rtab, tx, ty, ret_fourier ? 0 : 1, h->slices, h->stream));
     if (ret_fourier) {
-        FH_TRY(h, hipMemcpyAsync(out, h->slices, sizeof(float2) * P * (H + 1), hipMemcpyDeviceToHost, h->stream));
+        FH_TRY(h, d2h_staged(h, out, h->slices, sizeof(float2) * P * (H + 1)));
     } else {
         FH_TRY(h, launch_ift2d(h->slices, P, h->imgs, h->plan, h->tw, h->stream));
-        FH_TRY(h, hipMemcpyAsync(out, h->imgs, sizeof(float) * P * P, hipMemcpyDeviceToHost, h->stream));
+        FH_TRY(h, d2h_staged(h, out, h->imgs, sizeof(float) * P * P));
     }
     FH_TRY(h, hipStreamSynchronize(h->stream));
     return FH_OK;
@@ -1636,7 +1648,7 @@ static int agree_one(fh_reconstructor *h, const float2 *slice_d, const float *ro
 static int ensure_partial(fh_reconstructor *h)
 {
     if (h->partial) return FH_OK;
-    FH_TRY(h, hipMalloc(&h->partial, sizeof(double) * 8 * (size_t)agree_blocks(h->P) * h->nsym));
+    FH_TRY(h, dmalloc(h, &h->partial, sizeof(double) * 8 * (size_t)agree_blocks(h->P) * h->nsym));
     return FH_OK;
 }
 
@@ -1806,7 +1818,7 @@ int fh_determine_slice_agreement_ssnr(fh_reconstructor *h, const float *data, in
     }
     std::vector<float> rw(H + 1);
     if (sub) {
-        if (!h->rw1) FH_TRY(h, hipMalloc(&h->rw1, sizeof(float) * (H + 1)));
+        if (!h->rw1) FH_TRY(h, dmalloc(h, &h->rw1, sizeof(float) * (H + 1)));
         ssnr_radial(P, class_ssnr, ssnr_len, rw.data());
         FH_TRY(h, hipMemcpyAsync(h->rw1, rw.data(), sizeof(float) * (H + 1), hipMemcpyHostToDevice, h->stream));
     }
@@ -1837,9 +1849,9 @@ int fh_agreement_batch(fh_reconstructor *h, const float *imgs, int n, int box, c
     const int chunk = std::max(1, std::min(chunk_for(h->tune, h->P, box, xbytes), std::max(n, 1)));
     if ((rc = ensure_chunk(h, chunk, box))) return rc;
     if (!h->acc8 || h->acc8_cap < chunk) {
-        if (h->acc8) (void)hipFree(h->acc8);
+        if (h->acc8) dfree(h, h->acc8);
         h->acc8 = nullptr;
-        FH_TRY(h, hipMalloc(&h->acc8, sizeof(double) * 8 * (size_t)chunk));
+        FH_TRY(h, dmalloc(h, &h->acc8, sizeof(double) * 8 * (size_t)chunk));
         h->acc8_cap = chunk;
     }
     const InsertConst c = iconst(h);
@@ -1848,7 +1860,7 @@ int fh_agreement_batch(fh_reconstructor *h, const float *imgs, int n, int box, c
     // packing moves 28 bytes a voxel, 14 P^3; a slice then reads some 35 P^2 bytes less: worth it from about
     // 0.4 P slices on (pad 600, 8,000 slices: 0.62 ms for 9.6)
     if (!seq && (long long)n * h->nsym >= h->P) {
-        if (!h->pack && hipMalloc(&h->pack, sizeof(float4) * pack_elems(h->P)) != hipSuccess) {
+        if (!h->pack && dmalloc(h, &h->pack, sizeof(float4) * pack_elems(h->P)) != hipSuccess) {
             (void)hipGetLastError();  // no room: the volume and its weights are read as they are
             h->pack = nullptr;
         }
@@ -1908,24 +1920,24 @@ int fh_finish(fh_reconstructor *h, int doift, float *out, float *norm_out)
     const int P = h->P;
     const size_t n = vol_elems(P);
     float *planes = nullptr;
-    FH_TRY(h, hipMalloc(&planes, sizeof(float) * 2 * P * P));
+    FH_TRY(h, dmalloc(h, &planes, sizeof(float) * 2 * P * P));
     hipError_t e = launch_normalize(h->data, h->norm, P, h->sqrtnorm, planes, h->stream);
     if (e == hipSuccess && doift) {
         e = launch_fft3d_inverse_zy(h->data, P, h->plan, h->tw, h->stream);
         float *real = nullptr;
-        if (e == hipSuccess) e = hipMalloc(&real, sizeof(float) * (size_t)P * P * P);
+        if (e == hipSuccess) e = dmalloc(h, &real, sizeof(float) * (size_t)P * P * P);
         if (e == hipSuccess) {
             const float sc = 1.0f / (float)((size_t)P * P * P);
             e = launch_c2r_x(h->data, P, real, sc, h->plan, h->tw, h->stream);
             if (e == hipSuccess) e = d2h_staged(h, out, real, sizeof(float) * (size_t)P * P * P);
-            (void)hipFree(real);
+            dfree(h, real);
         }
     } else if (e == hipSuccess) {
         e = d2h_staged(h, out, h->data, sizeof(float2) * n);
     }
     if (e == hipSuccess && norm_out) e = d2h_staged(h, norm_out, h->norm, sizeof(float) * n);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    (void)hipFree(planes);
+    dfree(h, planes);
     if (e != hipSuccess) return fail(h, FH_ERR_DEVICE, std::string("finish: ") + hipGetErrorString(e));
     free_volume(h);  // ownership of the map passes to the caller (reconstructor.cpp:1633-1640)
     return FH_OK;
@@ -1944,14 +1956,14 @@ int fh_merge_add(fh_reconstructor *h, const float *threed, const float *normv, i
     void *tmp = nullptr;
     if (where != FH_DEVICE) {
         // staged through one temporary device buffer (12 bytes per stored voxel)
-        hipError_t e = hipMalloc(&tmp, (sizeof(float2) + sizeof(float)) * n);
+        hipError_t e = dmalloc(h, &tmp, (sizeof(float2) + sizeof(float)) * n);
         if (e != hipSuccess) return fail(h, FH_ERR_NOMEM, std::string("merge staging: ") + hipGetErrorString(e));
         float2 *t2 = static_cast<float2 *>(tmp);
         float *n2 = reinterpret_cast<float *>(t2 + n);
         e = hipMemcpyAsync(t2, threed, sizeof(float2) * n, hipMemcpyHostToDevice, h->stream);
         if (e == hipSuccess) e = hipMemcpyAsync(n2, normv, sizeof(float) * n, hipMemcpyHostToDevice, h->stream);
         if (e != hipSuccess) {
-            (void)hipFree(tmp);
+            dfree(h, tmp);
             return fail(h, FH_ERR_DEVICE, std::string("merge staging: ") + hipGetErrorString(e));
         }
         td = t2;
@@ -1959,7 +1971,7 @@ int fh_merge_add(fh_reconstructor *h, const float *threed, const float *normv, i
     }
     hipError_t e = launch_merge_add(h->data, h->norm, td, nd, n, h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (tmp) (void)hipFree(tmp);
+    if (tmp) dfree(h, tmp);
     if (e != hipSuccess) return fail(h, FH_ERR_DEVICE, std::string("merge_add: ") + hipGetErrorString(e));
     return FH_OK;
 }
@@ -1976,13 +1988,13 @@ int fh_merge_finish(fh_reconstructor *h, float *out)
     hipError_t e = launch_merge_scale(h->data, h->norm, n, h->stream);
     if (e == hipSuccess) e = launch_fft3d_inverse_zy(h->data, P, h->plan, h->tw, h->stream);
     float *real = nullptr;
-    if (e == hipSuccess) e = hipMalloc(&real, sizeof(float) * (size_t)P * P * P);
+    if (e == hipSuccess) e = dmalloc(h, &real, sizeof(float) * (size_t)P * P * P);
     if (e == hipSuccess) {
         const float sc = 1.0f / (float)((size_t)P * P * P);
         e = launch_c2r_x(h->data, P, real, sc, h->plan, h->tw, h->stream);
         if (e == hipSuccess) e = d2h_staged(h, out, real, sizeof(float) * (size_t)P * P * P);
         if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-        (void)hipFree(real);
+        dfree(h, real);
     }
     if (e != hipSuccess) return fail(h, FH_ERR_DEVICE, std::string("merge_finish: ") + hipGetErrorString(e));
     free_volume(h);
@@ -1999,7 +2011,7 @@ int fh_gauss_fft_volume(fh_reconstructor *h, const float *map)
     const int P = h->P;
     int rc = ensure_chunk(h, std::max(P, h->cap_n), std::max(P, h->cap_B));
     if (rc) return rc;
-    if (!h->pvol) FH_TRY(h, hipMalloc(&h->pvol, sizeof(float2) * vol_elems(P)));
+    if (!h->pvol) FH_TRY(h, dmalloc(h, &h->pvol, sizeof(float2) * vol_elems(P)));
     // xform.phaseorigin.tocorner and do_fft (projector.cpp:77-79) on the GPU; the
     // Fourier origin shift to the centre is a re-indexing, done by the reads
     FH_TRY(h, h2d_staged(h, h->imgs, map, sizeof(float) * (size_t)P * P * P));
@@ -2061,7 +2073,7 @@ int fh_gauss_fft_project(fh_reconstructor *h, int n, const float *xforms, int mo
     if (rc) return rc;
     if (!returnfft && (rc = ensure_ximgs(h, chunk))) return rc;
     float *tmp = nullptr;  // the projections' records on the device
-    FH_TRY(h, hipMalloc(&tmp, sizeof(float) * 12 * (size_t)chunk));
+    FH_TRY(h, dmalloc(h, &tmp, sizeof(float) * 12 * (size_t)chunk));
     float *rec_d = tmp;
     hipError_t e = hipSuccess;
     for (int c0 = 0; c0 < n && e == hipSuccess; c0 += chunk) {
@@ -2070,8 +2082,7 @@ int fh_gauss_fft_project(fh_reconstructor *h, int n, const float *xforms, int mo
         if (e == hipSuccess) e = launch_gauss_fft(h->pvol, P, m, mode, gw, rec_d, returnfft ? 1 : 0, h->slices, h->stream);
         if (e != hipSuccess) break;
         if (returnfft) {
-            e = hipMemcpyAsync(out + (size_t)c0 * P * (P + 2), h->slices, sizeof(float2) * (size_t)m * P * (H + 1),
-                               hipMemcpyDeviceToHost, h->stream);
+            e = d2h_staged(h, out + (size_t)c0 * P * (P + 2), h->slices, sizeof(float2) * (size_t)m * P * (H + 1));
         } else {
             // do_ift (x 1/P^2) written with the phase origin moved to the centre
             e = launch_ift2d_batch(h->slices, m, P, h->ximgs, 1.0f / ((float)P * (float)P), h->plan, h->tw, h->stream);
@@ -2087,7 +2098,7 @@ int fh_gauss_fft_project(fh_reconstructor *h, int n, const float *xforms, int mo
                     memcpy(&xf6[6 * (size_t)q], inv, sizeof(inv));
                 }
                 if ((rc = ensure_ximgs(h, chunk, true))) {
-                    (void)hipFree(tmp);
+                    dfree(h, tmp);
                     return rc;
                 }
                 e = hipMemcpyAsync(h->xfd, xf6.data(), sizeof(float) * 6 * m, hipMemcpyHostToDevice, h->stream);
@@ -2097,12 +2108,11 @@ int fh_gauss_fft_project(fh_reconstructor *h, int n, const float *xforms, int mo
             }
             if (e == hipSuccess) e = launch_gausskernelfix2d(img, P, m, gw, h->stream);
             if (e == hipSuccess)
-                e = hipMemcpyAsync(out + (size_t)c0 * P * P, img, sizeof(float) * (size_t)m * P * P, hipMemcpyDeviceToHost,
-                                   h->stream);
+                e = d2h_staged(h, out + (size_t)c0 * P * P, img, sizeof(float) * (size_t)m * P * P);
         }
         if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     }
-    (void)hipFree(tmp);
+    dfree(h, tmp);
     if (e != hipSuccess) return fail(h, FH_ERR_DEVICE, std::string("gauss_fft: ") + hipGetErrorString(e));
     return FH_OK;
 }

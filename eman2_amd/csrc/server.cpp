@@ -14,6 +14,8 @@
 #include <thread>
 #include <vector>
 
+#include "host_pool.hpp"
+
 namespace {
 
 struct Job {
@@ -41,6 +43,7 @@ struct fh_server {
     std::vector<std::thread> workers;
     std::chrono::steady_clock::time_point t0;
     std::string err;
+    fh::HostPool::Ref pool = fh::HostPool::get();  // the jobs' handles reuse each other's blocks and streams
 
     double now() const
     {
