@@ -2181,26 +2181,39 @@ __device__ __forceinline__ int isqrt24(int n)
     return r;
 }
 
-// gauss_2 / trilinear weights of the 8 corners (i0+di, j0+dj, k0+dk),
+// gauss_2 / trilinear weights of the 8 corners (floor(p) + (di, dj, dk)),
 // corner index di + 2 dj + 4 dk; each equals corner_weight() bit for bit.
-__device__ __forceinline__ void corner_weights8(int mode, int i0, int j0, int k0, float xx, float yy, float zz,
-                                                float h, float weight, const float *etab, float wg[8])
+// gauss_2's table index is read off the bits of one FMA rounded toward zero
+// (see g6_entries); the table starts the kernel's LDS.
+__device__ __forceinline__ void corner_weights8(int mode, float xx, float yy, float zz, float h, float weight, float wg[8])
 {
-    const float dx[2] = {(float)i0 - xx, (float)(i0 + 1) - xx};
-    const float dy[2] = {(float)j0 - yy, (float)(j0 + 1) - yy};
-    const float dz[2] = {(float)k0 - zz, (float)(k0 + 1) - zz};
+    const float fx = floorf(xx), fy = floorf(yy), fz = floorf(zz);
+    const float dx[2] = {fx - xx, (fx + 1.0f) - xx};
+    const float dy[2] = {fy - yy, (fy + 1.0f) - yy};
+    const float dz[2] = {fz - zz, (fz + 1.0f) - zz};
     if (mode == 0) {
+        float f[8];
 #pragma unroll
         for (int b = 0; b < 4; b++) {
             const float sxy = dx[b & 1] * dx[b & 1] + dy[b >> 1] * dy[b >> 1];
 #pragma unroll
-            for (int dk = 0; dk < 2; dk++) {
-                const float r = sxy + dz[dk] * dz[dk];       // Util::hypot3sq
-                const float f = r * h;
-                const int g = (int)__builtin_fma((double)f, 50.0, 0.5);  // Util::fast_exp index: f*50 is exact in double
-                wg[b + 4 * dk] = etab[g] * weight;
-            }
+            for (int dk = 0; dk < 2; dk++) f[b + 4 * dk] = (sxy + dz[dk] * dz[dk]) * h;  // Util::hypot3sq, times h
         }
+        asm("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 3\n\t"
+            "v_fma_f32 %0, %0, %8, %9\n\t"
+            "v_fma_f32 %1, %1, %8, %9\n\t"
+            "v_fma_f32 %2, %2, %8, %9\n\t"
+            "v_fma_f32 %3, %3, %8, %9\n\t"
+            "v_fma_f32 %4, %4, %8, %9\n\t"
+            "v_fma_f32 %5, %5, %8, %9\n\t"
+            "v_fma_f32 %6, %6, %8, %9\n\t"
+            "v_fma_f32 %7, %7, %8, %9\n\t"
+            "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0"
+            : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]), "+v"(f[6]), "+v"(f[7])
+            : "s"(50.0f), "v"(2097152.5f));
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+            wg[k] = *(const __attribute__((address_space(3))) float *)((unsigned)__float_as_int(f[k]) & 0xffcu) * weight;
     } else {
         double ax[2], ay[2], az[2];
 #pragma unroll
@@ -2221,6 +2234,7 @@ __device__ __forceinline__ void corner_weights8(int mode, int i0, int j0, int k0
 // weight computation they run along with the wave stays inside the tables.
 struct PendPix {
     float re, im, px, py, pz, pw;
+    int org;    // stencil origin: tag index in [0, BRICK^3), accumulator slot << 16
     bool pend;
 };
 
@@ -2229,11 +2243,9 @@ struct PendPix {
 // earlier windows take precedence over the window's new ones (`fresh`), so a
 // carried pixel is added in the next window it takes part in unless it
 // collides with another carried pixel.  The losers stay pending.
-__device__ __forceinline__ bool scatter_elect(const PendPix &st, bool fresh, const int lo[3], int lane,
-                                              unsigned char *tag)
+__device__ __forceinline__ bool scatter_elect(const PendPix &st, bool fresh, int lane, unsigned char *tag)
 {
-    const int i0 = (int)floorf(st.px) - lo[0], j0 = (int)floorf(st.py) - lo[1], k0 = (int)floorf(st.pz) - lo[2];
-    const int ti = st.pend ? i0 + BRICK * (j0 + BRICK * k0) : 0;  // in [0, BRICK^3) while pending
+    const int ti = st.org & 0xffff;
     if (st.pend && fresh) tag[ti] = (unsigned char)lane;
     wave_sync_lds();
     if (st.pend && !fresh) tag[ti] = (unsigned char)lane;
@@ -2247,21 +2259,18 @@ __device__ __forceinline__ bool scatter_elect(const PendPix &st, bool fresh, con
 // meet on a cell through different corners, so the corners go one after
 // another with a wave-level ordering point between them.
 template <int A>
-__device__ __forceinline__ void scatter_add(const PendPix &st, bool win, const int lo[3], const InsertConst &c,
-                                            float *acc, const float *etab)
+__device__ __forceinline__ void scatter_add(const PendPix &st, bool win, const InsertConst &c, float *acc)
 {
-    const int f0 = (int)floorf(st.px), f1 = (int)floorf(st.py), f2 = (int)floorf(st.pz);
     float wg[8];
-    corner_weights8(c.mode, f0, f1, f2, st.px, st.py, st.pz, c.h, st.pw, etab, wg);
-    const int cbase = acc_slot<A>(f0 - lo[0], f1 - lo[1], f2 - lo[2]);
-    float *const p_re = acc + cbase, *const p_im = acc + ACC_N + cbase, *const p_w = acc + 2 * ACC_N + cbase;
+    corner_weights8(c.mode, st.px, st.py, st.pz, c.h, st.pw, wg);
+    float *const p_re = acc + (st.org >> 16), *const p_im = p_re + ACC_N, *const p_w = p_re + 2 * ACC_N;
 #pragma unroll
     for (int cI = 0; cI < 8; cI++) {
         const int di = cI & 1, dj = (cI >> 1) & 1, dk = cI >> 2;
         if (win) {
             const int a = acc_slot<A>(di, dj, dk);
-            p_re[a] += st.re * wg[cI];
-            p_im[a] += st.im * wg[cI];
+            p_re[a] = __builtin_fmaf(st.re, wg[cI], p_re[a]);
+            p_im[a] = __builtin_fmaf(st.im, wg[cI], p_im[a]);
             p_w[a] += wg[cI];
         }
         wave_sync_lds();
@@ -2304,9 +2313,8 @@ __device__ __forceinline__ void fetch_group_slice(GroupSlice &gs, int s, int cou
 template <int A, bool SSNR>
 __device__ __forceinline__ void scatter_group(const float2 *__restrict__ slices, int nsym, const GroupSlice &gs,
                                               const InsertConst &c, const int lo[3], int lane, float *acc,
-                                              unsigned char *tag, int *mark, float4 *rec, const float *etab,
-                                              const float *rtab, const float *__restrict__ rw, PendPix &st,
-                                              bool &fresh)
+                                              unsigned char *tag, int *mark, float4 *rec, const float *rtab,
+                                              const float *__restrict__ rw, PendPix &st, bool &fresh)
 {
     const int H = c.H, P = c.P;
     const unsigned slice_elems = (unsigned)P * (unsigned)(H + 1);
@@ -2362,7 +2370,7 @@ __device__ __forceinline__ void scatter_group(const float2 *__restrict__ slices,
     // next pixels (slots next, next+1, ... in lane order), and the winners'
     // corner updates run while those slice reads are in flight.
     for (int next = 0; next < total;) {
-        const bool win = scatter_elect(st, fresh, lo, lane, tag);
+        const bool win = scatter_elect(st, fresh, lane, tag);
         const bool freed = !st.pend || win;
         const unsigned long long fm = __ballot(freed);
         const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(fm >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)fm, 0u));
@@ -2385,11 +2393,11 @@ __device__ __forceinline__ void scatter_group(const float2 *__restrict__ slices,
             const float pm[6] = {ra.x, ra.y, ra.z, ra.w, rb.x, rb.y};
             float px, py, pz;
             pixel_coords(x, ry, pm, rtab, H, c.Pf, px, py, pz);
-            const int f0 = (int)floorf(px), f1 = (int)floorf(py), f2 = (int)floorf(pz);
+            const int i0 = (int)floorf(px) - lo[0], i1 = (int)floorf(py) - lo[1], i2 = (int)floorf(pz) - lo[2];
             // x in [0, P/2] holds by construction; origins lie in [-P/2-1, ...): the
             // ones past P/2 only reach cells that are never merged
-            if ((unsigned)x <= (unsigned)H && (unsigned)(f0 - lo[0]) < (unsigned)BRICK &&
-                (unsigned)(f1 - lo[1]) < (unsigned)BRICK && (unsigned)(f2 - lo[2]) < (unsigned)BRICK) {
+            if ((unsigned)x <= (unsigned)H && (unsigned)i0 < (unsigned)BRICK && (unsigned)i1 < (unsigned)BRICK &&
+                (unsigned)i2 < (unsigned)BRICK) {
                 // slice_value() with the conjugation applied after the corner
                 // updates, so that nothing waits for the read before then
                 const bool cj = x == 0 && ry < 0;
@@ -2402,6 +2410,7 @@ __device__ __forceinline__ void scatter_group(const float2 *__restrict__ slices,
                 ns.px = px;
                 ns.py = py;
                 ns.pz = pz;
+                ns.org = i0 + BRICK * (i1 + BRICK * i2) + (acc_slot<A>(i0, i1, i2) << 16);
                 // class_ssnr weighting: the particle's weight at radius hypot_fast_int(x, y)
                 ns.pw = SSNR ? rw[(unsigned long long)(unsigned)__float_as_int(rb.w) * (unsigned)(H + 1) +
                                   (unsigned)hypot_int(x, ry)]
@@ -2410,7 +2419,7 @@ __device__ __forceinline__ void scatter_group(const float2 *__restrict__ slices,
             }
         }
         wave_sync_lds();  // rec reads before the next group rewrites them
-        if (__ballot(win)) scatter_add<A>(st, win, lo, c, acc, etab);
+        if (__ballot(win)) scatter_add<A>(st, win, c, acc);
         if (freed) {
             st.pend = ns.pend;
             if (ns.pend) {
@@ -2429,14 +2438,14 @@ __device__ __forceinline__ void scatter_item(const float2 *__restrict__ slices, 
                                              const float *__restrict__ t3d, const float *__restrict__ wq,
                                              const InsertConst &c, const int *__restrict__ list, const WorkItem &w,
                                              const int lo[3], int lane, float *acc, unsigned char *tag, int *mark,
-                                             float4 *rec, const float *etab, const float *rtab,
-                                             const float *__restrict__ rw, float *out)
+                                             float4 *rec, const float *rtab, const float *__restrict__ rw, float *out)
 {
     PendPix st;
     st.re = st.im = st.pw = 0.f;
     st.px = (float)lo[0];
     st.py = (float)lo[1];
     st.pz = (float)lo[2];
+    st.org = 0;
     st.pend = false;
     bool fresh = false;
     // list entries 64 at a time; each group's slice records fetched one group ahead
@@ -2454,11 +2463,11 @@ __device__ __forceinline__ void scatter_item(const float2 *__restrict__ slices, 
             }
             fetch_group_slice(nxt, s1, w.count, qbuf, qbase, lane, nslices, t3d, wq);
         }
-        scatter_group<A, SSNR>(slices, nsym, cur, c, lo, lane, acc, tag, mark, rec, etab, rtab, rw, st, fresh);
+        scatter_group<A, SSNR>(slices, nsym, cur, c, lo, lane, acc, tag, mark, rec, rtab, rw, st, fresh);
     }
     while (__ballot(st.pend)) {
-        const bool win = scatter_elect(st, fresh, lo, lane, tag);
-        scatter_add<A>(st, win, lo, c, acc, etab);
+        const bool win = scatter_elect(st, fresh, lane, tag);
+        scatter_add<A>(st, win, c, acc);
         st.pend = st.pend && !win;
         fresh = false;
     }
@@ -2477,6 +2486,12 @@ __device__ __forceinline__ void scatter_item(const float2 *__restrict__ slices, 
     wave_sync_lds();
 }
 
+// Bound by the random read-modify-writes into LDS (24 per pixel, about 0.73
+// of the rate at which the LDS serves them alone), the VALU work next to it.
+// Stencil origins kept as a tag and slot index from the bounds test on, table
+// indexes read off the bits of one FMA, and the table at a constant address:
+// 49.0 -> 47.8 ms for 8,000 particles of D7 at pad 288, 18.9 -> 18.5 ms for
+// 24,000 slices at pad 384.
 // SSNR: per-pixel weights from the particles' radial class_ssnr tables rw
 // ((P/2+1) floats per particle) instead of the slice weight.
 template <bool SSNR>
@@ -2488,15 +2503,15 @@ __global__ void __launch_bounds__(256) k_scatter_insert(const float2 *__restrict
                                                         const float *__restrict__ rw)
 {
     extern __shared__ float4 lds4[];
-    char *base = reinterpret_cast<char *>(lds4);
+    float *etab = reinterpret_cast<float *>(lds4);  // from LDS address 0
+    char *base = reinterpret_cast<char *>(etab + EXPN);
     const int lane = threadIdx.x & 63;
     char *mine = base + (size_t)(threadIdx.x >> 6) * WAVE_LDS_BYTES;
     float *acc = reinterpret_cast<float *>(mine);
     float4 *rec = reinterpret_cast<float4 *>(mine + REC_OFF);
     int *mark = reinterpret_cast<int *>(mine + MARK_OFF);
     unsigned char *tag = reinterpret_cast<unsigned char *>(mine + TAG_OFF);
-    float *etab = reinterpret_cast<float *>(base + (size_t)(blockDim.x >> 6) * WAVE_LDS_BYTES);
-    float *rtab = etab + EXPN;  // P+2 entries: fl(i/P), i in [-H, H+1]
+    float *rtab = reinterpret_cast<float *>(base + (size_t)(blockDim.x >> 6) * WAVE_LDS_BYTES);  // P+2 entries: fl(i/P)
     for (int i = threadIdx.x; i < EXPN; i += blockDim.x) etab[i] = exptab_g[i];
     for (int i = threadIdx.x; i < c.P + 2; i += blockDim.x) rtab[i] = rtab_g[i];
     __syncthreads();
@@ -2516,9 +2531,9 @@ __global__ void __launch_bounds__(256) k_scatter_insert(const float2 *__restrict
             if (lane + 64 * wv < 3 * ACC_N) acc[lane + 64 * wv] = 0.f;
         wave_sync_lds();
         float *out = bb.part + (size_t)it * PART_FLOATS;
-        if (A == 0) scatter_item<0, SSNR>(slices, nslices, nsym, t3d, wq, c, bb.list, w, lo, lane, acc, tag, mark, rec, etab, rtab, rw, out);
-        else if (A == 1) scatter_item<1, SSNR>(slices, nslices, nsym, t3d, wq, c, bb.list, w, lo, lane, acc, tag, mark, rec, etab, rtab, rw, out);
-        else scatter_item<2, SSNR>(slices, nslices, nsym, t3d, wq, c, bb.list, w, lo, lane, acc, tag, mark, rec, etab, rtab, rw, out);
+        if (A == 0) scatter_item<0, SSNR>(slices, nslices, nsym, t3d, wq, c, bb.list, w, lo, lane, acc, tag, mark, rec, rtab, rw, out);
+        else if (A == 1) scatter_item<1, SSNR>(slices, nslices, nsym, t3d, wq, c, bb.list, w, lo, lane, acc, tag, mark, rec, rtab, rw, out);
+        else scatter_item<2, SSNR>(slices, nslices, nsym, t3d, wq, c, bb.list, w, lo, lane, acc, tag, mark, rec, rtab, rw, out);
     }
 }
 
