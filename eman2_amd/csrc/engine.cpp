@@ -333,7 +333,7 @@ struct fh_reconstructor {
     float *ximgs = nullptr;     // 2-D transformed padded particles, P x P each
     float *ximgs2 = nullptr;    // second P x P staging: the flipped images' resampling (CTF with a 2-D part)
     float *xfd = nullptr;       // their inverse 2-D transforms, 6 per particle
-    int ximgs_cap = 0, ximgs2_cap = 0;
+    int ximgs_cap = 0, ximgs2_cap = 0, xfd_cap = 0;
     double *partial = nullptr;  // agreement partial sums
     double *acc8 = nullptr;     // batched agreement sums, 8 per particle
     int acc8_cap = 0;
@@ -516,10 +516,8 @@ static int ensure_chunk(fh_reconstructor *h, int n, int B)
     FH_TRY(h, dmalloc(h, &h->dfs, sizeof(float) * n));
     FH_TRY(h, dmalloc(h, &h->dfs2, sizeof(float) * n));
     FH_TRY(h, dmalloc(h, &h->slices, sizeof(float2) * (size_t)n * P * (H + 1)));
-    if (prep_column_first(P)) {
-        h->inter_n = std::min(n, PREP_INTER_PARTICLES);
-        FH_TRY(h, dmalloc(h, &h->inter, prep_inter_bytes(P, h->inter_n)));
-    }
+    h->inter_n = std::min(n, PREP_INTER_PARTICLES);
+    FH_TRY(h, dmalloc(h, &h->inter, prep_inter_bytes(P, h->inter_n)));
     FH_TRY(h, dmalloc(h, &h->t3d, sizeof(float) * 9 * ns));
     FH_TRY(h, dmalloc(h, &h->wq, sizeof(float) * ns));
     if (h->usessnr) FH_TRY(h, dmalloc(h, &h->rw, sizeof(float) * (size_t)n * (H + 1)));
@@ -688,7 +686,7 @@ long long footprint_bytes_for_mode(int P, int nsym, int chunk, const char *mode_
     // per key the slices reach
     const double pb2 = (double)P * P * (2 * g.bs + g.bsz) / (3.0 * g.bs * g.bs * g.bsz);
     const long long part_items = (long long)(1.1 * pb2 * nslices / 64) + g.nkeys / 2;
-    const long long inter = prep_column_first(P) ? (long long)prep_inter_bytes(P, std::min(chunk, PREP_INTER_PARTICLES)) : 0;
+    const long long inter = (long long)prep_inter_bytes(P, std::min(chunk, PREP_INTER_PARTICLES));
     return v + sl + inter + bins + 4LL * g.part_floats * part_items;
 }
 
@@ -903,8 +901,7 @@ int fh_setup_seed_map(fh_reconstructor *h, const float *map)
     if ((rc = ensure_chunk(h, std::max(P, h->cap_n), std::max(P, h->cap_B)))) return rc;
     FH_TRY(h, dmalloc(h, &h->ref, sizeof(float2) * vol_elems(P)));
     FH_TRY(h, h2d_staged(h, h->imgs, map, sizeof(float) * (size_t)P * P * P));
-    FH_TRY(h, launch_fill_f32(h->means, 0.f, P, h->stream));
-    FH_TRY(h, launch_fft3d_forward_corner(h->imgs, P, h->means, h->ref, h->plan, h->tw, h->stream));
+    FH_TRY(h, launch_fft3d_forward_corner(h->imgs, P, h->ref, h->inter, h->inter_n, h->plan, h->tw, h->stream));
     FH_TRY(h, hipStreamSynchronize(h->stream));
     return FH_OK;
 }
@@ -961,54 +958,41 @@ static hipError_t prep_kernels(fh_reconstructor *h, int n, int B, const float *d
     if ((e = launch_edge_mean(dev_imgs, n, B, h->means, h->stream)) != hipSuccess) return e;
     if (xfd && dfd) {
         // the reference's order (e2make3dpar.py:698-716): the padded image is
-        // flipped first -- FFT, CTF_SIGN (times the second sign), inverse FFT
-        // -- and preprocess_slice then resamples the flipped image with the
-        // 2-D part: the whole prep with the flip, back to real space (phase
-        // origin to the centre, 1 / (P^2 scale)), the resampling, the prep
-        // again without flip
+        // flipped first -- FFT, CTF_SIGN (times the second sign), inverse FFT,
+        // through the slices' memory -- and preprocess_slice then resamples the
+        // flipped image with the 2-D part, read by the prep without flip
         const int P = h->P;
-        if ((e = launch_prep2d(dev_imgs, n, B, P, h->means, h->slices, h->inter, h->inter_n, dfd, dfd2, cc, h->scale,
-                               h->plan, h->tw, h->stream)) != hipSuccess)
+        if ((e = launch_flip2d(dev_imgs, n, B, P, h->means, h->slices, h->inter, h->inter_n, dfd, dfd2, cc,
+                               1.0f / ((float)P * (float)P), h->ximgs, h->plan, h->tw, h->stream)) != hipSuccess)
             return e;
-        const float inv = 1.0f / ((float)P * (float)P * h->scale);
-        if ((e = launch_ift2d_batch(h->slices, n, P, h->ximgs, inv, h->plan, h->tw, h->stream)) != hipSuccess) return e;
-        if ((e = launch_fill_f32(h->means, 0.f, n, h->stream)) != hipSuccess) return e;
-        if ((e = launch_xform2d(h->ximgs, n, P, P, h->means, xfd, h->ximgs2, h->stream)) != hipSuccess) return e;
-        return launch_prep2d(h->ximgs2, n, P, P, h->means, h->slices, h->inter, h->inter_n, nullptr, nullptr, cc,
-                             h->scale, h->plan, h->tw, h->stream);
+        return launch_prep2d_xform(h->ximgs, n, P, P, nullptr, xfd, h->slices, h->inter, h->inter_n, h->scale, h->plan,
+                                   h->tw, h->stream);
     }
-    if (xfd) {
-        // pad + 2-D resampling into P x P images, then the prep of those (zero mean)
-        if ((e = launch_xform2d(dev_imgs, n, B, h->P, h->means, xfd, h->ximgs, h->stream)) != hipSuccess) return e;
-        if ((e = launch_fill_f32(h->means, 0.f, n, h->stream)) != hipSuccess) return e;
-        return launch_prep2d(h->ximgs, n, h->P, h->P, h->means, h->slices, h->inter, h->inter_n, nullptr, nullptr, cc,
-                             h->scale, h->plan, h->tw, h->stream);
-    }
+    if (xfd)
+        return launch_prep2d_xform(dev_imgs, n, B, h->P, h->means, xfd, h->slices, h->inter, h->inter_n, h->scale,
+                                   h->plan, h->tw, h->stream);
     return launch_prep2d(dev_imgs, n, B, h->P, h->means, h->slices, h->inter, h->inter_n, dfd, dfd2, cc, h->scale,
                          h->plan, h->tw, h->stream);
 }
 
-// staging of n 2-D transformed particles (P x P) and their inverse transforms;
-// two: also the second P x P buffer of the flip-then-resample order
-static int ensure_ximgs(fh_reconstructor *h, int n, bool two = false)
+// room for n particles' inverse 2-D transforms, and for `stagings` (0-2)
+// P x P images of each: the flipped ones, or projections and their resampling
+static int ensure_ximgs(fh_reconstructor *h, int n, int stagings)
 {
-    if (two && n > h->ximgs2_cap) {
-        if (h->ximgs2) dfree(h, h->ximgs2);
-        h->ximgs2 = nullptr;
-        h->ximgs2_cap = 0;
-        FH_TRY(h, dmalloc(h, &h->ximgs2, sizeof(float) * (size_t)n * h->P * h->P));
-        h->ximgs2_cap = n;
-    }
-    if (n <= h->ximgs_cap) return FH_OK;
-    if (h->ximgs) dfree(h, h->ximgs);
-    if (h->xfd) dfree(h, h->xfd);
-    h->ximgs = nullptr;
-    h->xfd = nullptr;
-    h->ximgs_cap = 0;
-    FH_TRY(h, dmalloc(h, &h->ximgs, sizeof(float) * (size_t)n * h->P * h->P));
-    FH_TRY(h, dmalloc(h, &h->xfd, sizeof(float) * 6 * (size_t)n));
-    h->ximgs_cap = n;
-    return FH_OK;
+    const size_t img = sizeof(float) * (size_t)n * h->P * h->P;
+    auto grow = [&](float *&p, int &cap, size_t bytes) -> int {
+        if (n <= cap) return FH_OK;
+        if (p) dfree(h, p);
+        p = nullptr;
+        cap = 0;
+        FH_TRY(h, dmalloc(h, &p, bytes));
+        cap = n;
+        return FH_OK;
+    };
+    int rc = grow(h->xfd, h->xfd_cap, sizeof(float) * 6 * (size_t)n);
+    if (!rc && stagings > 0) rc = grow(h->ximgs, h->ximgs_cap, img);
+    if (!rc && stagings > 1) rc = grow(h->ximgs2, h->ximgs2_cap, img);
+    return rc;
 }
 
 // prep of n particles already in h->imgs (box B) into h->slices; xf_host:
@@ -1030,7 +1014,7 @@ static int prep_chunk(fh_reconstructor *h, int n, int B, const float *dev_imgs, 
     }
     const float *xfd = nullptr;
     if (xf_host) {
-        int rc = ensure_ximgs(h, n, dfd != nullptr);
+        int rc = ensure_ximgs(h, n, dfd ? 1 : 0);
         if (rc) return rc;
         FH_TRY(h, hipMemcpyAsync(h->xfd, xf_host, sizeof(float) * 6 * n, hipMemcpyHostToDevice, h->stream));
         xfd = h->xfd;
@@ -1045,17 +1029,16 @@ static int prep_chunk(fh_reconstructor *h, int n, int B, const float *dev_imgs, 
 static int prep_single_raw(fh_reconstructor *h, const float *xf6)
 {
     const int P = h->P;
-    FH_TRY(h, launch_fill_f32(h->means, 0.f, 1, h->stream));
-    const float *src = h->imgs;
     if (xf6) {
-        int rc = ensure_ximgs(h, 1);
+        int rc = ensure_ximgs(h, 1, 0);
         if (rc) return rc;
         FH_TRY(h, hipMemcpyAsync(h->xfd, xf6, sizeof(float) * 6, hipMemcpyHostToDevice, h->stream));
-        FH_TRY(h, launch_xform2d(h->imgs, 1, P, P, h->means, h->xfd, h->ximgs, h->stream));
-        src = h->ximgs;
+        FH_TRY(h, launch_prep2d_xform(h->imgs, 1, P, P, nullptr, h->xfd, h->slices, h->inter, h->inter_n, h->scale,
+                                      h->plan, h->tw, h->stream));
+        return FH_OK;
     }
-    FH_TRY(h, launch_prep_rows(src, 1, P, P, h->means, h->slices, h->plan, h->tw, h->stream));
-    FH_TRY(h, launch_prep_cols(1, P, P, h->slices, nullptr, nullptr, CtfConst{}, h->scale, h->plan, h->tw, h->stream));
+    FH_TRY(h, launch_prep2d(h->imgs, 1, P, P, nullptr, h->slices, h->inter, h->inter_n, nullptr, nullptr, CtfConst{},
+                            h->scale, h->plan, h->tw, h->stream));
     return FH_OK;
 }
 
@@ -1072,7 +1055,7 @@ static int insert_batch_graph(fh_reconstructor *h, const float *imgs, int n, int
 {
     int rc = ensure_partials(h, h->bins.item_cap);
     if (rc) return rc;
-    if (xf_host && (rc = ensure_ximgs(h, chunk, defocus && ctf))) return rc;
+    if (xf_host && (rc = ensure_ximgs(h, chunk, defocus && ctf ? 1 : 0))) return rc;
     const InsertConst c = iconst(h);
     fh_stats st{};
     const int wpb = h->tune.waves_per_block;
@@ -1345,8 +1328,8 @@ static int insert_batch_impl(fh_reconstructor *h, const float *imgs, int n, int 
     std::vector<float> df2;
     second_defocus(defocus, ctf, n, df2);
     const float *df2h = df2.empty() ? nullptr : df2.data();
-    // a CTF flip before a 2-D resampling stages two P x P images per particle
-    const long long xbytes = xfh ? ((defocus && ctf) ? 8LL : 4LL) * h->P * h->P : 0;
+    // a CTF flip before a 2-D resampling stages a P x P image per particle
+    const long long xbytes = xfh && defocus && ctf ? 4LL * h->P * h->P : 0;
     // the brick list is indexed with int
     const long long max_slices = std::max(1LL, (long long)INT32_MAX / list_per_slice(brick_geom(h->P, h->mode)) - 1);
     const int chunk = (int)std::max(1LL, std::min({(long long)chunk_for(h->tune, h->P, box, xbytes),
@@ -2015,8 +1998,7 @@ int fh_gauss_fft_volume(fh_reconstructor *h, const float *map)
     // xform.phaseorigin.tocorner and do_fft (projector.cpp:77-79) on the GPU; the
     // Fourier origin shift to the centre is a re-indexing, done by the reads
     FH_TRY(h, h2d_staged(h, h->imgs, map, sizeof(float) * (size_t)P * P * P));
-    FH_TRY(h, launch_fill_f32(h->means, 0.f, P, h->stream));
-    FH_TRY(h, launch_fft3d_forward_corner(h->imgs, P, h->means, h->pvol, h->plan, h->tw, h->stream));
+    FH_TRY(h, launch_fft3d_forward_corner(h->imgs, P, h->pvol, h->inter, h->inter_n, h->plan, h->tw, h->stream));
     FH_TRY(h, hipStreamSynchronize(h->stream));
     return FH_OK;
 }
@@ -2071,7 +2053,7 @@ int fh_gauss_fft_project(fh_reconstructor *h, int n, const float *xforms, int mo
     const int chunk = std::max(1, std::min(n, 4096));
     int rc = ensure_chunk(h, std::max(chunk, h->cap_n), std::max(P, h->cap_B));
     if (rc) return rc;
-    if (!returnfft && (rc = ensure_ximgs(h, chunk))) return rc;
+    if (!returnfft && (rc = ensure_ximgs(h, chunk, 1))) return rc;
     float *tmp = nullptr;  // the projections' records on the device
     FH_TRY(h, dmalloc(h, &tmp, sizeof(float) * 12 * (size_t)chunk));
     float *rec_d = tmp;
@@ -2097,7 +2079,7 @@ int fh_gauss_fft_project(fh_reconstructor *h, int n, const float *xforms, int mo
                     xform2d_inverse(tr, inv);
                     memcpy(&xf6[6 * (size_t)q], inv, sizeof(inv));
                 }
-                if ((rc = ensure_ximgs(h, chunk, true))) {
+                if ((rc = ensure_ximgs(h, chunk, 2))) {
                     dfree(h, tmp);
                     return rc;
                 }

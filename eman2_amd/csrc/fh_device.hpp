@@ -207,40 +207,23 @@ __device__ __forceinline__ void dft<8>(float2 *v)
     v[7] = csub(e[3], o3);
 }
 
-// One Stockham autosort pass over T interleaved transforms of length N:
-// element (t, n) lives at buf[n*T + t].  tw[m] = exp(-2 pi i m / N).  Pass
-// p has stride Ns = prod(radix[<p]); j / Ns is taken with the plan's
-// multiply-high constant.
-template <int R, int T>
-__device__ __forceinline__ void stockham_pass(const float2 *__restrict__ src, float2 *__restrict__ dst,
-                                              int N, int Ns, unsigned mag, int twm, const float2 *__restrict__ tw)
+// The thread index, hidden from the compiler: in a persistent block it would
+// otherwise keep the addresses of every radix's passes in registers across
+// the tiles (1-3 waves per SIMD instead of 3-6).
+__device__ __forceinline__ int opaque_tid()
 {
-    const int NR = N / R;
-    const int total = NR * T;
-    for (int b = threadIdx.x; b < total; b += blockDim.x) {
-        const int t = b % T;
-        const int j = b / T;
-        const int q = Ns == 1 ? j : (int)__umulhi((unsigned)j, mag);
-        const int k = j - q * Ns;
-        float2 v[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            float2 a = src[(j + r * NR) * T + t];
-            if (r > 0) a = cmul(a, tw[r * k * twm]);
-            v[r] = a;
-        }
-        dft<R>(v);
-        const int base = q * Ns * R + k;
-#pragma unroll
-        for (int r = 0; r < R; r++) dst[(base + r * Ns) * T + t] = v[r];
-    }
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    return tid;
 }
 
-// In-place pass: every thread first reads and transforms all of its
-// butterflies (at most G per thread, G * R <= 18 registers of float2), then,
-// after a barrier, writes them back to their Stockham output positions in
-// the same buffer.
-template <int R, int T, int G>
+// One Stockham autosort pass over T interleaved transforms of length N in
+// place: element (t, n) lives at buf[n*T + t].  tw[m] = exp(-2 pi i m / N).
+// Pass p has stride Ns = prod(radix[<p]); j / Ns is taken with the plan's
+// multiply-high constant.  Every thread (of 256) first reads and transforms
+// all of its butterflies (at most G), then, after a barrier, writes them back
+// to their output positions.  FIRST: Ns = 1, unit twiddles.
+template <int R, int T, int G, bool FIRST>
 __device__ __forceinline__ void stockham_pass_inplace(float2 *buf, int N, int Ns, unsigned mag, int twm,
                                                       const float2 *__restrict__ tw)
 {
@@ -248,19 +231,20 @@ __device__ __forceinline__ void stockham_pass_inplace(float2 *buf, int N, int Ns
     const int total = NR * T;
     float2 v[G][R];
     int dsti[G];
+    const int tid = opaque_tid();
 #pragma unroll
     for (int gi = 0; gi < G; gi++) {
-        const int b = threadIdx.x + gi * blockDim.x;
+        const int b = tid + gi * 256;
         dsti[gi] = -1;
         if (b < total) {
             const int t = b % T;
             const int j = b / T;
-            const int q = Ns == 1 ? j : (int)__umulhi((unsigned)j, mag);
-            const int k = j - q * Ns;
+            const int q = FIRST ? j : (int)__umulhi((unsigned)j, mag);
+            const int k = FIRST ? 0 : j - q * Ns;
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 float2 a = buf[(j + r * NR) * T + t];
-                if (r > 0) a = cmul(a, tw[r * k * twm]);
+                if (!FIRST && r > 0) a = cmul(a, tw[r * k * twm]);
                 v[gi][r] = a;
             }
             dft<R>(v[gi]);
@@ -278,56 +262,33 @@ __device__ __forceinline__ void stockham_pass_inplace(float2 *buf, int N, int Ns
     __syncthreads();
 }
 
-// Full forward transform of T interleaved length-N transforms in place in
-// buf (T * N float2), 256 threads; requires N * T <= 3200.  Ends with a
-// barrier.
-template <int T>
-__device__ void fft_lds_inplace(float2 *buf, const FftPlan &plan, const float2 *tw)
+template <int T, int E, bool FIRST>
+__device__ __forceinline__ void stockham_pass_radix(int R, float2 *buf, int N, int Ns, unsigned mag, int twm,
+                                                    const float2 *__restrict__ tw)
 {
-    for (int p = 0; p < plan.npass; p++) {
-        const int R = plan.radix[p], Ns = plan.ns[p];
-        const unsigned mag = plan.mag[p];
-        const int twm = plan.twm[p];
-        switch (R) {
-        case 2: stockham_pass_inplace<2, T, 7>(buf, plan.N, Ns, mag, twm, tw); break;
-        case 3: stockham_pass_inplace<3, T, 5>(buf, plan.N, Ns, mag, twm, tw); break;
-        case 4: stockham_pass_inplace<4, T, 4>(buf, plan.N, Ns, mag, twm, tw); break;
-        case 5: stockham_pass_inplace<5, T, 3>(buf, plan.N, Ns, mag, twm, tw); break;
-        case 6: stockham_pass_inplace<6, T, 3>(buf, plan.N, Ns, mag, twm, tw); break;
-        case 7: stockham_pass_inplace<7, T, 2>(buf, plan.N, Ns, mag, twm, tw); break;
-        case 11: stockham_pass_inplace<11, T, 2>(buf, plan.N, Ns, mag, twm, tw); break;
-        case 13: stockham_pass_inplace<13, T, 1>(buf, plan.N, Ns, mag, twm, tw); break;
-        default: stockham_pass_inplace<8, T, 2>(buf, plan.N, Ns, mag, twm, tw); break;
-        }
+#define FH_RADIX(RR) stockham_pass_inplace<RR, T, (E + RR - 1) / RR, FIRST>(buf, N, Ns, mag, twm, tw)
+    switch (R) {
+    case 2: FH_RADIX(2); break;
+    case 3: FH_RADIX(3); break;
+    case 4: FH_RADIX(4); break;
+    case 5: FH_RADIX(5); break;
+    case 6: FH_RADIX(6); break;
+    case 7: FH_RADIX(7); break;
+    case 11: FH_RADIX(11); break;
+    case 13: FH_RADIX(13); break;
+    default: FH_RADIX(8); break;
     }
+#undef FH_RADIX
 }
 
-// Full forward transform (ping-pong between a and b); returns the buffer that
-// holds the result.  Ends with a barrier.
-template <int T>
-__device__ float2 *fft_lds(float2 *a, float2 *b, const FftPlan &plan, const float2 *tw)
+// Full forward transform of T interleaved transforms of length N in place,
+// 256 threads; requires T N <= 256 E.  Ends with a barrier.
+template <int T, int E>
+__device__ __forceinline__ void fft_lds_inplace(float2 *buf, const FftPlan &plan, const float2 *tw)
 {
-    for (int p = 0; p < plan.npass; p++) {
-        const int R = plan.radix[p], Ns = plan.ns[p];
-        const unsigned mag = plan.mag[p];
-        const int twm = plan.twm[p];
-        switch (R) {
-        case 2: stockham_pass<2, T>(a, b, plan.N, Ns, mag, twm, tw); break;
-        case 3: stockham_pass<3, T>(a, b, plan.N, Ns, mag, twm, tw); break;
-        case 4: stockham_pass<4, T>(a, b, plan.N, Ns, mag, twm, tw); break;
-        case 5: stockham_pass<5, T>(a, b, plan.N, Ns, mag, twm, tw); break;
-        case 6: stockham_pass<6, T>(a, b, plan.N, Ns, mag, twm, tw); break;
-        case 7: stockham_pass<7, T>(a, b, plan.N, Ns, mag, twm, tw); break;
-        case 11: stockham_pass<11, T>(a, b, plan.N, Ns, mag, twm, tw); break;
-        case 13: stockham_pass<13, T>(a, b, plan.N, Ns, mag, twm, tw); break;
-        default: stockham_pass<8, T>(a, b, plan.N, Ns, mag, twm, tw); break;
-        }
-        __syncthreads();
-        float2 *t = a;
-        a = b;
-        b = t;
-    }
-    return a;
+    stockham_pass_radix<T, E, true>(plan.radix[0], buf, plan.N, 1, 0, 0, tw);
+    for (int p = 1; p < plan.npass; p++)
+        stockham_pass_radix<T, E, false>(plan.radix[p], buf, plan.N, plan.ns[p], plan.mag[p], plan.twm[p], tw);
 }
 
 // ---------------------------------------------------------------------------
@@ -404,21 +365,36 @@ __device__ __forceinline__ void fft_fixed(float2 *buf, const float2 *tw)
     }
 }
 
-// In place when the tile fits the register bound of fft_lds_inplace, else
-// ping-pong through b (the launch sizes the LDS accordingly).
-template <int T>
-__device__ __forceinline__ float2 *fft_tile(float2 *a, float2 *b, const FftPlan &plan, const float2 *tw)
-{
-    if (plan.N * T <= 3200) {
-        fft_lds_inplace<T>(a, plan, tw);
-        return a;
-    }
-    return fft_lds<T>(a, b, plan, tw);
-}
-
 __device__ __forceinline__ void load_twiddles(float2 *tw, const float2 *__restrict__ g, int N)
 {
     for (int i = threadIdx.x; i < N; i += blockDim.x) tw[i] = g[i];
+}
+
+// Pixel (i, j) of the "xform" processor's resampling of the centre zero-padded,
+// edge-mean subtracted particle (libEM/processor.cpp:11025-11075): the padded
+// P x P image at inv . (i - P/2, j - P/2) + (P/2, P/2), bilinearly
+// (Util::bilinear_interpolate, libEM/util.h:543-547; the last row/column reuse
+// their own pixel), 0 outside.  m: inv's m00 m01 m03 m10 m11 m13; d: the
+// particle (box B, at padded position off); float operation order as the
+// reference.
+__device__ __forceinline__ float xform_sample(const float *__restrict__ d, int B, int P, int off, float mean,
+                                              const float *__restrict__ m, int i, int j)
+{
+#pragma clang fp contract(off)
+    const float x = (float)(i - P / 2), y = (float)(j - P / 2);
+    const float x2 = (m[0] * x + m[1] * y + m[2]) + (float)(P / 2);
+    const float y2 = (m[3] * x + m[4] * y + m[5]) + (float)(P / 2);
+    if (x2 < 0 || x2 >= (float)P || y2 < 0 || y2 >= (float)P) return 0.0f;
+    const int ii = (int)x2, jj = (int)y2;  // fast_floor of a non-negative value
+    const int i1 = ii == P - 1 ? ii : ii + 1, j1 = jj == P - 1 ? jj : jj + 1;
+    // the padded image: particle pixel minus its edge mean inside the box, 0 outside
+    auto px = [&](int a, int b) -> float {
+        const int xa = a - off, yb = b - off;
+        return ((unsigned)xa < (unsigned)B && (unsigned)yb < (unsigned)B) ? d[(size_t)yb * B + xa] - mean : 0.0f;
+    };
+    const float p1 = px(ii, jj), p2 = px(i1, jj), p3 = px(ii, j1), p4 = px(i1, j1);
+    const float t = x2 - (float)ii, u = y2 - (float)jj;
+    return (1 - t) * (1 - u) * p1 + t * (1 - u) * p2 + (1 - t) * u * p3 + t * u * p4;
 }
 
 }  // namespace fh

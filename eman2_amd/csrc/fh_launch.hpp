@@ -123,17 +123,18 @@ __host__ __device__ constexpr bool gauss6(int mode) { return mode == 2 || mode =
 
 // ---- prep (prep_kernels.hip) ----
 hipError_t launch_edge_mean(const float *imgs, int n, int B, float *means, hipStream_t s);
-hipError_t launch_prep_rows(const float *imgs, int n, int B, int P, const float *means, float2 *slices,
-                            const FftPlan &plan, const float2 *tw, hipStream_t s);
-hipError_t launch_prep_cols(int n, int B, int P, float2 *slices, const float *defocus, const float *defocus2,
-                            CtfConst cc, float scale, const FftPlan &plan, const float2 *tw, hipStream_t s);
 hipError_t launch_ift2d_batch(float2 *data, int n, int P, float *out, float scale, const FftPlan &plan,
                               const float2 *tw, hipStream_t s);
 int prep_inter_pitch(int B);
-bool prep_column_first(int P);
 hipError_t launch_prep2d(const float *imgs, int n, int B, int P, const float *means, float2 *slices,
                          float2 *inter, int inter_n, const float *defocus, const float *defocus2, CtfConst cc,
                          float scale, const FftPlan &plan, const float2 *tw, hipStream_t s);
+hipError_t launch_prep2d_xform(const float *imgs, int n, int B, int P, const float *means, const float *xf,
+                               float2 *slices, float2 *inter, int inter_n, float scale, const FftPlan &plan,
+                               const float2 *tw, hipStream_t s);
+hipError_t launch_flip2d(const float *imgs, int n, int B, int P, const float *means, float2 *work, float2 *inter,
+                         int inter_n, const float *defocus, const float *defocus2, CtfConst cc, float scale,
+                         float *out, const FftPlan &plan, const float2 *tw, hipStream_t s);
 // ---- finish (prep_kernels.hip) ----
 hipError_t launch_normalize(float2 *data, float *norm, int P, int sqrtnorm, float *plane_tmp,
                             hipStream_t s);
@@ -141,8 +142,8 @@ hipError_t launch_fft3d_inverse_zy(float2 *data, int P, const FftPlan &plan, con
                                    hipStream_t s);
 hipError_t launch_c2r_x(const float2 *data, int P, float *out, float scale, const FftPlan &plan,
                         const float2 *tw, hipStream_t s);
-hipError_t launch_fft3d_forward_corner(const float *vol, int P, const float *zeros, float2 *out, const FftPlan &plan,
-                                       const float2 *tw, hipStream_t s);
+hipError_t launch_fft3d_forward_corner(const float *vol, int P, float2 *out, float2 *inter, int inter_n,
+                                       const FftPlan &plan, const float2 *tw, hipStream_t s);
 // gauss_fft projector (modes 0-2) of n projections (rec: 12 floats each) from the map's transform pv
 hipError_t launch_gauss_fft(const float2 *pv, int P, int n, int mode, float gw, const float *rec, int ramp,
                             float2 *out, hipStream_t s);

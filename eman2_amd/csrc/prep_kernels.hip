@@ -35,23 +35,6 @@ bool make_plan(int N, FftPlan *p)
     return true;
 }
 
-// Transforms per block: 4 for the row pass and the finish passes (the
-// in-place tile, 5 P float2 with the twiddles, lets 8 blocks share a CU),
-// 8 for the column pass up to P = 400 (its CTF epilogue keeps it busier per
-// block).  Pads above 3200 / T take the ping-pong form.
-static int pick_T(int P)
-{
-    (void)P;
-    return 4;
-}
-static int pick_T_cols(int P) { return P <= 400 ? 8 : 4; }
-
-// twiddles + one tile (in place) or two (ping-pong), see fft_tile
-static size_t fft_lds_bytes(int P, int T)
-{
-    return sizeof(float2) * (size_t)P * (P * T <= 3200 ? T + 1 : 2 * T + 1);
-}
-
 // ---------------------------------------------------------------- edge mean
 // EMData::get_edge_mean, 2-D branch (libEM/emdata_metadata.cpp:713-736):
 // float pair sums of opposite edge pixels accumulated in double.
@@ -85,143 +68,7 @@ hipError_t launch_edge_mean(const float *imgs, int n, int B, float *means, hipSt
     return hipGetLastError();
 }
 
-// ---------------------------------------------------------------- row pass
-// Each block transforms 2T padded rows of one particle: the rows are packed
-// pairwise into T complex transforms z = a + i c (two-for-one real FFT).
-// Input element xs of padded row yp is the phase-origin shifted
-// (ifftshift) padded image; output row ys = (yp + P/2) mod P.
-// NF: the pad as a compile-time constant (0: the runtime plan and P).
-template <int T, int NF>
-__global__ void __launch_bounds__(256) k_prep_rows(const float *__restrict__ imgs, int B, int Pr, int off,
-                                                   const float *__restrict__ means, float2 *__restrict__ slices,
-                                                   FftPlan plan, const float2 *__restrict__ twg)
-{
-    const int P = NF ? NF : Pr;
-    extern __shared__ float2 smem[];
-    float2 *tw = smem;
-    float2 *A = tw + P;
-    float2 *Bf = A + T * P;
-    const int H = P / 2;
-    const int p = blockIdx.y;
-    const int b0 = blockIdx.x * 2 * T;
-    load_twiddles(tw, twg, P);
-    const float mean = means[p];
-    const float *img = imgs + (size_t)p * B * B;
-    for (int idx = threadIdx.x; idx < T * P; idx += blockDim.x) {
-        const int t = idx % T;  // transform fastest: consecutive LDS slots
-        const int xs = idx / T;
-        const int xp = xs + H < P ? xs + H : xs + H - P;
-        const int bx = xp - off;
-        float re = 0.f, im = 0.f;
-        if (bx >= 0 && bx < B) {
-            const int r0 = b0 + 2 * t;
-            if (r0 < B) re = img[(size_t)r0 * B + bx] - mean;
-            if (r0 + 1 < B) im = img[(size_t)(r0 + 1) * B + bx] - mean;
-        }
-        A[xs * T + t] = make_float2(re, im);
-    }
-    __syncthreads();
-    float2 *R = A;
-    if constexpr (NF != 0) fft_fixed<T, NF>(A, tw);
-    else R = fft_tile<T>(A, Bf, plan, tw);
-    float2 *out = slices + (size_t)p * P * (H + 1);
-    for (int idx = threadIdx.x; idx < T * (H + 1); idx += blockDim.x) {
-        const int t = idx % T;
-        const int k = idx / T;
-        const int r0 = b0 + 2 * t;
-        if (r0 >= B) continue;
-        const float2 z1 = R[k * T + t];
-        const float2 z2 = R[(k == 0 ? 0 : P - k) * T + t];
-        const float2 a = make_float2(0.5f * (z1.x + z2.x), 0.5f * (z1.y - z2.y));
-        const float2 c = make_float2(0.5f * (z1.y + z2.y), -0.5f * (z1.x - z2.x));
-        int ys0 = r0 + off + H;  // < 2P
-        if (ys0 >= P) ys0 -= P;
-        out[(size_t)ys0 * (H + 1) + k] = a;
-        if (r0 + 1 < B) {
-            const int ys1 = ys0 + 1 == P ? 0 : ys0 + 1;
-            out[(size_t)ys1 * (H + 1) + k] = c;
-        }
-    }
-}
-
-// Persistent row pass for the compile-time plans: each block walks tiles
-// (particle, 2T rows) and reads the next tile's pixels into registers while
-// it transforms the current one, so the global read latency hides behind
-// the FFT.  Same arithmetic as k_prep_rows.
-template <int T, int NF>
-__global__ void __launch_bounds__(256) k_prep_rows_pipe(const float *__restrict__ imgs, int B, int off, int n,
-                                                        const float *__restrict__ means, float2 *__restrict__ slices,
-                                                        const float2 *__restrict__ twg)
-{
-    constexpr int P = NF, H = P / 2, KX = (P + 255) / 256;
-    extern __shared__ float2 smem[];
-    float2 *tw = smem;
-    float2 *A = tw + P;
-    load_twiddles(tw, twg, P);
-    const int nrb = (B + 2 * T - 1) / (2 * T);
-    const int ntiles = nrb * n;
-    // raw pixels of a tile: thread x-slot k holds padded column xs = tid + 256 k of all 2T rows, so
-    // each load instruction reads 64 consecutive pixels of one row; out-of-image slots hold the mean
-    // (zero after the subtraction)
-    float v[KX][2 * T];
-    float vmean = 0.f;
-    auto fetch = [&](int tile) {
-        const int p = tile / nrb, b0 = (tile - p * nrb) * 2 * T;
-        const float mean = means[p];
-        const float *img = imgs + (size_t)p * B * B;
-        vmean = mean;
-#pragma unroll
-        for (int k = 0; k < KX; k++) {
-            const int xs = threadIdx.x + 256 * k;
-            const int xp = xs + H < P ? xs + H : xs + H - P;
-            const int bx = xp - off;
-            const bool in = xs < P && bx >= 0 && bx < B;
-#pragma unroll
-            for (int e = 0; e < 2 * T; e++) v[k][e] = in && b0 + e < B ? img[(size_t)(b0 + e) * B + bx] : mean;
-        }
-    };
-    int tile = blockIdx.x;
-    if (tile < ntiles) fetch(tile);
-    for (; tile < ntiles; tile += gridDim.x) {
-        const int p = tile / nrb, b0 = (tile - p * nrb) * 2 * T;
-        const float mean = vmean;
-#pragma unroll
-        for (int k = 0; k < KX; k++) {
-            const int xs = threadIdx.x + 256 * k;
-            if (xs < P) {
-                // transform t takes rows b0 + 2t (real part) and b0 + 2t + 1 (imaginary part)
-                float4 *dst = reinterpret_cast<float4 *>(A + xs * T);
-#pragma unroll
-                for (int t2 = 0; t2 < T / 2; t2++)
-                    dst[t2] = make_float4(v[k][4 * t2] - mean, v[k][4 * t2 + 1] - mean, v[k][4 * t2 + 2] - mean,
-                                          v[k][4 * t2 + 3] - mean);
-            }
-        }
-        __syncthreads();
-        if (tile + (int)gridDim.x < ntiles) fetch(tile + gridDim.x);
-        fft_fixed<T, NF>(A, tw);
-        float2 *out = slices + (size_t)p * P * (H + 1);
-        for (int idx = threadIdx.x; idx < T * (H + 1); idx += 256) {
-            const int t = idx % T;
-            const int k = idx / T;
-            const int r0 = b0 + 2 * t;
-            if (r0 >= B) continue;
-            const float2 z1 = A[k * T + t];
-            const float2 z2 = A[(k == 0 ? 0 : P - k) * T + t];
-            const float2 a = make_float2(0.5f * (z1.x + z2.x), 0.5f * (z1.y - z2.y));
-            const float2 c = make_float2(0.5f * (z1.y + z2.y), -0.5f * (z1.x - z2.x));
-            int ys0 = r0 + off + H;  // < 2P
-            if (ys0 >= P) ys0 -= P;
-            out[(size_t)ys0 * (H + 1) + k] = a;
-            if (r0 + 1 < B) {
-                const int ys1 = ys0 + 1 == P ? 0 : ys0 + 1;
-                out[(size_t)ys1 * (H + 1) + k] = c;
-            }
-        }
-        __syncthreads();  // the tile is read before the next one is stored
-    }
-}
-
+// ---------------------------------------------------------------- launch shapes
 // Compute units of the current device (persistent grids), cached per device.
 static int device_cus()
 {
@@ -236,43 +83,91 @@ static int device_cus()
     return cus[dev];
 }
 
-// Pads with a compile-time plan; others take the runtime plan.
-#define FH_FIXED_PADS(X) X(4, 96) X(4, 192) X(4, 288) X(4, 384) X(4, 480) X(4, 600)
-#define FH_FIXED_PADS_COLS(X) X(8, 96) X(8, 192) X(8, 288) X(8, 384) X(4, 480) X(4, 600)
+// Every transform pass below is one kernel family: T interleaved transforms of
+// length P per tile in LDS, 256 threads, E tile elements per thread, the next
+// tile read into registers while the current one is transformed.  E is a
+// template bound (T P <= 256 E), so that the register arrays and the
+// butterflies per thread are sized to the length's class and not to the
+// longest one.  T = 8 (64-byte runs of adjacent columns) up to P = 400 where
+// the passes walk along columns, 4 above and for the passes along rows.
+#define FH_ROW_CLASS(P, CALL)             \
+    do {                                  \
+        if ((P) <= 256) { CALL(4, 4); }   \
+        else if ((P) <= 512) { CALL(4, 8); } \
+        else if ((P) <= 640) { CALL(4, 10); } \
+        else { CALL(4, 16); }             \
+    } while (0)
+#define FH_COL_CLASS(P, CALL)             \
+    do {                                  \
+        if ((P) <= 128) { CALL(8, 4); }   \
+        else if ((P) <= 256) { CALL(8, 8); } \
+        else if ((P) <= 400) { CALL(8, 13); } \
+        else if ((P) <= 512) { CALL(4, 8); } \
+        else if ((P) <= 640) { CALL(4, 10); } \
+        else { CALL(4, 16); }             \
+    } while (0)
 
-hipError_t launch_prep_rows(const float *imgs, int n, int B, int P, const float *means, float2 *slices,
-                            const FftPlan &plan, const float2 *tw, hipStream_t s)
-{
-    if (n <= 0) return hipSuccess;
-    // centre zero-pad (clip_inplace Region((B-P)//2, ...), e2make3dpar.py:651-652)
-    const int d = B - P;
-    const int fl = d >= 0 ? d / 2 : -((-d + 1) / 2);
-    const int off = -fl;
-    const int T = pick_T(P);
-    const size_t lds = fft_lds_bytes(P, T);
-    dim3 grid((B + 2 * T - 1) / (2 * T), n);
-    const int ntiles = (int)grid.x * n;
-#define FH_ROWS_CASE(TT, NN)                                                                                    \
-    if (T == TT && P == NN) {                                                                                   \
-        int per = 0;                                                                                            \
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_prep_rows_pipe<TT, NN>, 256, lds) != hipSuccess || \
-            per < 1)                                                                                            \
-            per = 1;                                                                                            \
-        const int pgrid = std::min(ntiles, device_cus() * per);                                                 \
-        hipLaunchKernelGGL((k_prep_rows_pipe<TT, NN>), dim3(pgrid), dim3(256), lds, s, imgs, B, off, n, means, slices, \
-                           tw);                                                                                 \
-        return hipGetLastError();                                                                               \
+// Pads with a compile-time plan; others take the runtime plan.
+#define FIXED_PADS(X) X(96) X(192) X(288) X(384) X(480) X(600)
+
+// Waves per SIMD the register allocation of the runtime-plan passes must
+// allow (none of them spills; the compile-time ones are left alone, held to
+// 3-4 waves they spill at 600 and take 1.67 instead of 1.12 ms).
+constexpr int tile_waves(int nf, int E) { return nf ? 1 : E <= 4 ? 5 : E <= 8 ? 4 : E < 16 ? 3 : 2; }
+
+// twiddles + one tile
+static size_t tile_lds(int P, int T) { return sizeof(float2) * (size_t)P * (T + 1); }
+
+// Persistent blocks: the tiles of XCD x (blocks b = x mod 8) are the
+// contiguous range [x ntiles / 8, (x + 1) ntiles / 8), so the tiles that share
+// cache lines meet in the same L2.
+struct TileWalk {
+    int t, end, step;
+    __device__ TileWalk(int ntiles)
+    {
+        const int G8 = gridDim.x / 8, x = blockIdx.x % 8, lb = blockIdx.x / 8;
+        const int lo = (int)((long long)ntiles * x / 8), hi = (int)((long long)ntiles * (x + 1) / 8);
+        t = lo + lb;
+        end = hi;
+        step = G8;
     }
-    FH_FIXED_PADS(FH_ROWS_CASE)
-#undef FH_ROWS_CASE
-    if (T == 8)
-        hipLaunchKernelGGL((k_prep_rows<8, 0>), grid, dim3(256), lds, s, imgs, B, P, off, means, slices, plan, tw);
-    else
-        hipLaunchKernelGGL((k_prep_rows<4, 0>), grid, dim3(256), lds, s, imgs, B, P, off, means, slices, plan, tw);
-    return hipGetLastError();
+};
+
+// Their grid: resident blocks per CU times the CUs, a multiple of 8 (one
+// share per XCD), at most the tiles rounded up to 8.
+template <typename K>
+static int persistent_grid(K kernel, size_t lds, int ntiles)
+{
+    const int cus = device_cus();
+    if (ntiles <= cus) return (ntiles + 7) / 8 * 8;
+    int per = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, 256, lds) != hipSuccess || per < 1) per = 1;
+    const int g = std::min(cus * per, (ntiles + 7) / 8 * 8);
+    return std::max(8, g / 8 * 8);
 }
 
-// ---------------------------------------------------------------- column pass
+// fixed plan (NF, compile time) or the runtime plan
+template <int T, int NF, int E>
+__device__ __forceinline__ void fft_run(float2 *A, const FftPlan &plan, const float2 *tw)
+{
+    if constexpr (NF != 0) fft_fixed<T, NF>(A, tw);
+    else fft_lds_inplace<T, E>(A, plan, tw);
+}
+
+// The spectra a, c (k = 0..P/2) of two real signals A, C as the conjugate of
+// A + iC, element k and its mirror P - k: a forward transform of it is the
+// conjugate of the pair's inverse transform.
+template <int T>
+__device__ __forceinline__ void store_pair(float2 *A, int k, int t, int P, float4 v)
+{
+    const int H = P / 2;
+    const bool self = k == 0 || k == H;
+    if (self) v.y = v.w = 0.f;
+    A[k * T + t] = make_float2(v.x - v.w, -(v.y + v.z));
+    if (!self) A[(P - k) * T + t] = make_float2(v.x + v.w, v.y - v.z);
+}
+
+// ---------------------------------------------------------------- CTF sign
 // CTF_SIGN of EMAN2Ctf::compute_2d_complex (libEM/ctf.cpp:1076-1090) at
 // the Fourier pixel of radius hyp = Util::hypot_fast(x, y).  Evaluated with the reference's float
 // operation order (no contraction); the sign of cos is taken in double.
@@ -300,100 +195,9 @@ __device__ __forceinline__ float ctf_sign(float hyp, float defocus, const CtfCon
     return cos(t) < 0 ? -1.0f : 1.0f;
 }
 
-// defocus2 (optional): a second defocus per particle; the flip is then the
-// product of the two signs (the dfdf flip of e2make3dpar.py:698-709)
-template <int T, int NF>
-__global__ void __launch_bounds__(256) k_prep_cols(int B, int Pr, int off, float2 *__restrict__ slices,
-                                                   const float *__restrict__ defocus,
-                                                   const float *__restrict__ defocus2, CtfConst cc, float scale,
-                                                   FftPlan plan, const float2 *__restrict__ twg)
-{
-    const int P = NF ? NF : Pr;
-    extern __shared__ float2 smem[];
-    float2 *tw = smem;
-    float2 *A = tw + P;
-    float2 *Bf = A + T * P;
-    const int H = P / 2;
-    // XCD-aware order: the hardware deals consecutive blocks round-robin to
-    // the 8 XCDs (separate L2s); blocks k, k+8, k+16, ... of one XCD take
-    // consecutive (column group, particle) tiles, so the column groups that
-    // share a cache line meet in the same L2.
-    unsigned lin = blockIdx.x + gridDim.x * blockIdx.y;
-    const unsigned per = (gridDim.x * gridDim.y) / 8;
-    if (lin < 8 * per) lin = (lin % 8) * per + lin / 8;
-    const int p = (int)(lin / gridDim.x);
-    const int x0 = (int)(lin % gridDim.x) * T;
-    load_twiddles(tw, twg, P);
-    float2 *sl = slices + (size_t)p * P * (H + 1);
-    for (int idx = threadIdx.x; idx < T * P; idx += blockDim.x) {
-        const int y = idx / T;
-        const int t = idx - y * T;
-        const int x = x0 + t;
-        int b = y - off - H;  // in [-P, P/2)
-        if (b < 0) b += P;
-        float2 v = make_float2(0.f, 0.f);
-        if (x <= H && b < B) v = sl[(size_t)y * (H + 1) + x];
-        A[y * T + t] = v;
-    }
-    __syncthreads();
-    float2 *R = A;
-    if constexpr (NF != 0) fft_fixed<T, NF>(A, tw);
-    else R = fft_tile<T>(A, Bf, plan, tw);
-    const float df = defocus ? defocus[p] : 0.f;
-    const float df2 = defocus2 ? defocus2[p] : 0.f;
-    // the sign depends on x^2 + y^2 only: rows y and P - y (signed y and -y,
-    // 0 < y < P/2) share one evaluation
-    for (int idx = threadIdx.x; idx < T * (H + 1); idx += blockDim.x) {
-        const int y = idx / T;  // 0 .. P/2; row P/2 is signed -P/2
-        const int t = idx - y * T;
-        const int x = x0 + t;
-        if (x > H) continue;
-        // (v * (sg + 0i)) * scale with sg = +-1 equals v * (sg * scale) exactly
-        // (up to the sign of a zero)
-        const float hyp = defocus ? sqrt_int_rn(x * x + y * y) : 0.f;  // Util::hypot_fast(x, y)
-        float ss = defocus ? ctf_sign(hyp, df, cc) * scale : scale;
-        if (defocus2) ss = ss * ctf_sign(hyp, df2, cc);
-#pragma unroll
-        for (int m = 0; m < 2; m++) {
-            const int row = m == 0 ? y : P - y;
-            if (m == 1 && (y == 0 || y == H)) break;
-            const float2 v = R[row * T + t];
-            sl[(size_t)row * (H + 1) + x] = make_float2(v.x * ss, v.y * ss);
-        }
-    }
-}
-
-hipError_t launch_prep_cols(int n, int B, int P, float2 *slices, const float *defocus, const float *defocus2,
-                            CtfConst cc, float scale, const FftPlan &plan, const float2 *tw, hipStream_t s)
-{
-    if (n <= 0) return hipSuccess;
-    const int d = B - P;
-    const int fl = d >= 0 ? d / 2 : -((-d + 1) / 2);
-    const int off = -fl;
-    const int T = pick_T_cols(P);
-    const int H = P / 2;
-    const size_t lds = fft_lds_bytes(P, T);
-    dim3 grid((H + 1 + T - 1) / T, n);
-#define FH_COLS_CASE(TT, NN)                                                                                      \
-    if (T == TT && P == NN) {                                                                                     \
-        hipLaunchKernelGGL((k_prep_cols<TT, NN>), grid, dim3(256), lds, s, B, P, off, slices, defocus, defocus2, cc, \
-                           scale, plan, tw);                                                                      \
-        return hipGetLastError();                                                                                 \
-    }
-    FH_FIXED_PADS_COLS(FH_COLS_CASE)
-#undef FH_COLS_CASE
-    if (T == 8)
-        hipLaunchKernelGGL((k_prep_cols<8, 0>), grid, dim3(256), lds, s, B, P, off, slices, defocus, defocus2, cc, scale,
-                           plan, tw);
-    else
-        hipLaunchKernelGGL((k_prep_cols<4, 0>), grid, dim3(256), lds, s, B, P, off, slices, defocus, defocus2, cc, scale,
-                           plan, tw);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------- column-first prep
-// The compile-time pads take the 2-D r2c transform columns first, so that
-// the larger second pass reads and writes whole rows.
+// ---------------------------------------------------------------- 2-D prep
+// The 2-D r2c transform runs columns first, so that the larger second pass
+// reads and writes whole rows.
 // Pass 1 (k_prep_ycols): 2T image columns per block, packed pairwise into T
 // complex transforms along y (padded row ys = (b + off + P/2) mod P of image
 // row b, edge mean subtracted, zero outside the image); the half spectrum
@@ -405,74 +209,79 @@ hipError_t launch_prep_cols(int n, int B, int P, float2 *slices, const float *de
 // kx = 0..P/2 and, for 0 < ky < P/2, row P - ky takes the conjugates of
 // kx' = (P - kx) mod P (F(kx, -ky) = conj F(-kx, ky) for a real image), both
 // times the CTF sign and scale of (kx, |ky|), evaluated once for the pair.
-// The same output as k_prep_rows + k_prep_cols up to float rounding.
-// Persistent blocks: the tiles of XCD x (blocks b = x mod 8) are the
-// contiguous range [x ntiles / 8, (x + 1) ntiles / 8), so the tiles of a
-// particle that share cache lines meet in the same L2; each block reads the
-// next tile into registers while it transforms and stores the current one.
-struct TileWalk {
-    int t, end, step;
-    __device__ TileWalk(int ntiles)
-    {
-        const int G8 = gridDim.x / 8, x = blockIdx.x % 8, lb = blockIdx.x / 8;
-        const int lo = (int)((long long)ntiles * x / 8), hi = (int)((long long)ntiles * (x + 1) / 8);
-        t = lo + lb;
-        end = hi;
-        step = G8;
-    }
-};
-
-template <int T, int NF>
-__global__ void __launch_bounds__(256) k_prep_ycols(const float *__restrict__ imgs, int B, int off, int n,
-                                                    const float *__restrict__ means, float2 *__restrict__ inter,
-                                                    int IP, const float2 *__restrict__ twg)
+// XF: the image of pass 1 is the "xform" processor's resampling of the
+// source (xform_sample), taken where it is read, all P x P of it.
+// FLIP: pass 2 of the flip back to real space: the row's spectrum times the
+// sign goes through the inverse x transform in the same tile, and row ky of
+// J[p][ky][x] (pitch P, the slice's own memory) is written; pass 3
+// (k_flip_ycols) takes J back along y to the flipped P x P image.
+// Bound by memory where the plan is a compile-time one (2.0 and 3.0 GB per
+// 3,000 particles of 256 px at pad 384 in 0.54 and 0.78 ms, 3.8 TB/s; a copy
+// reaches 4.9), by address and twiddle arithmetic where it is not: the same
+// through the runtime plan 0.58 and 1.03 ms.  5,000 particles of 169 px at pad
+// 256, flipped, resampled and transformed again: 5.1 ms, 8.9 by rows, then
+// columns in place, columns back, rows back and a resampling pass.
+template <int T, int NF, int E, bool XF>
+__global__ void __launch_bounds__(256, tile_waves(NF, E))
+    k_prep_ycols(const float *__restrict__ imgs, int B, int Pr, int off, int n, const float *__restrict__ means,
+                 const float *__restrict__ xf, float2 *__restrict__ inter, int IP, FftPlan plan,
+                 const float2 *__restrict__ twg)
 {
-    constexpr int P = NF, H = P / 2, E = (T * P + 255) / 256;
+    const int P = NF ? NF : Pr, H = P / 2;
+    constexpr int EL = NF ? (T * NF + 255) / 256 : E;
+    const int Bv = XF ? P : B, offv = XF ? 0 : off;  // the image that is transformed
     extern __shared__ float2 smem[];
     float2 *tw = smem;
     float2 *A = tw + P;
     load_twiddles(tw, twg, P);
-    const int ng = (B + 2 * T - 1) / (2 * T);
+    const int ng = (Bv + 2 * T - 1) / (2 * T);
     TileWalk w(ng * n);
     // element e of the thread: (ys, t) = ((tid + 256 e) / T, (tid + 256 e) % T), image columns c, c + 1
     // of padded row ys; slots outside the image hold the mean (zero after the subtraction)
-    float2 v[E];
+    float2 v[EL];
     float vmean = 0.f;
     auto fetch = [&](int tile) {
+        const int tid = NF ? (int)threadIdx.x : opaque_tid();
         const int p = tile / ng, c0 = (tile - p * ng) * 2 * T;
-        const float mean = means[p];
+        const float mean = means ? means[p] : 0.f;
         const float *img = imgs + (size_t)p * B * B;
-        vmean = mean;
+        vmean = XF ? 0.f : mean;
 #pragma unroll
-        for (int e = 0; e < E; e++) {
-            const int idx = threadIdx.x + 256 * e;
+        for (int e = 0; e < EL; e++) {
+            const int idx = tid + 256 * e;
             const int t = idx % T, ys = idx / T;
-            int b = ys - off - H;  // image row of padded row ys, in [-P, P/2)
+            int b = ys - offv - H;  // image row of padded row ys, in [-P, P/2)
             if (b < 0) b += P;
             const int c = c0 + 2 * t;
-            const bool in = idx < T * P && b < B;
-            v[e].x = in && c < B ? img[(size_t)b * B + c] : mean;
-            v[e].y = in && c + 1 < B ? img[(size_t)b * B + c + 1] : mean;
+            const bool in = idx < T * P && b < Bv;
+            if constexpr (XF) {
+                v[e].x = in && c < Bv ? xform_sample(img, B, P, off, mean, xf + 6 * (size_t)p, c, b) : 0.f;
+                v[e].y = in && c + 1 < Bv ? xform_sample(img, B, P, off, mean, xf + 6 * (size_t)p, c + 1, b) : 0.f;
+            } else {
+                v[e].x = in && c < Bv ? img[(size_t)b * B + c] : mean;
+                v[e].y = in && c + 1 < Bv ? img[(size_t)b * B + c + 1] : mean;
+            }
         }
     };
     if (w.t < w.end) fetch(w.t);
     for (; w.t < w.end; w.t += w.step) {
+        const int tid = NF ? (int)threadIdx.x : opaque_tid();
         const int p = w.t / ng, c0 = (w.t - p * ng) * 2 * T;
         const float mean = vmean;
 #pragma unroll
-        for (int e = 0; e < E; e++) {
-            const int idx = threadIdx.x + 256 * e;
-            if (E * 256 == T * P || idx < T * P) A[idx] = make_float2(v[e].x - mean, v[e].y - mean);  // A[ys T + t]
+        for (int e = 0; e < EL; e++) {
+            const int idx = tid + 256 * e;
+            if (idx < T * P) A[idx] = make_float2(v[e].x - mean, v[e].y - mean);  // A[ys T + t]
         }
         __syncthreads();
         if (w.t + w.step < w.end) fetch(w.t + w.step);
-        fft_fixed<T, NF>(A, tw);
+        fft_run<T, NF, E>(A, plan, tw);
         float2 *I = inter + (size_t)p * (H + 1) * IP;
-        for (int idx = threadIdx.x; idx < T * (H + 1); idx += 256) {
+        for (int idx = tid; idx < T * (H + 1); idx += 256) {
             const int t = idx % T;
             const int k = idx / T;
             const int c = c0 + 2 * t;
-            if (c >= B) continue;
+            if (c >= Bv) continue;
             const float2 z1 = A[k * T + t];
             const float2 z2 = A[(k == 0 ? 0 : P - k) * T + t];
             // columns c and c + 1 (for odd B the last pair's second column is
@@ -484,13 +293,16 @@ __global__ void __launch_bounds__(256) k_prep_ycols(const float *__restrict__ im
     }
 }
 
-template <int T, int NF>
-__global__ void __launch_bounds__(256) k_prep_xrows(int B, int off, int n, const float2 *__restrict__ inter, int IP,
-                                                    float2 *__restrict__ slices, const float *__restrict__ defocus,
-                                                    const float *__restrict__ defocus2, CtfConst cc, float scale,
-                                                    const float2 *__restrict__ twg)
+// defocus2 (optional): a second defocus per particle; the flip is then the
+// product of the two signs (the dfdf flip of e2make3dpar.py:698-709)
+template <int T, int NF, int E, bool FLIP>
+__global__ void __launch_bounds__(256, tile_waves(NF, E))
+    k_prep_xrows(int B, int Pr, int off, int n, const float2 *__restrict__ inter, int IP, float2 *__restrict__ slices,
+                 const float *__restrict__ defocus, const float *__restrict__ defocus2, CtfConst cc, float scale,
+                 FftPlan plan, const float2 *__restrict__ twg)
 {
-    constexpr int P = NF, H = P / 2, E = (T * P + 255) / 256, NG = (H + 1 + T - 1) / T;
+    const int P = NF ? NF : Pr, H = P / 2, NG = (H + T) / T;
+    constexpr int EL = NF ? (T * NF + 255) / 256 : E;
     extern __shared__ float2 smem[];
     float2 *tw = smem;
     float2 *A = tw + P;
@@ -498,13 +310,14 @@ __global__ void __launch_bounds__(256) k_prep_xrows(int B, int off, int n, const
     TileWalk w(NG * n);
     // element e of the thread: (xs, t) = ((tid + 256 e) / T, (tid + 256 e) % T): a wave reads runs of
     // 64 / T columns of T intermediate rows and writes LDS without bank conflicts
-    float2 v[E];
+    float2 v[EL];
     auto fetch = [&](int tile) {
+        const int tid = NF ? (int)threadIdx.x : opaque_tid();
         const int p = tile / NG, k0 = (tile - p * NG) * T;
         const float2 *I = inter + (size_t)p * (H + 1) * IP;
 #pragma unroll
-        for (int e = 0; e < E; e++) {
-            const int idx = threadIdx.x + 256 * e;
+        for (int e = 0; e < EL; e++) {
+            const int idx = tid + 256 * e;
             const int t = idx % T, xs = idx / T;
             const int k = k0 + t;
             int c = xs - off - H;  // image column of padded column xs
@@ -514,109 +327,233 @@ __global__ void __launch_bounds__(256) k_prep_xrows(int B, int off, int n, const
     };
     if (w.t < w.end) fetch(w.t);
     for (; w.t < w.end; w.t += w.step) {
+        const int tid = NF ? (int)threadIdx.x : opaque_tid();
         const int p = w.t / NG, k0 = (w.t - p * NG) * T;
 #pragma unroll
-        for (int e = 0; e < E; e++) {
-            const int idx = threadIdx.x + 256 * e;
-            if (E * 256 == T * P || idx < T * P) A[idx] = v[e];  // A[xs T + t]
+        for (int e = 0; e < EL; e++) {
+            const int idx = tid + 256 * e;
+            if (idx < T * P) A[idx] = v[e];  // A[xs T + t]
         }
         __syncthreads();
         if (w.t + w.step < w.end) fetch(w.t + w.step);
-        fft_fixed<T, NF>(A, tw);
+        fft_run<T, NF, E>(A, plan, tw);
         const float df = defocus ? defocus[p] : 0.f;
         const float df2 = defocus2 ? defocus2[p] : 0.f;
+        auto flip = [&](int kx, int ky) {  // sign times scale
+            const float hyp = defocus ? sqrt_int_rn(kx * kx + ky * ky) : 0.f;  // Util::hypot_fast(x, y)
+            float ss = defocus ? ctf_sign(hyp, df, cc) * scale : scale;
+            if (defocus2) ss = ss * ctf_sign(hyp, df2, cc);
+            return ss;
+        };
         float2 *sl = slices + (size_t)p * P * (H + 1);
-        // two rows per lane (one 16-byte LDS read per column), lanes along the
-        // rows: whole-row store runs
-        static_assert(T % 2 == 0, "row pairs");
-        for (int idx = threadIdx.x; idx < (T / 2) * (H + 1); idx += 256) {
-            const int t0 = 2 * (idx / (H + 1));
-            const int kx = idx - (t0 / 2) * (H + 1);
-            const float4 u2 = *reinterpret_cast<const float4 *>(A + kx * T + t0);
-            const float4 q2 = *reinterpret_cast<const float4 *>(A + (kx == 0 ? 0 : P - kx) * T + t0);
+        if constexpr (FLIP) {
+            for (int idx = tid; idx < T * (H + 1); idx += 256) {
+                const int t = idx % T, k = idx / T;
+                const float ss = flip(k, k0 + t);
+                float2 *a = A + k * T + t;
+                *a = make_float2(a->x * ss, -(a->y * ss));
+                if (k > 0 && k < H) {
+                    a = A + (P - k) * T + t;
+                    *a = make_float2(a->x * ss, -(a->y * ss));
+                }
+            }
+            __syncthreads();
+            fft_run<T, NF, E>(A, plan, tw);
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int ky = k0 + t0 + h;
-                if (ky > H) continue;
-                const float hyp = defocus ? sqrt_int_rn(kx * kx + ky * ky) : 0.f;  // Util::hypot_fast(x, y)
-                float ss = defocus ? ctf_sign(hyp, df, cc) * scale : scale;
-                if (defocus2) ss = ss * ctf_sign(hyp, df2, cc);
-                const float ux = h ? u2.z : u2.x, uy = h ? u2.w : u2.y;
-                const float qx = h ? q2.z : q2.x, qy = h ? q2.w : q2.y;
-                sl[(size_t)ky * (H + 1) + kx] = make_float2(ux * ss, uy * ss);
-                if (ky > 0 && ky < H) sl[(size_t)(P - ky) * (H + 1) + kx] = make_float2(qx * ss, -qy * ss);
+            for (int e = 0; e < EL; e++) {
+                const int idx = tid + 256 * e;
+                const int t = idx % T, xs = idx / T;
+                if (idx < T * P && k0 + t <= H) sl[(size_t)(k0 + t) * P + xs] = make_float2(A[idx].x, -A[idx].y);
+            }
+        } else {
+            // two rows per lane (one 16-byte LDS read per column), lanes along the
+            // rows: whole-row store runs
+            static_assert(T % 2 == 0, "row pairs");
+            constexpr int TH = 256 / (T / 2);  // threads per row pair
+            const int t0 = 2 * (tid / TH);
+            for (int kx = tid % TH; kx <= H; kx += TH) {
+                const float4 u2 = *reinterpret_cast<const float4 *>(A + kx * T + t0);
+                const float4 q2 = *reinterpret_cast<const float4 *>(A + (kx == 0 ? 0 : P - kx) * T + t0);
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int ky = k0 + t0 + h;
+                    if (ky > H) continue;
+                    const float ss = flip(kx, ky);
+                    const float ux = h ? u2.z : u2.x, uy = h ? u2.w : u2.y;
+                    const float qx = h ? q2.z : q2.x, qy = h ? q2.w : q2.y;
+                    sl[(size_t)ky * (H + 1) + kx] = make_float2(ux * ss, uy * ss);
+                    if (ky > 0 && ky < H) sl[(size_t)(P - ky) * (H + 1) + kx] = make_float2(qx * ss, -qy * ss);
+                }
             }
         }
         __syncthreads();  // the tile is read before the next one is stored
     }
 }
 
-// Persistent grid of a column-first pass: resident blocks per CU times the
-// CUs, a multiple of 8 (one share per XCD), at most the tiles rounded up to 8.
-template <typename K>
-static int persistent_grid(K kernel, size_t lds, int ntiles)
+// J[p][ky][x] (k_prep_xrows<FLIP>) along y to real P x P images times scale,
+// phase origin to the centre: pairs of real columns per complex transform
+template <int T, int E>
+__global__ void __launch_bounds__(256, tile_waves(0, E))
+    k_flip_ycols(const float2 *__restrict__ J, int P, int n, float *__restrict__ out, float scale, FftPlan plan,
+                 const float2 *__restrict__ twg)
 {
-    int per = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, 256, lds) != hipSuccess || per < 1) per = 1;
-    const int g = std::min(device_cus() * per, (ntiles + 7) / 8 * 8);
-    return std::max(8, g / 8 * 8);
+    const int H = P / 2, ng = (P + 2 * T - 1) / (2 * T);
+    constexpr int EH = E / 2 + 1;
+    extern __shared__ float2 smem[];
+    float2 *tw = smem;
+    float2 *A = tw + P;
+    load_twiddles(tw, twg, P);
+    TileWalk w(ng * n);
+    float4 v[EH];
+    auto fetch = [&](int tile) {
+        const int tid = opaque_tid();
+        const int p = tile / ng, c0 = (tile - p * ng) * 2 * T;
+        const float2 *src = J + (size_t)p * P * (H + 1);
+#pragma unroll
+        for (int e = 0; e < EH; e++) {
+            const int idx = tid + 256 * e;
+            const int c = c0 + 2 * (idx % T), k = idx / T;
+            v[e] = k <= H && c < P ? *reinterpret_cast<const float4 *>(src + (size_t)k * P + c)
+                                   : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    if (w.t < w.end) fetch(w.t);
+    for (; w.t < w.end; w.t += w.step) {
+        const int tid = opaque_tid();
+        const int p = w.t / ng, c0 = (w.t - p * ng) * 2 * T;
+#pragma unroll
+        for (int e = 0; e < EH; e++) {
+            const int idx = tid + 256 * e;
+            if (idx / T <= H) store_pair<T>(A, idx / T, idx % T, P, v[e]);
+        }
+        __syncthreads();
+        if (w.t + w.step < w.end) fetch(w.t + w.step);
+        fft_run<T, 0, E>(A, plan, tw);
+        float *o = out + (size_t)p * P * P;
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int idx = tid + 256 * e;
+            const int c = c0 + 2 * (idx % T), y = idx / T;
+            if (y >= P || c >= P) continue;
+            const float2 r = A[idx];
+            float *row = o + (size_t)(y + H < P ? y + H : y + H - P) * P;
+            row[c + H < P ? c + H : c + H - P] = r.x * scale;
+            row[c + 1 + H < P ? c + 1 + H : c + 1 + H - P] = -r.y * scale;
+        }
+        __syncthreads();  // the tile is read before the next one is stored
+    }
 }
 
 // Intermediate row pitch of box B (a multiple of 16 columns: 128-byte rows,
 // and one padding column for odd B).
 int prep_inter_pitch(int B) { return (B + 16) & ~15; }
 
-bool prep_column_first(int P)
-{
-#define FH_CF_CASE(TT, NN) if (P == NN) return true;
-    FH_FIXED_PADS(FH_CF_CASE)
-#undef FH_CF_CASE
-    return false;
-}
-
-// The whole prep of n particles: column-first through `inter` (room for
-// inter_n particles of box P) in sub-batches for the compile-time pads, else
-// the row pass and the column pass in place.
-hipError_t launch_prep2d(const float *imgs, int n, int B, int P, const float *means, float2 *slices,
-                         float2 *inter, int inter_n, const float *defocus, const float *defocus2, CtfConst cc,
-                         float scale, const FftPlan &plan, const float2 *tw, hipStream_t s)
+// n particles through the two passes, in sub-batches of the intermediate's
+// room (inter_n particles of box P).  xf: resample by these inverse 2-D
+// transforms first; flip_back: leave J instead of slices.
+static hipError_t prep2d_passes(const float *imgs, int n, int B, int P, const float *means, const float *xf,
+                                bool flip_back, float2 *slices, float2 *inter, int inter_n, const float *defocus,
+                                const float *defocus2, CtfConst cc, float scale, const FftPlan &plan, const float2 *tw,
+                                hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    if (!inter || inter_n <= 0 || !prep_column_first(P) || B > P) {
-        hipError_t e = launch_prep_rows(imgs, n, B, P, means, slices, plan, tw, s);
-        if (e != hipSuccess) return e;
-        return launch_prep_cols(n, B, P, slices, defocus, defocus2, cc, scale, plan, tw, s);
-    }
     const int d = B - P;
-    const int fl = d >= 0 ? d / 2 : -((-d + 1) / 2);  // (B - P) // 2, as in the row pass
+    const int fl = d >= 0 ? d / 2 : -((-d + 1) / 2);  // clip_inplace Region((B-P)//2, ...), e2make3dpar.py:651-652
     const int off = -fl;
-    const int H = P / 2, IP = prep_inter_pitch(B);
-    // particles per sub-batch: inter holds inter_n particles at the pitch of box P
+    const int Bt = xf ? P : B, offt = xf ? 0 : off;  // what is transformed
+    const int H = P / 2, IP = prep_inter_pitch(Bt);
     const long long room = (long long)inter_n * prep_inter_pitch(P);
     const int sub = (int)std::max(1LL, room / IP);
     for (int i0 = 0; i0 < n; i0 += sub) {
         const int m = std::min(sub, n - i0);
         const float *im = imgs + (size_t)i0 * B * B;
-        const float *mn = means + i0;
+        const float *mn = means ? means + i0 : nullptr;
+        const float *xm = xf ? xf + 6 * (size_t)i0 : nullptr;
         float2 *sl = slices + (size_t)i0 * P * (H + 1);
         const float *df = defocus ? defocus + i0 : nullptr;
         const float *df2 = defocus2 ? defocus2 + i0 : nullptr;
-#define FH_CF_LAUNCH(TT, NN)                                                                                      \
-        if (P == NN) {                                                                                            \
-            constexpr int T1 = 8, T2 = 4;                                                         \
-            const size_t l1 = sizeof(float2) * (T1 + 1) * NN, l2 = sizeof(float2) * (T2 + 1) * NN;                \
-            const int g1 = persistent_grid(k_prep_ycols<T1, NN>, l1, (B + 2 * T1 - 1) / (2 * T1) * m);              \
-            const int g2 = persistent_grid(k_prep_xrows<T2, NN>, l2, (H + T2) / T2 * m);                          \
-            hipLaunchKernelGGL((k_prep_ycols<T1, NN>), dim3(g1), dim3(256), l1, s, im, B, off, m, mn, inter, IP, tw); \
-            hipLaunchKernelGGL((k_prep_xrows<T2, NN>), dim3(g2), dim3(256), l2, s, B, off, m, inter, IP, sl, df, df2, \
-                               cc, scale, tw);                                                                    \
+#define FH_Y(TT, EE, NN, XX)                                                                                      \
+        {                                                                                                         \
+            const auto k = k_prep_ycols<TT, NN, EE, XX>;                                                          \
+            const size_t l = tile_lds(P, TT);                                                                     \
+            hipLaunchKernelGGL(k, dim3(persistent_grid(k, l, (Bt + 2 * TT - 1) / (2 * TT) * m)), dim3(256), l, s, im, \
+                               B, P, off, m, mn, xm, inter, IP, plan, tw);                                        \
         }
-        FH_FIXED_PADS(FH_CF_LAUNCH)
-#undef FH_CF_LAUNCH
+#define FH_X(TT, EE, NN, FF)                                                                                      \
+        {                                                                                                         \
+            const auto k = k_prep_xrows<TT, NN, EE, FF>;                                                          \
+            const size_t l = tile_lds(P, TT);                                                                     \
+            hipLaunchKernelGGL(k, dim3(persistent_grid(k, l, (H + TT) / TT * m)), dim3(256), l, s, Bt, P, offt, m, \
+                               inter, IP, sl, df, df2, cc, scale, plan, tw);                                      \
+        }
+#define FH_Y_PLAIN(TT, EE) FH_Y(TT, EE, 0, false)
+#define FH_Y_XF(TT, EE) FH_Y(TT, EE, 0, true)
+#define FH_X_PLAIN(TT, EE) FH_X(TT, EE, 0, false)
+#define FH_X_FLIP(TT, EE) FH_X(TT, EE, 0, true)
+#define FH_FIXED(NN)                                                        \
+        if (!xf && !flip_back && P == NN) {                                 \
+            FH_Y(8, 0, NN, false)                                           \
+            FH_X(4, 0, NN, false)                                           \
+        } else
+        FIXED_PADS(FH_FIXED)
+        {
+            if (xf) FH_COL_CLASS(P, FH_Y_XF);
+            else FH_COL_CLASS(P, FH_Y_PLAIN);
+            if (flip_back) FH_ROW_CLASS(P, FH_X_FLIP);
+            else FH_ROW_CLASS(P, FH_X_PLAIN);
+        }
+#undef FH_FIXED
+#undef FH_Y_PLAIN
+#undef FH_Y_XF
+#undef FH_X_PLAIN
+#undef FH_X_FLIP
+#undef FH_Y
+#undef FH_X
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+// The whole prep of n particles into their slices.
+hipError_t launch_prep2d(const float *imgs, int n, int B, int P, const float *means, float2 *slices,
+                         float2 *inter, int inter_n, const float *defocus, const float *defocus2, CtfConst cc,
+                         float scale, const FftPlan &plan, const float2 *tw, hipStream_t s)
+{
+    return prep2d_passes(imgs, n, B, P, means, nullptr, false, slices, inter, inter_n, defocus, defocus2, cc, scale,
+                         plan, tw, s);
+}
+
+// The prep of n particles (box B, edge means or null) resampled by the
+// inverse 2-D transforms xf (6 floats each), without a flip.
+hipError_t launch_prep2d_xform(const float *imgs, int n, int B, int P, const float *means, const float *xf,
+                               float2 *slices, float2 *inter, int inter_n, float scale, const FftPlan &plan,
+                               const float2 *tw, hipStream_t s)
+{
+    return prep2d_passes(imgs, n, B, P, means, xf, false, slices, inter, inter_n, nullptr, nullptr, CtfConst{}, scale,
+                         plan, tw, s);
+}
+
+// The padded particles flipped in Fourier space and back in real space: P x P
+// images, phase origin at the centre, times scale.  work: n slices of memory.
+hipError_t launch_flip2d(const float *imgs, int n, int B, int P, const float *means, float2 *work, float2 *inter,
+                         int inter_n, const float *defocus, const float *defocus2, CtfConst cc, float scale,
+                         float *out, const FftPlan &plan, const float2 *tw, hipStream_t s)
+{
+    if (n <= 0) return hipSuccess;
+    hipError_t e = prep2d_passes(imgs, n, B, P, means, nullptr, true, work, inter, inter_n, defocus, defocus2, cc, 1.0f,
+                                 plan, tw, s);
+    if (e != hipSuccess) return e;
+#define FH_CALL(TT, EE)                                                                                           \
+    {                                                                                                             \
+        const auto k = k_flip_ycols<TT, EE>;                                                                      \
+        const size_t l = tile_lds(P, TT);                                                                         \
+        hipLaunchKernelGGL(k, dim3(persistent_grid(k, l, (P + 2 * TT - 1) / (2 * TT) * n)), dim3(256), l, s, work, P, \
+                           n, out, scale, plan, tw);                                                              \
+    }
+    FH_COL_CLASS(P, FH_CALL);
+#undef FH_CALL
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------- normalise
@@ -683,64 +620,85 @@ hipError_t launch_normalize(float2 *data, float *norm, int P, int sqrtnorm, floa
 }
 
 // ---------------------------------------------------------------- 3-D inverse
-// In-place inverse complex transform of length P along z (pass 0) or y
-// (pass 1) for tiles of T consecutive x; inverse = conj o forward o conj.
+// Bound by memory: 0.46 GB per pass at 384^3 in 0.13 ms (3.5 TB/s); by blocks
+// of one tile each, whose reads nothing covers, 0.31 along an axis and 0.27 to
+// real rows.
+// In-place inverse complex transform of length P along one axis (stride
+// axis_stride) for tiles of T consecutive x; inverse = conj o forward o conj.
 // FWD: the forward transform instead (no conjugation), each output n times
 // (-1)^n: the axis's phase origin moved to the corner
-template <int T, int FWD = 0>
-__global__ void __launch_bounds__(256) k_fft_axis_inv(float2 *__restrict__ data, int P, size_t axis_stride,
-                                                      size_t outer_stride, FftPlan plan,
-                                                      const float2 *__restrict__ twg)
+template <int T, int E, int FWD>
+__global__ void __launch_bounds__(256, tile_waves(0, E))
+    k_fft_axis(float2 *__restrict__ data, int P, size_t axis_stride, size_t outer_stride, int outer, FftPlan plan,
+               const float2 *__restrict__ twg)
 {
     extern __shared__ float2 smem[];
     float2 *tw = smem;
     float2 *A = tw + P;
-    float2 *Bf = A + T * P;
-    const int H = P / 2;
-    const int x0 = blockIdx.x * T;
-    float2 *base = data + (size_t)blockIdx.y * outer_stride;
+    const int H = P / 2, ng = (H + T) / T;
     load_twiddles(tw, twg, P);
-    for (int idx = threadIdx.x; idx < T * P; idx += blockDim.x) {
-        const int n = idx / T;
-        const int t = idx - n * T;
-        const int x = x0 + t;
-        float2 v = make_float2(0.f, 0.f);
-        if (x <= H) v = FWD ? base[(size_t)n * axis_stride + x] : conjf2(base[(size_t)n * axis_stride + x]);
-        A[n * T + t] = v;
-    }
-    __syncthreads();
-    float2 *R = fft_tile<T>(A, Bf, plan, tw);
-    for (int idx = threadIdx.x; idx < T * P; idx += blockDim.x) {
-        const int n = idx / T;
-        const int t = idx - n * T;
-        const int x = x0 + t;
-        if (x <= H) {
-            const float2 r = R[n * T + t];
-            base[(size_t)n * axis_stride + x] = FWD ? ((n & 1) ? make_float2(-r.x, -r.y) : r) : conjf2(r);
+    TileWalk w(ng * outer);
+    float2 v[E];
+    auto fetch = [&](int tile) {
+        const int tid = opaque_tid();
+        const int o = tile / ng, x0 = (tile - o * ng) * T;
+        const float2 *base = data + (size_t)o * outer_stride;
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int idx = tid + 256 * e;
+            const int x = x0 + idx % T, j = idx / T;
+            v[e] = j < P && x <= H ? base[(size_t)j * axis_stride + x] : make_float2(0.f, 0.f);
         }
+    };
+    if (w.t < w.end) fetch(w.t);
+    for (; w.t < w.end; w.t += w.step) {
+        const int tid = opaque_tid();
+        const int o = w.t / ng, x0 = (w.t - o * ng) * T;
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int idx = tid + 256 * e;
+            if (idx < T * P) A[idx] = FWD ? v[e] : conjf2(v[e]);
+        }
+        __syncthreads();
+        if (w.t + w.step < w.end) fetch(w.t + w.step);
+        fft_lds_inplace<T, E>(A, plan, tw);
+        float2 *base = data + (size_t)o * outer_stride;
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int idx = tid + 256 * e;
+            const int x = x0 + idx % T, j = idx / T;
+            if (j < P && x <= H) {
+                const float2 r = A[idx];
+                base[(size_t)j * axis_stride + x] = FWD ? ((j & 1) ? make_float2(-r.x, -r.y) : r) : conjf2(r);
+            }
+        }
+        __syncthreads();  // the tile is read before the next one is stored
     }
+}
+
+template <int FWD>
+static hipError_t fft_axis(float2 *data, int P, size_t axis_stride, size_t outer_stride, int outer,
+                           const FftPlan &plan, const float2 *tw, hipStream_t s)
+{
+    const int H = P / 2;
+#define FH_CALL(TT, EE)                                                                                           \
+    {                                                                                                             \
+        const auto k = k_fft_axis<TT, EE, FWD>;                                                                   \
+        const size_t l = tile_lds(P, TT);                                                                         \
+        hipLaunchKernelGGL(k, dim3(persistent_grid(k, l, (H + TT) / TT * outer)), dim3(256), l, s, data, P,       \
+                           axis_stride, outer_stride, outer, plan, tw);                                           \
+    }
+    FH_COL_CLASS(P, FH_CALL);
+#undef FH_CALL
+    return hipGetLastError();
 }
 
 hipError_t launch_fft3d_inverse_zy(float2 *data, int P, const FftPlan &plan, const float2 *tw, hipStream_t s)
 {
-    const int H = P / 2;
-    const int T = pick_T(P);
-    const size_t lds = fft_lds_bytes(P, T);
-    const size_t row = H + 1;
-    dim3 grid((H + 1 + T - 1) / T, P);
-    // z pass: tiles at fixed y
-    if (T == 8)
-        hipLaunchKernelGGL(k_fft_axis_inv<8>, grid, dim3(256), lds, s, data, P, (size_t)P * row, row, plan, tw);
-    else
-        hipLaunchKernelGGL(k_fft_axis_inv<4>, grid, dim3(256), lds, s, data, P, (size_t)P * row, row, plan, tw);
-    hipError_t e = hipGetLastError();
+    const size_t row = P / 2 + 1, plane = (size_t)P * row;
+    hipError_t e = fft_axis<0>(data, P, plane, row, P, plan, tw, s);  // along z, at fixed y
     if (e != hipSuccess) return e;
-    // y pass: tiles at fixed z
-    if (T == 8)
-        hipLaunchKernelGGL(k_fft_axis_inv<8>, grid, dim3(256), lds, s, data, P, row, (size_t)P * row, plan, tw);
-    else
-        hipLaunchKernelGGL(k_fft_axis_inv<4>, grid, dim3(256), lds, s, data, P, row, (size_t)P * row, plan, tw);
-    return hipGetLastError();
+    return fft_axis<0>(data, P, row, plane, P, plan, tw, s);  // along y, at fixed z
 }
 
 // c2r along x for row pairs, x 1/P^3 (do_ift_inplace, emdata_transform.cpp:392-425),
@@ -748,69 +706,78 @@ hipError_t launch_fft3d_inverse_zy(float2 *data, int P, const FftPlan &plan, con
 // nz planes of P rows; shift 1: fftshift of the written volume (3-D finish),
 // shift 2: fftshift of each plane (a batch of 2-D images), 0: rows written
 // in place (2-D projection).
-template <int T>
-__global__ void __launch_bounds__(256) k_c2r_x(const float2 *__restrict__ data, int P, int nz, int shift,
-                                               float *__restrict__ out, float scale, FftPlan plan,
-                                               const float2 *__restrict__ twg)
+template <int T, int E>
+__global__ void __launch_bounds__(256, tile_waves(0, E))
+    k_c2r_x(const float2 *__restrict__ data, int P, int nz, int shift, float *__restrict__ out, float scale,
+            FftPlan plan, const float2 *__restrict__ twg)
 {
+    constexpr int EH = E / 2 + 1;
     extern __shared__ float2 smem[];
     float2 *tw = smem;
     float2 *A = tw + P;
-    float2 *Bf = A + T * P;
     const int H = P / 2;
-    const size_t nrows = (size_t)nz * P;
-    const size_t row0 = (size_t)blockIdx.x * 2 * T;
+    const size_t nrows = (size_t)nz * P;  // even: P is
     load_twiddles(tw, twg, P);
-    for (int idx = threadIdx.x; idx < T * P; idx += blockDim.x) {
-        const int t = idx / P;
-        const int k = idx - t * P;
-        const size_t ra = row0 + 2 * t, rc = ra + 1;
-        float2 a = make_float2(0.f, 0.f), c = make_float2(0.f, 0.f);
-        if (ra < nrows) {
-            a = k <= H ? data[ra * (H + 1) + k] : conjf2(data[ra * (H + 1) + (P - k)]);
-            if (k == 0 || k == H) a.y = 0.f;
-        }
-        if (rc < nrows) {
-            c = k <= H ? data[rc * (H + 1) + k] : conjf2(data[rc * (H + 1) + (P - k)]);
-            if (k == 0 || k == H) c.y = 0.f;
-        }
-        // Z = A + iC, inverse via conj o forward o conj
-        A[k * T + t] = make_float2(a.x - c.y, -(a.y + c.x));
-    }
-    __syncthreads();
-    float2 *R = fft_tile<T>(A, Bf, plan, tw);
-    for (int idx = threadIdx.x; idx < T * P; idx += blockDim.x) {
-        const int t = idx / P;
-        const int x = idx - t * P;
-        const size_t ra = row0 + 2 * t;
-        const float2 z = conjf2(R[x * T + t]);
-        const int xc = x + H < P ? x + H : x + H - P;
-        for (int q = 0; q < 2; q++) {
-            const size_t r = ra + q;
-            if (r >= nrows) break;
-            if (!shift) {
-                out[r * P + x] = (q == 0 ? z.x : z.y) * scale;
-                continue;
+    TileWalk w((int)((nrows + 2 * T - 1) / (2 * T)));
+    float4 v[EH];
+    auto fetch = [&](int tile) {
+        const int tid = opaque_tid();
+#pragma unroll
+        for (int e = 0; e < EH; e++) {
+            const int idx = tid + 256 * e;
+            const size_t r = (size_t)tile * 2 * T + 2 * (idx % T);
+            const int k = idx / T;
+            v[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (k <= H && r < nrows) {
+                const float2 a = data[r * (H + 1) + k], c = data[(r + 1) * (H + 1) + k];
+                v[e] = make_float4(a.x, a.y, c.x, c.y);
             }
-            const int y = (int)(r % P), zz = (int)(r / P);
-            const int yc = y + H < P ? y + H : y + H - P;
-            const int zc = shift == 2 ? zz : (zz + H < P ? zz + H : zz + H - P);
-            out[((size_t)zc * P + yc) * P + xc] = (q == 0 ? z.x : z.y) * scale;
         }
+    };
+    if (w.t < w.end) fetch(w.t);
+    for (; w.t < w.end; w.t += w.step) {
+        const int tid = opaque_tid();
+#pragma unroll
+        for (int e = 0; e < EH; e++) {
+            const int idx = tid + 256 * e;
+            if (idx / T <= H) store_pair<T>(A, idx / T, idx % T, P, v[e]);
+        }
+        __syncthreads();
+        if (w.t + w.step < w.end) fetch(w.t + w.step);
+        fft_lds_inplace<T, E>(A, plan, tw);
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int idx = tid + 256 * e;
+            const size_t r = (size_t)w.t * 2 * T + 2 * (idx % T);
+            const int x = idx / T;
+            if (x >= P || r >= nrows) continue;
+            const float2 z = A[idx];
+            const int xc = !shift ? x : x + H < P ? x + H : x + H - P;
+            const int zz = (int)(r / P), y = (int)(r - (size_t)zz * P);
+            const int zc = shift != 1 ? zz : zz + H < P ? zz + H : zz + H - P;
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const int yq = y + q, yc = !shift ? yq : yq + H < P ? yq + H : yq + H - P;
+                out[((size_t)zc * P + yc) * P + xc] = (q == 0 ? z.x : -z.y) * scale;
+            }
+        }
+        __syncthreads();  // the tile is read before the next one is stored
     }
 }
 
 static hipError_t c2r_rows(const float2 *data, int P, int nz, int shift, float *out, float scale,
                            const FftPlan &plan, const float2 *tw, hipStream_t s)
 {
-    const int T = pick_T(P);
-    const size_t lds = fft_lds_bytes(P, T);
-    const size_t nrows = (size_t)nz * P;
-    dim3 grid((unsigned)((nrows + 2 * T - 1) / (2 * T)));
-    if (T == 8)
-        hipLaunchKernelGGL(k_c2r_x<8>, grid, dim3(256), lds, s, data, P, nz, shift, out, scale, plan, tw);
-    else
-        hipLaunchKernelGGL(k_c2r_x<4>, grid, dim3(256), lds, s, data, P, nz, shift, out, scale, plan, tw);
+    const int nrows = nz * P;
+#define FH_CALL(TT, EE)                                                                                           \
+    {                                                                                                             \
+        const auto k = k_c2r_x<TT, EE>;                                                                           \
+        const size_t l = tile_lds(P, TT);                                                                         \
+        hipLaunchKernelGGL(k, dim3(persistent_grid(k, l, (nrows + 2 * TT - 1) / (2 * TT))), dim3(256), l, s, data, P, \
+                           nz, shift, out, scale, plan, tw);                                                      \
+    }
+    FH_ROW_CLASS(P, FH_CALL);
+#undef FH_CALL
     return hipGetLastError();
 }
 
@@ -824,64 +791,37 @@ hipError_t launch_c2r_x(const float2 *data, int P, float *out, float scale, cons
 // inverse FFT along y of the P/2+1 columns, c2r along x, x 1/P^2.
 hipError_t launch_ift2d(float2 *data, int P, float *out, const FftPlan &plan, const float2 *tw, hipStream_t s)
 {
-    const int H = P / 2;
-    const int T = pick_T(P);
-    const size_t lds = fft_lds_bytes(P, T);
-    const size_t row = H + 1;
-    dim3 grid((H + 1 + T - 1) / T, 1);
-    if (T == 8)
-        hipLaunchKernelGGL(k_fft_axis_inv<8>, grid, dim3(256), lds, s, data, P, row, (size_t)0, plan, tw);
-    else
-        hipLaunchKernelGGL(k_fft_axis_inv<4>, grid, dim3(256), lds, s, data, P, row, (size_t)0, plan, tw);
-    hipError_t e = hipGetLastError();
+    hipError_t e = fft_axis<0>(data, P, P / 2 + 1, 0, 1, plan, tw, s);
     if (e != hipSuccess) return e;
     return c2r_rows(data, P, 1, 0, out, 1.0f / ((float)P * (float)P), plan, tw, s);
 }
 
 // do_ift of n complex images (P x (P/2+1) each, in place: overwritten) into n
-// real P x P images with scale, phase origin to the centre: the inverse of the
-// row and column passes (the particle's flip back to real space)
+// real P x P images with scale, phase origin to the centre
 hipError_t launch_ift2d_batch(float2 *data, int n, int P, float *out, float scale, const FftPlan &plan,
                               const float2 *tw, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    const int H = P / 2;
-    const int T = pick_T(P);
-    const size_t lds = fft_lds_bytes(P, T);
-    const size_t row = H + 1;
-    dim3 grid((H + 1 + T - 1) / T, n);
-    if (T == 8)
-        hipLaunchKernelGGL(k_fft_axis_inv<8>, grid, dim3(256), lds, s, data, P, row, (size_t)P * row, plan, tw);
-    else
-        hipLaunchKernelGGL(k_fft_axis_inv<4>, grid, dim3(256), lds, s, data, P, row, (size_t)P * row, plan, tw);
-    hipError_t e = hipGetLastError();
+    const size_t row = P / 2 + 1;
+    hipError_t e = fft_axis<0>(data, P, row, (size_t)P * row, n, plan, tw, s);
     if (e != hipSuccess) return e;
     return c2r_rows(data, P, n, 2, out, scale, plan, tw, s);
 }
 
 // ---------------------------------------------------------------- forward 3-D
 // do_fft of a real P^3 volume with the phase origin moved to the corner (the
-// Fourier-space xform.phaseorigin.tocorner, center_origin_fft): the row and
-// column passes of the particle prep over the P z planes (their load index
-// applies the x and y shift), then the z transform, each output times
-// (-1)^z.  vol: P^3 floats, out: P x P x (P/2+1) complex.
-hipError_t launch_fft3d_forward_corner(const float *vol, int P, const float *zeros, float2 *out, const FftPlan &plan,
-                                       const float2 *tw, hipStream_t s)
+// Fourier-space xform.phaseorigin.tocorner, center_origin_fft): the particle
+// prep's passes over the P z planes (their load index applies the x and y
+// shift), then the z transform, each output times (-1)^z.  vol: P^3 floats,
+// out: P x P x (P/2+1) complex.
+hipError_t launch_fft3d_forward_corner(const float *vol, int P, float2 *out, float2 *inter, int inter_n,
+                                       const FftPlan &plan, const float2 *tw, hipStream_t s)
 {
-    hipError_t e = launch_prep_rows(vol, P, P, P, zeros, out, plan, tw, s);
+    hipError_t e = launch_prep2d(vol, P, P, P, nullptr, out, inter, inter_n, nullptr, nullptr, CtfConst{}, 1.0f, plan,
+                                 tw, s);
     if (e != hipSuccess) return e;
-    e = launch_prep_cols(P, P, P, out, nullptr, nullptr, CtfConst{}, 1.0f, plan, tw, s);
-    if (e != hipSuccess) return e;
-    const int H = P / 2;
-    const int T = pick_T(P);
-    const size_t lds = fft_lds_bytes(P, T);
-    const size_t row = H + 1;
-    dim3 grid((H + 1 + T - 1) / T, P);
-    if (T == 8)
-        hipLaunchKernelGGL((k_fft_axis_inv<8, 1>), grid, dim3(256), lds, s, out, P, (size_t)P * row, row, plan, tw);
-    else
-        hipLaunchKernelGGL((k_fft_axis_inv<4, 1>), grid, dim3(256), lds, s, out, P, (size_t)P * row, row, plan, tw);
-    return hipGetLastError();
+    const size_t row = P / 2 + 1;
+    return fft_axis<1>(out, P, (size_t)P * row, row, P, plan, tw, s);
 }
 
 // ---------------------------------------------------------------- task merge
