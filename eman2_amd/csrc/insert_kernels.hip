@@ -19,11 +19,14 @@
 //                    the brick with plain read-modify-writes (lanes sharing
 //                    a stencil origin take turns, elected by an LDS tag).
 //                    Each item writes its partial brick to HBM.
+//  k_reduce_items    the items of a brick summed into its first one, where
+//                    the batch has more than about two per brick.
 //  k_merge_partials  one thread per half-volume voxel sums the partial
 //                    bricks of its unfolded source cells under the Hermitian
 //                    fold of add_complex_at_fast and adds them with plain
 //                    stores (each voxel has one owner: no atomics).
 #pragma clang fp contract(off)
+#include <climits>
 #include "fh_device.hpp"
 
 namespace fh {
@@ -3211,6 +3214,72 @@ hipError_t launch_scatter_wide(const float2 *slices, int nslices, int nsym, cons
 }
 
 // ------------------------------------------------------------ merge of partial bricks
+// Items per brick from which they are summed before the merge reads them: 2
+// where the batch has an item per brick of the grid (bricks outside the
+// sphere of slices, about half, have none), else never.
+__device__ __forceinline__ int reduce_least(const int *__restrict__ item_off, int nbricks)
+{
+    return item_off[3 * nbricks] >= nbricks ? 2 : INT_MAX;
+}
+
+// The items of every such brick summed into its first one's partial brick.
+// A unit is 256 floats of a brick; the units go round the blocks, and the
+// waves of a block share the ones of its turn that have work.  Read in whole
+// runs here, the items cost their bytes; the merge, whose lanes read rows of 9
+// floats out of neighbouring bricks, and one item after the other, took 1.08
+// ms (24,000 slices at pad 384, 2.6 items per brick), 1.19 (112,000 at 288,
+// 11) and 0.11 (2,000 at 96, 6): now 1.02, 0.59 and 0.033, this pass
+// included.  Below an item per brick of the grid nothing is gained (8,000
+// gauss_var slices at pad 384, 0.5: 4.6 ms, and 4.7 with a pass over all).
+__global__ void __launch_bounds__(256) k_reduce_items(float *__restrict__ part, const int *__restrict__ item_off,
+                                                      int nbricks, int pf)
+{
+    __shared__ int q[256][3];  // first item, items, segment
+    __shared__ int nq;
+    const int least = reduce_least(item_off, nbricks);
+    if (least == INT_MAX) return;
+    const int segs = (pf + 255) / 256, lane = threadIdx.x & 63;
+    const long long units = (long long)nbricks * segs;
+    for (long long r = 0; r * 256 * gridDim.x < units; r++) {
+        if (threadIdx.x == 0) nq = 0;
+        __syncthreads();
+        const long long u = (r * 256 + threadIdx.x) * gridDim.x + blockIdx.x;
+        if (u < units) {
+            const int b = (int)(u / segs), i0 = item_off[3 * b], n = item_off[3 * b + 3] - i0;
+            if (n >= least) {
+                const int slot = atomicAdd(&nq, 1);
+                q[slot][0] = i0;
+                q[slot][1] = n;
+                q[slot][2] = (int)(u - (long long)b * segs);
+            }
+        }
+        __syncthreads();
+        const int m = nq;
+        for (int e = threadIdx.x >> 6; e < m; e += 4) {
+            const int n = __builtin_amdgcn_readfirstlane(q[e][1]);
+            const int c0 = 256 * __builtin_amdgcn_readfirstlane(q[e][2]) + lane;
+            float *p = part + (size_t)__builtin_amdgcn_readfirstlane(q[e][0]) * pf;
+            float sum[4] = {0.f, 0.f, 0.f, 0.f};
+            for (int it = 0; it < n; it += 4) {
+                float v[4][4];
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        v[k][j] = it + k < n && c0 + 64 * j < pf ? p[(size_t)(it + k) * pf + c0 + 64 * j] : 0.f;
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) sum[j] += v[k][j];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (c0 + 64 * j < pf) p[c0 + 64 * j] = sum[j];
+        }
+        __syncthreads();  // the queue is read before the next turn fills it
+    }
+}
+
 // Sum over the work items of the bricks whose cells include unfolded cell
 // (i, j, k): brick b covers cells [ow + BS*b, ow + BS*b + HL) per axis (z:
 // BZ, HZ), so a cell lies in the bricks floor(u / BS) down to
@@ -3219,8 +3288,8 @@ hipError_t launch_scatter_wide(const float2 *slices, int nslices, int nsym, cons
 // first, also the previous brick).
 template <int BS, int HL, int BZ, int HZ>
 __device__ __forceinline__ void partial_sum(const float *__restrict__ part, const int *__restrict__ item_off, int nb,
-                                            int nbz, int ow, int pf, int i, int j, int k, float &re, float &im,
-                                            float &w)
+                                            int nbz, int ow, int pf, int least, int i, int j, int k, float &re,
+                                            float &im, float &w)
 {
     constexpr int HC = HL * HL * HZ;
     const int ui = i - ow, uj = j - ow, uk = k - ow;  // >= 0 for cells >= -H
@@ -3233,7 +3302,8 @@ __device__ __forceinline__ void partial_sum(const float *__restrict__ part, cons
             for (int bi = bi1; bi >= bi0; bi--) {
                 const int b = (bk * nb + bj) * nb + bi;
                 const int cc = ((uk - BZ * bk) * HL + (uj - BS * bj)) * HL + (ui - BS * bi);
-                const int i0 = item_off[3 * b], i1 = item_off[3 * b + 3];
+                const int i0 = item_off[3 * b], n = item_off[3 * b + 3] - i0;
+                const int i1 = i0 + (n >= least ? 1 : n);  // summed into the first one
                 for (int it = i0; it < i1; it++) {
                     const float *p = part + (size_t)it * pf + cc;
                     re += p[0];
@@ -3254,6 +3324,7 @@ template <int BS, int HL, int BZ, int HZ>
 __global__ void __launch_bounds__(256) k_merge_partials(const float *__restrict__ part, const int *__restrict__ item_off,
                                                         BrickGeom g, InsertConst c, float2 *data, float *norm)
 {
+    const int least = reduce_least(item_off, g.nb * g.nb * g.nbz);
     const int H = c.H, P = c.P, nb = g.nb, nbz = g.nbz, ow = g.ow, pf = g.part_floats;
     const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (long long)P * P * (H + 1)) return;
@@ -3262,10 +3333,10 @@ __global__ void __launch_bounds__(256) k_merge_partials(const float *__restrict_
     const int ys = (int)(rest % P), zs = (int)(rest / P);
     float r, i, w;
     if (ys == 0 && zs == 0 && (xs == 0 || xs == H)) {
-        partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, xs, 0, 0, r, i, w);
+        partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, least, xs, 0, 0, r, i, w);
         if (xs == H) {
             float r2, i2, w2;
-            partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, -H, 0, 0, r2, i2, w2);
+            partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, least, -H, 0, 0, r2, i2, w2);
             r += r2;
             i += i2;
             w += w2;
@@ -3290,7 +3361,7 @@ __global__ void __launch_bounds__(256) k_merge_partials(const float *__restrict_
     float dre = 0.f, dim = 0.f, dw = 0.f;
     for (int a = 0; a < njd; a++)
         for (int b = 0; b < nkd; b++) {
-            partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, xs, jd[a], kd[b], r, i, w);
+            partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, least, xs, jd[a], kd[b], r, i, w);
             dre += r;
             dim += i;
             dw += w;
@@ -3298,17 +3369,17 @@ __global__ void __launch_bounds__(256) k_merge_partials(const float *__restrict_
     for (int a = 0; a < njn; a++)
         for (int b = 0; b < nkn; b++) {
             if (xs == 0 || xs == H) {
-                partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, xs, jn[a], kn[b], r, i, w);
+                partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, least, xs, jn[a], kn[b], r, i, w);
                 dre += r;
                 dim -= i;
                 if (xs == H) {
-                    partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, -H, jn[a], kn[b], r, i, w);
+                    partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, least, -H, jn[a], kn[b], r, i, w);
                     dre += 2.f * r;
                     dim -= 2.f * i;
                     dw += w;
                 }
             } else {
-                partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, -xs, jn[a], kn[b], r, i, w);
+                partial_sum<BS, HL, BZ, HZ>(part, item_off, nb, nbz, ow, pf, least, -xs, jn[a], kn[b], r, i, w);
                 dre += r;
                 dim -= i;
                 dw += w;
@@ -3326,6 +3397,12 @@ hipError_t launch_merge_partials(BrickGeom g, BinBuffers b, InsertConst c, float
 {
     const long long n = (long long)c.P * c.P * (c.H + 1);
     const dim3 grid((unsigned)((n + 255) / 256));
+    const int nbricks = g.nb * g.nb * g.nbz;
+    const long long units = (long long)nbricks * ((g.part_floats + 255) / 256);
+    hipLaunchKernelGGL(k_reduce_items, dim3((unsigned)std::min(2048LL, (units + 3) / 4)), dim3(256), 0, s, b.part,
+                       b.item_off, nbricks, g.part_floats);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
 #define FH_MERGE(BS, HL, BZ, HZ)                                                                                       \
     if (g.bs == BS && g.halo == HL && g.bsz == BZ && g.haloz == HZ) {                                                  \
         hipLaunchKernelGGL((k_merge_partials<BS, HL, BZ, HZ>), grid, dim3(256), 0, s, b.part, b.item_off, g, c, data,  \
