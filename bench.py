@@ -353,13 +353,13 @@ def main():
     elapsed = time.perf_counter() - t0
     value = a.steps * n / elapsed
 
-    # roofline of the dominant kernel (k_scatter_insert; k_scatter_wide for
-    # the wide stencils): scatter model, one 12-byte (complex + weight) update
+    # roofline of the dominant kernel (k_scatter_insert; k_scatter_gauss6 and
+    # k_scatter_wide for the wide stencils): scatter model, one 12-byte (complex + weight) update
     # per gridding contribution, 8 per pixel per symmetry copy (S^3 for a
     # stencil of S cells per axis)
     wide = {"gauss_var": 6, "gauss_5": 6, "gauss_3": 3, "kaiser_bessel": 5, "gridding_5": 5, "gridding_7": 7,
             "kaiser_bessel_derived": 9}.get(a.mode)
-    kname = "k_scatter_wide" if wide else "k_scatter_insert"
+    kname = "k_scatter_gauss6" if wide == 6 else "k_scatter_wide" if wide else "k_scatter_insert"
     bytes_per_particle = nsym * npix(P) * (wide ** 3 if wide else 8) * 12
     launches = sum(s["chunks"] for s in stats)
     avg_ms = kern_ms / max(1, launches)
@@ -380,9 +380,10 @@ def main():
             "kernel": kname, "avg_launch_ms": round(avg_ms, 3),
             "algorithmic_bytes_per_launch": int(per_launch_bytes)}
     if wide and achieved:
-        # the wide-stencil scatter accumulates in LDS and is VALU-issue bound: its roofline is the
-        # CUs' VALU issue rate (one wave64 instruction per CU per clock) over the VALU wave
-        # instructions per contribution that the PMC run of this shape counted
+        # the 6-cell Gaussians' scatter accumulates in registers and is VALU bound: its roofline is
+        # the CUs' VALU rate (128 FP32 lanes per CU per clock, the published vector peak: two
+        # wave64 instructions) over the VALU wave instructions per contribution that the PMC run
+        # of this shape counted
         contrib = nsym * npix(P) * wide ** 3 * (a.steps * n) / max(1, launches)
         gcs = contrib / (avg_ms * 1e-3) / 1e9
         peak = None
@@ -392,7 +393,7 @@ def main():
                 t = json.load(f)
             if t.get("P") == P and t.get("sym") == a.sym and t.get("box") == B and t.get("mode") == a.mode:
                 cus = torch.cuda.get_device_properties(0).multi_processor_count
-                peak = cus * ENGINE_CLOCK_HZ / t["valu_insts_per_contribution"] / 1e9
+                peak = 2 * cus * ENGINE_CLOCK_HZ / t["valu_insts_per_contribution"] / 1e9
         roof = {"bound": "valu", "achieved": round(gcs, 1), "peak": round(peak, 1) if peak else None,
                 "unit": "G contributions/s", "frac": round(gcs / peak, 4) if peak else None, "traffic": None,
                 "kernel": kname, "avg_launch_ms": round(avg_ms, 3), "contributions_per_launch": int(contrib),

@@ -1122,7 +1122,8 @@ __device__ __forceinline__ unsigned pack_index(unsigned x, unsigned y, unsigned 
 // double sums per particle accumulated with float64 atomics into acc[p][8].
 // vol: the volume as float4 (re, im, weight, 0) per voxel, or null, then data
 // and norm are read.  n3: the low-resolution band is 9 < x^2 + y^2 < n3.
-// Bound: VALU issue (92 % at pad 600), then the volume's cache lines.  8,000
+// Bound: VALU (0.24 instructions per SIMD and clock at pad 600), then the
+// volume's cache lines.  8,000
 // slices at pad 600: 36.5 ms before, 23.8 now.  What it took: the voxels read
 // before the patch is staged and at most 80 registers (3 workgroups of 8 waves
 // per CU; 34 ms with 2), the packed volume in 2^3 cubes (0.60 G instead of
@@ -2734,14 +2735,15 @@ __global__ void __launch_bounds__(256) k_scatter_wide(const float2 *__restrict__
 // the sums are three FMAs into fixed registers (one copy of the passes per
 // z offset of the origin).
 //
-// Bound: VALU issue (a wave64 FP32 instruction holds a SIMD for 4 cycles), 50
-// instructions per pixel in the passes that stay within the table.  The form
+// Bound: VALU, 0.35 instructions per SIMD and clock (0.70 of the published
+// vector rate), 50 per pixel in the passes that stay within the table, 70 in
+// all; the LDS is busy 83 % of the cycles with table reads and records.  The form
 // before kept the cells in LDS (54 lanes per pass, 4 passes, 6 LDS operations
 // and 28 VALU instructions each; an 8 x 8 window of candidate pixels tested
 // per slice): 142 VALU instructions per pixel, 116 ms for 8,000 x pad 384
 // gauss_var, now 41 ms; for 2,000 x pad 160 of fourier_iter with a reference
 // (its cells read from memory for every term before, kept in the lanes'
-// registers now) 37.3 ms, now 4.6 ms.  Taking the pixels' values by readlane
+// registers now) 37.3 ms, now 3.3 ms.  Taking the pixels' values by readlane
 // instead of through LDS: 68 ms.  At 4 waves per SIMD, without spills: 43.5.
 // The table index floor(f 50 + 1/2), f = r^2 h, which the reference takes in
 // double, is one FMA rounded toward zero with 2^21 + 1/2 added: the sum's low
