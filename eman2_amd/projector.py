@@ -5,8 +5,9 @@ libEM/projector.cpp:69-295), as e2make3dpar.py:716-721 calls it:
 
     pj = Projectors.get("gauss_fft", {"transform": xf, "returnfft": 1}).project3d(ref_map)
 
-Modes 0 (trilinear, the default), 1 (nearest) and 2 (Gaussian).  The map's
-transform is computed once per volume on the GPU and kept there, so
+Modes 0 (trilinear, the default), 1 (nearest) and 2 (Gaussian).  Each call
+uploads its map and transforms it on the GPU, as project3d transforms its
+image, so a map changed between calls is projected as it is then;
 ``project_batch(volume, xforms)`` makes many projections of one map in one
 call.  There is no CPU path.
 """
@@ -25,7 +26,6 @@ class GaussFFTProjector:
     def __init__(self, params=None):
         self.params = {}
         self._ctx = None          # a fourier_hip handle of the volume's size: the GPU context
-        self._vol_key = None
         self.set_params(params or {})
 
     def set_params(self, params):
@@ -43,12 +43,7 @@ class GaussFFTProjector:
             raise _lib.FourierHipError(3, "gauss_fft projects an even cubic real volume")
         if self._ctx is None or self._ctx.P != P:
             self._ctx = FourierHipReconstructor({"size": (P, P, P), "device": int(self.params.get("device", 0))})
-            self._vol_key = None
-        key = (vol.__array_interface__["data"][0], vol.shape, float(vol.ravel()[::max(1, vol.size // 64)].sum()))
-        if key != self._vol_key:
-            self._ctx._check(self._ctx._lib.fh_gauss_fft_volume(self._ctx._need(),
-                                                                 vol.ctypes.data_as(ctypes.c_void_p)))
-            self._vol_key = key
+        self._ctx._check(self._ctx._lib.fh_gauss_fft_volume(self._ctx._need(), vol.ctypes.data_as(ctypes.c_void_p)))
         return self._ctx
 
     def project_batch(self, volume, xforms, mode=None, returnfft=None):
