@@ -1321,9 +1321,15 @@ __global__ void __launch_bounds__(AgreeTile<SYM ? 16 : 32>::THREADS) __attribute
         }
         const float vr = a.vr, vi = x0 < 0 ? -a.vi : a.vi, nv = a.nv;  // get_complex_at conjugate for x<0
         if (a.now && nv != 0.f) {
-            // value v over weight nv against d: dot and powers weighted by nv, nv cancelled once
+            // value v over weight nv against d: dot and powers weighted by nv, nv cancelled once.  |v|^2 / nv with
+            // nv = m 2^e, m in [1/2, 1): the exponent goes to one factor before the product (squares of v leave
+            // the float range for weights from about 1e19 on and below 1e-19), 1 / m by a Newton step.
             const float dotv = vr * a.d.x + vi * a.d.y;
-            const float pw = __fdiv_rn(vr * vr + vi * vi, nv);
+            const int e = __builtin_amdgcn_frexp_expf(nv);
+            const float mn = __builtin_amdgcn_frexp_mantf(nv);
+            float rm = __builtin_amdgcn_rcpf(mn);
+            rm = __builtin_fmaf(__builtin_fmaf(-mn, rm, 1.0f), rm, rm);
+            const float pw = __builtin_fmaf(vr, ldexpf(vr, -e), vi * ldexpf(vi, -e)) * rm;
             const float pw2 = (a.d.x * a.d.x + a.d.y * a.d.y) * nv;
             if (r2d > 9 && r2d < n3) {  // 3 < hypot_fast(x, y) < rmax
                 acc[4] += dotv;
