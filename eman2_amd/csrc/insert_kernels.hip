@@ -1001,7 +1001,8 @@ __device__ __forceinline__ void gather_some_offsets(const AgreePx *px, int list,
                            (double)weight);
         }
     }
-    // each term as the insertion adds it, so that a voxel only this particle reached cancels to 0
+    // each term as the insertion adds it, so that a voxel that only this particle reached, through one or two
+    // terms, cancels to 0 (the order of more than two is not the insertion's)
 #pragma unroll
     for (int k = 0; k < N; k++) {
         const float gg = ((unsigned)(kc - q[k].key) & ~AP_DIGITS) == 0u ? g[k] : 0.f;
@@ -1130,11 +1131,14 @@ __device__ __forceinline__ unsigned pack_index(unsigned x, unsigned y, unsigned 
 // 0.92 G line misses; data and weights read apart: 33.4 ms), offsets in groups
 // of four so that their LDS reads overlap, 32 x 32 tiles (halo 1.27 instead of
 // 1.41).  1,500 particles of d2 at pad 192: 7.1 -> 5.6 ms, the other planes'
-// gather by full waves (with the volume as it is 5.7).
+// gather by full waves (with the volume as it is 5.7).  The whole call 5.8 ms
+// with their sums in double; 5.9 with float atomics, whose order showed in the
+// results; 7.6 plane by plane without atomics, the waves half empty (300
+// particles of d7: 7.0, 7.7 and 13.6).
 template <int MODE, bool SYM, bool PACKED>
 __global__ void __launch_bounds__(AgreeTile<SYM ? 16 : 32>::THREADS) __attribute__((amdgpu_waves_per_eu(SYM ? 5 : 6)))
     k_agree_batch(const float2 *__restrict__ slices, int nsym, const float *__restrict__ t3d, const float *__restrict__ wq,
-                  InsertConst c, int n3, int sub, const float2 *__restrict__ data, const float *__restrict__ norm,
+                  InsertConst c, int n3, int sub, int qcap, const float2 *__restrict__ data, const float *__restrict__ norm,
                   const float4 *__restrict__ vol, const float *__restrict__ exptab, const float *__restrict__ rtab_g,
                   double *__restrict__ acc_out)
 {
@@ -1149,25 +1153,26 @@ __global__ void __launch_bounds__(AgreeTile<SYM ? 16 : 32>::THREADS) __attribute
     const float *t3dp = t3d + 9 * (size_t)p * nsym;
     const float *m = t3d + 9 * (size_t)q;
     const float weight = wq[q];
-    // dynamic LDS, from address 0: fast_exp table, patch, mirror patch, queued compare pixels, near planes;
-    // with symmetry each wave's queue and sums of the other planes
+    // dynamic LDS, from address 0: fast_exp table, patch, mirror patch; with symmetry the near planes; counters;
+    // with symmetry the sums of the other planes, fl(i/P), the pixels' cells (keys) and the other planes' queue
+    // of qcap entries; the queued compare pixels
     extern __shared__ float4 agree_lds[];
     float *etab = reinterpret_cast<float *>(agree_lds);
     AgreePx *ppx = reinterpret_cast<AgreePx *>(etab + EXPN);
     AgreePx *mpx = ppx + AT::PATCH;
-    unsigned long long *near_ops = reinterpret_cast<unsigned long long *>(mpx + AT::MPATCH);  // 64 words
-    int *dn = reinterpret_cast<int *>(near_ops + 64);
-    unsigned short *dq = reinterpret_cast<unsigned short *>(dn + 2);  // AT_X * AY queued compare pixels (tile index)
-    // with symmetry: fl(i/P), the pixels' cells (keys), the sums and the queue of the other planes
-    constexpr int NPX = AT_X * AY, QUEUE = 3 * NPX;
-    float *rtab_l = reinterpret_cast<float *>(dq + NPX);
-    int *cell = reinterpret_cast<int *>(rtab_l + P + 2);
-    float *osum = reinterpret_cast<float *>(cell + NPX);
-    int *queue = reinterpret_cast<int *>(osum + 3 * NPX);
+    unsigned long long *near_ops = reinterpret_cast<unsigned long long *>(mpx + AT::MPATCH);  // a bit per plane
+    const int nwords = (nsym + 63) / 64;  // symmetries of more than 4096 operators take every plane
+    int *dn = reinterpret_cast<int *>(near_ops + (SYM ? min(nwords, 64) : 0));
+    constexpr int NPX = AT_X * AY;
+    double *osum = reinterpret_cast<double *>(dn + 4);
+    float *rtab_l = reinterpret_cast<float *>(osum + (SYM ? 3 * NPX : 0));
+    int *cell = reinterpret_cast<int *>(rtab_l + (SYM ? P + 2 : 0));
+    unsigned short *queue = reinterpret_cast<unsigned short *>(cell + (SYM ? NPX : 0));
+    unsigned short *dq = queue;  // at most NPX compare pixels (tile index), after the other planes are through
     const float *rtab = SYM ? rtab_l : rtab_g;
     if (SYM) {
         for (int i = threadIdx.x; i < P + 2; i += AT::THREADS) rtab_l[i] = rtab_g[i];
-        for (int i = threadIdx.x; i < 3 * NPX; i += AT::THREADS) osum[i] = 0.f;
+        for (int i = threadIdx.x; i < 3 * NPX; i += AT::THREADS) osum[i] = 0.0;
     }
     for (int i = threadIdx.x; i < EXPN; i += AT::THREADS) etab[i] = exptab[i];
     AgreePatch pt{ppx, tx0 - AT_HALO, ty0 - AT_HALO, AT::PY};
@@ -1202,7 +1207,6 @@ __global__ void __launch_bounds__(AgreeTile<SYM ? 16 : 32>::THREADS) __attribute
     // the other symmetry planes that pass within reach of the tile's nearest cells: |n . p| <= sqrt(3)
     // (gather_cell's bound) + sqrt(3) / 2
     const int lane = threadIdx.x & 63;
-    const int nwords = (nsym + 63) / 64;  // symmetries of more than 4096 operators take every plane
     if (SYM && fastkeys && nwords <= 64) {
         for (int wd = threadIdx.x >> 6; wd < nwords; wd += AT::WAVES) {
             const int sop = 64 * wd + lane;
@@ -1309,9 +1313,9 @@ __global__ void __launch_bounds__(AgreeTile<SYM ? 16 : 32>::THREADS) __attribute
                 oim = i - i2;
                 ow = x0 == 0 ? w : w + w2;
                 if (SYM && reach) {
-                    ore += osum[a.l];
-                    oim += osum[NPX + a.l];
-                    ow += osum[2 * NPX + a.l];
+                    ore += (float)osum[a.l];
+                    oim += (float)osum[NPX + a.l];
+                    ow += (float)osum[2 * NPX + a.l];
                 }
                 oim = x0 >= 0 ? oim : -oim;
             }
@@ -1378,25 +1382,27 @@ __global__ void __launch_bounds__(AgreeTile<SYM ? 16 : 32>::THREADS) __attribute
             stage(e % AT_MX - 4, my0 + e / AT_MX, mpx[e]);
     __syncthreads();
     if (SYM && fastkeys && inner) {
-        // The other planes' contributions to the pixels' nearest cells and their mirrors: the (pixel, plane,
-        // sign) triples whose cell lies within the plane's reach are queued, so that full waves run the
-        // gather for the few pixels along the planes' intersections, and summed per pixel: value of the
-        // cell minus the conjugate of its mirror's, weights (the mirror's not on x0 = 0).  What the queue
-        // does not hold is gathered at once.
-        auto gather = [&](int e) {
-            const int l = e & (NPX - 1), kc = cell[l], is = e >> 10 & 1 ? -1 : 1;
-            const int x0 = (kc & 1023) - 512, y0 = (kc >> 10 & 1023) - 512, z0 = (kc >> 20) - 512;
-            float a = 0.f, b = 0.f, g = 0.f;
-            gather_cell(S, t3dp + 9 * (e >> 11), is * x0, is * y0, is * z0, c, weight, etab, rtab, a, b, g);
-            if (a != 0.f || b != 0.f || g != 0.f) {
-                atomicAdd(&osum[l], a);
-                atomicAdd(&osum[NPX + l], is < 0 ? -b : b);
-                if (is > 0 || x0 != 0) atomicAdd(&osum[2 * NPX + l], g);
-            }
-        };
+        // The other planes' contributions to the pixels' nearest cells and their mirrors, 64 planes at a time:
+        // the (pixel, sign, plane) triples whose cell lies within the plane's reach are queued, so that full
+        // waves run the gather for the few pixels along the planes' intersections, and summed per pixel: value
+        // of the cell minus the conjugate of its mirror's, weights (the mirror's not on x0 = 0).  What the queue
+        // does not hold is gathered at once.  The lanes come to a pixel in any order: summed in double and
+        // rounded to float once, the sum does not show it (two terms give their float sum).
         for (int wd = 0; wd < nwords; wd++) {
+            int *count = dn + 1 + (wd & 1);  // the other one is cleared before the barrier
+            auto gather = [&](int e) {
+                const int l = e & (NPX - 1), kc = cell[l], is = e >> 9 & 1 ? -1 : 1;
+                const int x0 = (kc & 1023) - 512, y0 = (kc >> 10 & 1023) - 512, z0 = (kc >> 20) - 512;
+                float a = 0.f, b = 0.f, g = 0.f;
+                gather_cell(S, t3dp + 9 * (64 * wd + (e >> 10)), is * x0, is * y0, is * z0, c, weight, etab, rtab, a, b, g);
+                if (a != 0.f || b != 0.f || g != 0.f) {
+                    atomicAdd(&osum[l], (double)a);
+                    atomicAdd(&osum[NPX + l], (double)(is < 0 ? -b : b));
+                    if (is > 0 || x0 != 0) atomicAdd(&osum[2 * NPX + l], (double)g);
+                }
+            };
             for (unsigned long long ops = nwords <= 64 ? near_ops[wd] : ~0ull; ops; ops &= ops - 1) {
-                const int sop = 64 * wd + __builtin_ctzll(ops);
+                const int k = __builtin_ctzll(ops), sop = 64 * wd + k;
                 if (sop >= nsym) break;
                 if (sop == own) continue;
                 const float *o = t3dp + 9 * sop;
@@ -1413,21 +1419,22 @@ __global__ void __launch_bounds__(AgreeTile<SYM ? 16 : 32>::THREADS) __attribute
                         const unsigned long long hm = __ballot(hit);
                         if (!hm) continue;
                         int base = 0;
-                        if (lane == 0) base = atomicAdd(&dn[1], __popcll(hm));
+                        if (lane == 0) base = atomicAdd(count, __popcll(hm));
                         base = __builtin_amdgcn_readfirstlane(base) + __popcll(hm & ((1ull << lane) - 1ull));
                         if (hit) {
-                            const int e = a.l | sgn << 10 | sop << 11;
-                            if (base < QUEUE) queue[base] = e;
+                            const int e = a.l | sgn << 9 | k << 10;
+                            if (base < qcap) queue[base] = (unsigned short)e;
                             else gather(e);
                         }
                     }
                 }
             }
+            if (threadIdx.x == 0) dn[1 + ((wd + 1) & 1)] = 0;
+            __syncthreads();
+            const int n = min(*count, qcap);
+            for (int k = threadIdx.x; k < n; k += AT::THREADS) gather(queue[k]);
+            __syncthreads();
         }
-        __syncthreads();
-        const int n = min(dn[1], QUEUE);
-        for (int k = threadIdx.x; k < n; k += AT::THREADS) gather(queue[k]);
-        __syncthreads();
     }
 #pragma unroll
     for (int it = 0; it < NP; it++) {
@@ -1499,12 +1506,18 @@ hipError_t launch_agree_batch(const float2 *slices, int nsym, const float *t3d, 
     const int AY = sym ? 16 : 32;
     const int ntx = (c.P / 2 + 2 + AT_X - 1) / AT_X, nty = (c.P + AY - 1) / AY;
     const size_t patch = sym ? AgreeTile<16>::PATCH + AgreeTile<16>::MPATCH : AgreeTile<32>::PATCH + AgreeTile<32>::MPATCH;
-    const size_t lds = sizeof(float) * EXPN + sizeof(AgreePx) * patch + 8 * 64 + 8 + sizeof(short) * AT_X * AY +
-                       (sym ? sizeof(float) * (c.P + 2 + (1 + 3 + 3) * AT_X * AY) : 0);
+    // With symmetry the other planes' queue takes what four workgroups per CU leave: 1,792 entries at pad 192, 976
+    // at 600, the fewest (the compare pixels share it) from about pad 830 on.  Three workgroups: 7.2 ms instead of
+    // 5.8 for 1,500 particles of d2 at pad 192.
+    const int npx = AT_X * AY;
+    const size_t fixed = sizeof(float) * EXPN + sizeof(AgreePx) * patch + 16 +
+                         (sym ? 8 * std::min((nsym + 63) / 64, 64) + sizeof(float) * (c.P + 2) + (4 + 3 * 8) * npx : 0);
+    const int qcap = sym ? (int)std::max<long long>(npx, ((40 << 10) - (long long)fixed) / 2) : npx;
+    const size_t lds = fixed + sizeof(short) * qcap;
 #define FH_AGREE(M, S, K)                                                                                               \
     if (c.mode == M && sym == S && (vol != nullptr) == K) {                                                             \
         hipLaunchKernelGGL((k_agree_batch<M, S, K>), dim3(ntx * nty, nslices), dim3(16 * AY), lds, s, slices, nsym, t3d, \
-                           wq, c, n3, sub, data, norm, vol, exptab, rtab, acc);                                         \
+                           wq, c, n3, sub, qcap, data, norm, vol, exptab, rtab, acc);                                         \
         return hipGetLastError();                                                                                       \
     }
     FH_AGREE(0, false, false)
