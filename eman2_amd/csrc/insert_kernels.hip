@@ -3263,7 +3263,10 @@ hipError_t launch_scatter_wide(const float2 *slices, int nslices, int nsym, cons
 // ------------------------------------------------------------ merge of partial bricks
 // Items per brick from which they are summed before the merge reads them: 2
 // where the batch has an item per brick of the grid (bricks outside the
-// sphere of slices, about half, have none), else never.
+// sphere of slices, about half, have none), else never.  A batch that overran
+// the item list (bb.ctl[3], an internal error that the host reports, in a
+// captured sequence after the merge) has offsets past the partial bricks:
+// both kernels leave it alone.
 __device__ __forceinline__ int reduce_least(const int *__restrict__ item_off, int nbricks)
 {
     return item_off[3 * nbricks] >= nbricks ? 2 : INT_MAX;
@@ -3279,12 +3282,12 @@ __device__ __forceinline__ int reduce_least(const int *__restrict__ item_off, in
 // included.  Below an item per brick of the grid nothing is gained (8,000
 // gauss_var slices at pad 384, 0.5: 4.6 ms, and 4.7 with a pass over all).
 __global__ void __launch_bounds__(256) k_reduce_items(float *__restrict__ part, const int *__restrict__ item_off,
-                                                      int nbricks, int pf)
+                                                      const int *__restrict__ ctl, int nbricks, int pf)
 {
     __shared__ int q[256][3];  // first item, items, segment
     __shared__ int nq;
     const int least = reduce_least(item_off, nbricks);
-    if (least == INT_MAX) return;
+    if (least == INT_MAX || ctl[3]) return;
     const int segs = (pf + 255) / 256, lane = threadIdx.x & 63;
     const long long units = (long long)nbricks * segs;
     for (long long r = 0; r * 256 * gridDim.x < units; r++) {
@@ -3378,8 +3381,10 @@ __device__ __forceinline__ void partial_sum(const float *__restrict__ part, cons
 // instead of 0.65 at 192.
 template <int BS, int HL, int BZ, int HZ, bool PATCH>
 __global__ void __launch_bounds__(256) k_merge_partials(const float *__restrict__ part, const int *__restrict__ item_off,
-                                                        BrickGeom g, InsertConst c, float2 *data, float *norm)
+                                                        const int *__restrict__ ctl, BrickGeom g, InsertConst c,
+                                                        float2 *data, float *norm)
 {
+    if (ctl[3]) return;
     const int least = reduce_least(item_off, g.nb * g.nb * g.nbz);
     const int H = c.H, P = c.P, nb = g.nb, nbz = g.nbz, ow = g.ow, pf = g.part_floats;
     int xs, ys, zs;
@@ -3466,13 +3471,13 @@ hipError_t launch_merge_partials(BrickGeom g, BinBuffers b, InsertConst c, float
     const int nbricks = g.nb * g.nb * g.nbz;
     const long long units = (long long)nbricks * ((g.part_floats + 255) / 256);
     hipLaunchKernelGGL(k_reduce_items, dim3((unsigned)std::min(2048LL, (units + 3) / 4)), dim3(256), 0, s, b.part,
-                       b.item_off, nbricks, g.part_floats);
+                       b.item_off, b.ctl, nbricks, g.part_floats);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
 #define FH_MERGE(BS, HL, BZ, HZ, PATCH)                                                                                \
     if (g.bs == BS && g.halo == HL && g.bsz == BZ && g.haloz == HZ) {                                                  \
         hipLaunchKernelGGL((k_merge_partials<BS, HL, BZ, HZ, PATCH>), dim3(PATCH ? patches : linear), dim3(256), 0, s, \
-                           b.part, b.item_off, g, c, data, norm);                                                      \
+                           b.part, b.item_off, b.ctl, g, c, data, norm);                                                      \
         return hipGetLastError();                                                                                      \
     }
     FH_MERGE(BRICK, HALO, BRICK, HALO, false)
