@@ -7,8 +7,10 @@
 // Everything here lives while a handle or a server does (HostPool::Ref): the
 // last one to go gives it all back.  Kept blocks are bounded (KEEP_DEVICE
 // bytes per device, KEEP_STREAMS, KEEP_PINNED) and are released when an
-// allocation fails.  All calls may come from any thread.  Who gives a block
-// back has waited for the work that uses it.
+// allocation fails.  All calls may come from any thread; the lock is held for
+// the bookkeeping only, not over calls of the runtime, which may wait for other
+// handles' kernels.  Nothing is thrown.  Who gives a block back has waited for
+// the work that uses it.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -45,19 +47,23 @@ public:
             memcpy(dst, src, len);
             return;
         }
-        auto job = std::make_shared<Job>();
-        job->dst = dst;
-        job->src = src;
-        job->len = len;
-        job->nseg = (len + SEG - 1) / SEG;
-        {
+        std::shared_ptr<Job> job;
+        try {
+            job = std::make_shared<Job>();
+            job->dst = dst;
+            job->src = src;
+            job->len = len;
+            job->nseg = (len + SEG - 1) / SEG;
             std::lock_guard<std::mutex> lk(mu_);
+            jobs_.push_back(job);
             try {
                 while (threads_.size() < THREADS) threads_.emplace_back([this] { work(); });
             } catch (...) {
                 // no (more) threads: the caller copies what they do not
             }
-            jobs_.push_back(job);
+        } catch (...) {  // no memory for the job: the caller copies all
+            memcpy(dst, src, len);
+            return;
         }
         cv_.notify_all();
         job->run();
@@ -133,103 +139,170 @@ public:
         return r;
     }
 
+    HostPool()
+    {
+        streams_.reserve(KEEP_STREAMS);  // giving back never allocates
+        pinned_.reserve(KEEP_PINNED);
+    }
     ~HostPool()
     {
-        for (auto &d : dev_) release(d.second);
+        for (auto &d : dev_)
+            for (auto &b : d.second.blocks)
+                if (b.second.idle) (void)hipFree(b.first);
         for (char *p : pinned_) (void)hipHostFree(p);
         for (auto &s : streams_) (void)hipStreamDestroy(s.second);
     }
 
     // `bytes` on the current device `device`: a kept block of at most a quarter more, or a new one
-    hipError_t alloc(int device, void **p, size_t bytes)
+    hipError_t alloc(int device, void **p, size_t bytes) noexcept
     {
         bytes = std::max<size_t>(bytes, 256);
-        std::lock_guard<std::mutex> lk(mu_);
-        Device &d = dev_[device];
-        auto it = d.kept.lower_bound(bytes);
-        if (it != d.kept.end() && it->first <= bytes + bytes / 4 + 4096) {
-            *p = it->second;
-            d.sizes[*p] = it->first;
-            d.bytes -= it->first;
-            d.kept.erase(it);
+        try {
+            std::unique_lock<std::mutex> lk(mu_);
+            Device &d = dev_[device];
+            auto best = d.blocks.end();
+            for (auto it = d.blocks.begin(); it != d.blocks.end(); ++it)
+                if (it->second.idle && it->second.size >= bytes && it->second.size <= bytes + bytes / 4 + 4096 &&
+                    (best == d.blocks.end() || it->second.size < best->second.size))
+                    best = it;
+            if (best != d.blocks.end()) {
+                best->second.idle = false;
+                d.idle -= best->second.size;
+                *p = best->first;
+                return hipSuccess;
+            }
+            lk.unlock();
+            hipError_t e = hipMalloc(p, bytes);
+            if (e == hipErrorOutOfMemory) {
+                (void)hipGetLastError();
+                lk.lock();
+                shrink(lk, d, 0);
+                freed_.wait(lk, [this] { return freeing_ == 0; });
+                lk.unlock();
+                e = hipMalloc(p, bytes);
+            }
+            if (e != hipSuccess) return e;
+            lk.lock();
+            try {
+                d.blocks.emplace(*p, Block{bytes, 0, false});
+            } catch (...) {
+                lk.unlock();
+                (void)hipFree(*p);
+                throw;
+            }
             return hipSuccess;
+        } catch (...) {
+            return hipErrorOutOfMemory;
         }
-        hipError_t e = hipMalloc(p, bytes);
-        if (e == hipErrorOutOfMemory && !d.kept.empty()) {
-            (void)hipGetLastError();
-            release(d);
-            e = hipMalloc(p, bytes);
-        }
-        if (e == hipSuccess) d.sizes[*p] = bytes;
-        return e;
     }
 
-    void free(int device, void *p)
+    void free(int device, void *p) noexcept
     {
-        std::lock_guard<std::mutex> lk(mu_);
-        Device &d = dev_[device];
-        const size_t n = d.sizes[p];
-        d.sizes.erase(p);
-        if (d.bytes + n > KEEP_DEVICE) {
-            (void)hipFree(p);
+        std::unique_lock<std::mutex> lk(mu_);
+        Device &d = dev_.find(device)->second;
+        Block &b = d.blocks.find(p)->second;
+        if (d.idle + b.size > KEEP_DEVICE) {
+            d.blocks.erase(p);
+            release(lk, p);
             return;
         }
-        d.kept.emplace(n, p);
-        d.bytes += n;
+        b.idle = true;
+        b.since = ++clock_;
+        d.idle += b.size;
     }
 
     hipError_t stream(int device, hipStream_t *s)
     {
-        std::lock_guard<std::mutex> lk(mu_);
-        for (size_t i = 0; i < streams_.size(); i++)
-            if (streams_[i].first == device) {
-                *s = streams_[i].second;
-                streams_.erase(streams_.begin() + i);
-                return hipSuccess;
-            }
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            for (size_t i = 0; i < streams_.size(); i++)
+                if (streams_[i].first == device) {
+                    *s = streams_[i].second;
+                    streams_.erase(streams_.begin() + i);
+                    return hipSuccess;
+                }
+        }
         return hipStreamCreate(s);
     }
 
-    void give_stream(int device, hipStream_t s)  // idle
+    void give_stream(int device, hipStream_t s) noexcept  // idle
     {
-        std::lock_guard<std::mutex> lk(mu_);
-        if (streams_.size() < KEEP_STREAMS) streams_.emplace_back(device, s);
-        else (void)hipStreamDestroy(s);
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            if (streams_.size() < KEEP_STREAMS) {
+                streams_.emplace_back(device, s);
+                return;
+            }
+        }
+        (void)hipStreamDestroy(s);
     }
 
     hipError_t pinned(char **p)
     {
-        std::lock_guard<std::mutex> lk(mu_);
-        if (!pinned_.empty()) {
-            *p = pinned_.back();
-            pinned_.pop_back();
-            return hipSuccess;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            if (!pinned_.empty()) {
+                *p = pinned_.back();
+                pinned_.pop_back();
+                return hipSuccess;
+            }
         }
         return hipHostMalloc((void **)p, PIN_SLOTS * PIN_SLOT, hipHostMallocDefault);
     }
 
-    void give_pinned(char *p)
+    void give_pinned(char *p) noexcept
     {
-        std::lock_guard<std::mutex> lk(mu_);
-        if (pinned_.size() < KEEP_PINNED) pinned_.push_back(p);
-        else (void)hipHostFree(p);
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            if (pinned_.size() < KEEP_PINNED) {
+                pinned_.push_back(p);
+                return;
+            }
+        }
+        (void)hipHostFree(p);
     }
 
     CopyThreads copies;
 
 private:
-    struct Device {
-        std::multimap<size_t, void *> kept;
-        std::unordered_map<void *, size_t> sizes;  // blocks in use
-        size_t bytes = 0;                          // of kept
+    struct Block {
+        size_t size;
+        unsigned long long since;  // of the idle ones: when they were given back
+        bool idle;
     };
-    static void release(Device &d)
+    struct Device {
+        std::unordered_map<void *, Block> blocks;  // in use and idle: giving one back only marks it
+        size_t idle = 0;                           // bytes of the idle ones
+    };
+
+    // the idle blocks given back longest ago, until at most `most` bytes are left
+    void shrink(std::unique_lock<std::mutex> &lk, Device &d, size_t most) noexcept
     {
-        for (auto &b : d.kept) (void)hipFree(b.second);
-        d.kept.clear();
-        d.bytes = 0;
+        while (d.idle > most) {
+            auto old = d.blocks.end();
+            for (auto it = d.blocks.begin(); it != d.blocks.end(); ++it)
+                if (it->second.idle && (old == d.blocks.end() || it->second.since < old->second.since)) old = it;
+            void *p = old->first;
+            d.idle -= old->second.size;
+            d.blocks.erase(old);
+            release(lk, p);
+        }
     }
+
+    // hipFree waits for the device's work: the lock is let go, so that other handles go on
+    void release(std::unique_lock<std::mutex> &lk, void *p) noexcept
+    {
+        freeing_++;
+        lk.unlock();
+        (void)hipFree(p);
+        lk.lock();
+        if (--freeing_ == 0) freed_.notify_all();
+    }
+
     std::mutex mu_;
+    std::condition_variable freed_;
+    int freeing_ = 0;  // blocks on their way back to the device
+    unsigned long long clock_ = 0;
     std::map<int, Device> dev_;
     std::vector<std::pair<int, hipStream_t>> streams_;
     std::vector<char *> pinned_;
