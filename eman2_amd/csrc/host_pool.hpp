@@ -6,7 +6,8 @@
 //
 // Everything here lives while a handle or a server does (HostPool::Ref): the
 // last one to go gives it all back.  Kept blocks are bounded (KEEP_DEVICE
-// bytes per device, KEEP_STREAMS, KEEP_PINNED) and are released when an
+// bytes per device, KEEP_STREAMS, KEEP_PINNED): the ones given back last stay,
+// so that sizes which do not come again make room.  They are released when an
 // allocation fails.  All calls may come from any thread; the lock is held for
 // the bookkeeping only, not over calls of the runtime, which may wait for other
 // handles' kernels.  Nothing is thrown.  Who gives a block back has waited for
@@ -201,7 +202,7 @@ public:
         std::unique_lock<std::mutex> lk(mu_);
         Device &d = dev_.find(device)->second;
         Block &b = d.blocks.find(p)->second;
-        if (d.idle + b.size > KEEP_DEVICE) {
+        if (b.size > KEEP_DEVICE) {
             d.blocks.erase(p);
             release(lk, p);
             return;
@@ -209,6 +210,7 @@ public:
         b.idle = true;
         b.since = ++clock_;
         d.idle += b.size;
+        shrink(lk, d, KEEP_DEVICE);
     }
 
     hipError_t stream(int device, hipStream_t *s)

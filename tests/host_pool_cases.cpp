@@ -96,6 +96,27 @@ static void bounds()
           stub::hosts.size() <= HostPool::KEEP_PINNED);
 }
 
+// the blocks given back last are the ones that stay: sizes that do not come again make room
+static void oldest_first()
+{
+    auto p = HostPool::get();
+    std::vector<void *> v;
+    for (int i = 0; i < 8; i++) v.push_back(get(*p, 900 * MB + i));
+    for (void *x : v) p->free(0, x);
+    const int before = stub::mallocs;
+    for (int i = 0; i < 20; i++) {
+        void *a = get(*p, 2 * GB), *b = get(*p, 3 * GB);
+        p->free(0, a);
+        p->free(0, b);
+    }
+    CHECK(stub::mallocs == before + 2);
+    void *c = get(*p, 9 * GB);  // larger than all that is kept: straight back, the others stay
+    p->free(0, c);
+    void *d = get(*p, 3 * GB);
+    CHECK(stub::mallocs == before + 3);
+    p->free(0, d);
+}
+
 // an allocation that does not fit beside the idle blocks takes their place
 static void out_of_memory()
 {
@@ -241,7 +262,7 @@ static void threads()
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
-        {"reuse", reuse},   {"last_one", last_one},         {"bounds", bounds},   {"out_of_memory", out_of_memory},
+        {"reuse", reuse},   {"last_one", last_one},         {"bounds", bounds},   {"oldest_first", oldest_first}, {"out_of_memory", out_of_memory},
         {"waiting_free", waiting_free}, {"no_host_memory", no_host_memory}, {"copies", copies}, {"threads", threads},
     };
     if (argc == 1)
