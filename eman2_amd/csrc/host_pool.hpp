@@ -8,7 +8,8 @@
 // last one to go gives it all back.  Kept blocks are bounded (KEEP_DEVICE
 // bytes per device, KEEP_STREAMS, KEEP_PINNED): the ones given back last stay,
 // so that sizes which do not come again make room.  They are released when an
-// allocation fails.  All calls may come from any thread; the lock is held for
+// allocation fails, and stay within the budget of every server of the device.
+// All calls may come from any thread; the lock is held for
 // the bookkeeping only, not over calls of the runtime, which may wait for other
 // handles' kernels.  Nothing is thrown.  Who gives a block back has waited for
 // the work that uses it.
@@ -168,7 +169,9 @@ public:
                     best = it;
             if (best != d.blocks.end()) {
                 best->second.idle = false;
+                best->second.asked = bytes;
                 d.idle -= best->second.size;
+                d.spare += best->second.size - bytes;
                 *p = best->first;
                 return hipSuccess;
             }
@@ -185,7 +188,7 @@ public:
             if (e != hipSuccess) return e;
             lk.lock();
             try {
-                d.blocks.emplace(*p, Block{bytes, 0, false});
+                d.blocks.emplace(*p, Block{bytes, bytes, 0, false});
             } catch (...) {
                 lk.unlock();
                 (void)hipFree(*p);
@@ -202,7 +205,8 @@ public:
         std::unique_lock<std::mutex> lk(mu_);
         Device &d = dev_.find(device)->second;
         Block &b = d.blocks.find(p)->second;
-        if (b.size > KEEP_DEVICE) {
+        d.spare -= b.size - b.asked;
+        if (b.size > keep(device, d)) {
             d.blocks.erase(p);
             release(lk, p);
             return;
@@ -210,7 +214,38 @@ public:
         b.idle = true;
         b.since = ++clock_;
         d.idle += b.size;
-        shrink(lk, d, KEEP_DEVICE);
+        shrink(lk, d, keep(device, d));
+    }
+
+    // While `owner` has a limit, the device bytes that no handle asked for (idle blocks, and the rest of
+    // blocks larger than asked) stay within it: a server's budget less what it has committed to its jobs.
+    void limit(const void *owner, int device, long long bytes)
+    {
+        std::unique_lock<std::mutex> lk(mu_);
+        limits_[owner] = {device, bytes};
+        Device &d = dev_[device];
+        shrink(lk, d, keep(device, d));
+    }
+    void change_limit(const void *owner, long long by) noexcept
+    {
+        std::unique_lock<std::mutex> lk(mu_);
+        auto it = limits_.find(owner);
+        it->second.second += by;
+        const int device = it->second.first;
+        Device &d = dev_.find(device)->second;
+        shrink(lk, d, keep(device, d));
+    }
+    void no_limit(const void *owner) noexcept
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        limits_.erase(owner);
+    }
+    // what the blocks in use have beyond what was asked for
+    size_t spare(int device) noexcept
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        auto it = dev_.find(device);
+        return it == dev_.end() ? 0 : it->second.spare;
     }
 
     hipError_t stream(int device, hipStream_t *s)
@@ -268,14 +303,25 @@ public:
 
 private:
     struct Block {
-        size_t size;
+        size_t size, asked;
         unsigned long long since;  // of the idle ones: when they were given back
         bool idle;
     };
     struct Device {
         std::unordered_map<void *, Block> blocks;  // in use and idle: giving one back only marks it
         size_t idle = 0;                           // bytes of the idle ones
+        size_t spare = 0;                          // bytes of the ones in use beyond what was asked for
     };
+
+    // the most idle bytes of a device
+    size_t keep(int device, const Device &d) const noexcept
+    {
+        size_t most = KEEP_DEVICE;
+        for (auto &l : limits_)
+            if (l.second.first == device)
+                most = (size_t)std::min<long long>(most, std::max(0LL, l.second.second - (long long)d.spare));
+        return most;
+    }
 
     // the idle blocks given back longest ago, until at most `most` bytes are left
     void shrink(std::unique_lock<std::mutex> &lk, Device &d, size_t most) noexcept
@@ -306,6 +352,7 @@ private:
     int freeing_ = 0;  // blocks on their way back to the device
     unsigned long long clock_ = 0;
     std::map<int, Device> dev_;
+    std::map<const void *, std::pair<int, long long>> limits_;  // by owner: device, bytes
     std::vector<std::pair<int, hipStream_t>> streams_;
     std::vector<char *> pinned_;
 };

@@ -99,6 +99,7 @@ static void run_job(fh_server *s, Job *job)
     }
     if (rc == FH_OK && j.out_map) rc = fh_finish(h, 1, j.out_map, nullptr);
     else if (rc == FH_OK) rc = fh_sync(h);
+    s->pool->change_limit(s, job->st.footprint_bytes);  // its blocks become idle ones
     fh_destroy(h);
     std::lock_guard<std::mutex> lk(s->mu);
     s->committed -= job->st.footprint_bytes;
@@ -122,8 +123,10 @@ static void worker(fh_server *s)
             if (s->stop) return true;
             if (s->pending.empty()) return false;
             const Job *j = s->jobs[s->pending.front()].get();
+            // reused blocks may be larger than the jobs asked for
+            const long long spare = s->running ? (long long)s->pool->spare(s->device) : 0;
             return j->st.footprint_bytes > s->budget || j->cancel ||
-                   s->committed + j->st.footprint_bytes <= s->budget;
+                   s->committed + spare + j->st.footprint_bytes <= s->budget;
         });
         if (s->stop) return;
         Job *job = s->jobs[s->pending.front()].get();
@@ -147,6 +150,8 @@ static void worker(fh_server *s)
         job->st.t_admit = s->now();
         s->cv.notify_all();
         lk.unlock();
+        // idle blocks make room for the job: admitted and idle bytes stay within the budget
+        s->pool->change_limit(s, -job->st.footprint_bytes);
         run_job(s, job);
         lk.lock();
     }
@@ -166,6 +171,7 @@ int fh_server_create(int device, long long hbm_budget_bytes, int max_active, int
     s->max_active = max_active;
     s->chunk = chunk;
     s->t0 = std::chrono::steady_clock::now();
+    s->pool->limit(s, device, hbm_budget_bytes);
     for (int i = 0; i < max_active; i++) s->workers.emplace_back(worker, s);
     *out = s;
     return FH_OK;
@@ -242,6 +248,7 @@ int fh_server_destroy(fh_server *s)
         s->cv.notify_all();
     }
     for (auto &t : s->workers) t.join();
+    s->pool->no_limit(s);
     delete s;
     return FH_OK;
 }

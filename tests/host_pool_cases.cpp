@@ -117,6 +117,39 @@ static void oldest_first()
     p->free(0, d);
 }
 
+// a limit holds for idle blocks and for what reused blocks have beyond what was asked for
+static void limits()
+{
+    auto p = HostPool::get();
+    int a, b;
+    p->limit(&a, 0, 2 * GB);
+    std::vector<void *> v;
+    for (int i = 0; i < 6; i++) v.push_back(get(*p, 500 * MB));
+    for (void *x : v) p->free(0, x);
+    CHECK(stub::used == 2000 * MB);
+    p->change_limit(&a, -(long long)GB);
+    CHECK(stub::used == 1000 * MB);
+    void *x = get(*p, 420 * MB);
+    CHECK(p->spare(0) == 80 * MB);
+    p->change_limit(&a, -400ll * (long long)MB);  // 624 MB: 80 in use, 500 idle
+    CHECK(stub::used == 1000 * MB);
+    p->change_limit(&a, -100ll * (long long)MB);
+    CHECK(stub::used == 500 * MB);
+    p->limit(&b, 0, 0);
+    p->free(0, x);
+    CHECK(stub::used == 0 && p->spare(0) == 0);
+    p->no_limit(&b);
+    p->change_limit(&a, 2 * (long long)GB);
+    p->free(0, get(*p, 2 * GB));
+    CHECK(stub::used == 2 * GB);
+    p->limit(&b, 1, 0);  // of another device
+    p->no_limit(&a);
+    p->free(0, get(*p, 4 * GB));
+    CHECK(stub::used == 6 * GB);
+    p->change_limit(&b, -(long long)GB);
+    p->no_limit(&b);
+}
+
 // an allocation that does not fit beside the idle blocks takes their place
 static void out_of_memory()
 {
@@ -262,7 +295,7 @@ static void threads()
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
-        {"reuse", reuse},   {"last_one", last_one},         {"bounds", bounds},   {"oldest_first", oldest_first}, {"out_of_memory", out_of_memory},
+        {"reuse", reuse},   {"last_one", last_one},         {"bounds", bounds},   {"oldest_first", oldest_first}, {"limits", limits}, {"out_of_memory", out_of_memory},
         {"waiting_free", waiting_free}, {"no_host_memory", no_host_memory}, {"copies", copies}, {"threads", threads},
     };
     if (argc == 1)
