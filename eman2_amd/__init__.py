@@ -12,7 +12,7 @@ from .transform import Transform, euler_eman_matrix, euler_eman_matrices  # noqa
 def __getattr__(name):
     # the reconstructor surface loads the HIP library lazily so that the
     # CPU-side helpers stay importable without it
-    if name in ("Reconstructors", "FourierHipReconstructor", "EMData"):
+    if name in ("Reconstructors", "FourierHipReconstructor", "EMData", "trim"):
         from . import reconstructor
         return getattr(reconstructor, name)
     raise AttributeError(name)

@@ -66,6 +66,7 @@ EXPORTS = {
     "fh_server_clock": (_c_double, [_vp]),
     "fh_server_destroy": (_c_int, [_vp]),
     "fh_server_last_error": (ctypes.c_char_p, [_vp]),
+    "fh_trim": (_c_int, [_c_int]),
     "fh_create": (_c_int, [ctypes.POINTER(Params), ctypes.POINTER(_vp)]),
     "fh_destroy": (_c_int, [_vp]),
     "fh_last_error": (ctypes.c_char_p, [_vp]),

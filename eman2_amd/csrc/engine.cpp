@@ -2140,6 +2140,12 @@ int fh_get_stats(const fh_reconstructor *h, fh_stats *s)
     return FH_OK;
 }
 
+int fh_trim(int device)
+{
+    if (HostPool::Ref pool = HostPool::get(false)) pool->trim(device);
+    return FH_OK;
+}
+
 int fh_sync(fh_reconstructor *h)
 {
     if (!h) return FH_ERR_NULL;

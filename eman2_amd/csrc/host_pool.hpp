@@ -8,8 +8,9 @@
 // last one to go gives it all back.  Kept blocks are bounded (KEEP_DEVICE
 // bytes per device, KEEP_STREAMS, KEEP_PINNED): the ones given back last stay,
 // so that sizes which do not come again make room.  They are released when an
-// allocation fails, and stay within the budget of every server of the device.
-// All calls may come from any thread; the lock is held for
+// allocation fails, stay within the budget of every server of the device, and
+// give way where the device is nearly full; fh_trim gives them all back.  All
+// calls may come from any thread; the lock is held for
 // the bookkeeping only, not over calls of the runtime, which may wait for other
 // handles' kernels.  Nothing is thrown.  Who gives a block back has waited for
 // the work that uses it.
@@ -129,15 +130,16 @@ class HostPool {
 public:
     using Ref = std::shared_ptr<HostPool>;
     static constexpr size_t KEEP_DEVICE = 8ull << 30, KEEP_STREAMS = 16, KEEP_PINNED = 4;
+    static constexpr size_t LARGE = 32ull << 20;  // from here on a block is kept by what the device has left
     static constexpr size_t PIN_SLOTS = 4, PIN_SLOT = 16u << 20;  // a staging ring: 4 slots of 16 MB
 
-    static Ref get()
+    static Ref get(bool make = true)
     {
         static std::mutex mu;
         static std::weak_ptr<HostPool> pool;
         std::lock_guard<std::mutex> lk(mu);
         Ref r = pool.lock();
-        if (!r) pool = r = std::make_shared<HostPool>();
+        if (!r && make) pool = r = std::make_shared<HostPool>();
         return r;
     }
 
@@ -206,7 +208,18 @@ public:
         Device &d = dev_.find(device)->second;
         Block &b = d.blocks.find(p)->second;
         d.spare -= b.size - b.asked;
-        if (b.size > keep(device, d)) {
+        b.asked = b.size;
+        size_t most = KEEP_DEVICE;
+        if (b.size >= LARGE) {
+            // beside other programs, and other allocators of this one, that fill the device: at most a third of
+            // what it has left (2 us)
+            size_t left = 0, total = 0;
+            lk.unlock();
+            if (hipMemGetInfo(&left, &total) == hipSuccess) most = left / 3;
+            lk.lock();
+        }
+        most = std::min(most, keep(device, d));
+        if (b.size > most) {
             d.blocks.erase(p);
             release(lk, p);
             return;
@@ -214,7 +227,15 @@ public:
         b.idle = true;
         b.since = ++clock_;
         d.idle += b.size;
-        shrink(lk, d, keep(device, d));
+        shrink(lk, d, most);
+    }
+
+    // the idle blocks back to the device
+    void trim(int device) noexcept
+    {
+        std::unique_lock<std::mutex> lk(mu_);
+        auto it = dev_.find(device);
+        if (it != dev_.end()) shrink(lk, it->second, 0);
     }
 
     // While `owner` has a limit, the device bytes that no handle asked for (idle blocks, and the rest of

@@ -498,6 +498,12 @@ class FourierIterHipReconstructor(FourierHipReconstructor):
         return {}
 
 
+def trim(device=0):
+    """gives device memory kept from earlier handles for the next ones back to
+    the device, for programs that share it with other allocators"""
+    _lib.check(_lib.load().fh_trim(int(device)))
+
+
 class Reconstructors:
     """Factory<Reconstructor> (libEM/emobject.h:724-889) with
     "fourier_hip" and "fourier_iter_hip" registered; ``add`` mirrors

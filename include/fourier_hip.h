@@ -278,6 +278,11 @@ int fh_get_state(fh_reconstructor *h, float *data, float *weights);
 int fh_set_tuning(fh_reconstructor *h, const fh_tuning *t);
 int fh_get_tuning(const fh_reconstructor *h, fh_tuning *t);
 int fh_get_stats(const fh_reconstructor *h, fh_stats *s);
+/* Device memory that handles gave back stays with the process for the next
+ * ones while any handle or server lives: at most 8 GiB per device, within
+ * every server's budget, less where the device is nearly full.  fh_trim gives
+ * it back now, for programs that share the device with other allocators. */
+int fh_trim(int device);
 /* wait for all queued device work of this handle */
 int fh_sync(fh_reconstructor *h);
 /* Symmetry3D::get_symmetries (libEM/symmetry.cpp:1240-1246): the rotation

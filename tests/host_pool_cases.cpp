@@ -150,6 +150,30 @@ static void limits()
     p->no_limit(&b);
 }
 
+// idle blocks give way where others fill the device, and on request
+static void others()
+{
+    auto p = HostPool::get();
+    stub::capacity = 20 * GB;
+    void *a = get(*p, 3 * GB), *b = get(*p, 2 * GB), *c = get(*p, GB);
+    stub::others = 11 * GB;  // 3 GB left
+    p->free(0, a);
+    CHECK(stub::used == 3 * GB);
+    p->free(0, c);           // 6 GB left, a third of it 2
+    p->free(0, b);
+    CHECK(stub::used == 2 * GB);
+    stub::others = 0;
+    p->trim(1);
+    CHECK(stub::used == 2 * GB);
+    p->trim(0);
+    CHECK(stub::used == 0);
+    p->free(0, get(*p, 3 * GB));
+    CHECK(stub::used == 3 * GB);
+    CHECK(HostPool::get(false) == p);
+    p.reset();
+    CHECK(!HostPool::get(false) && stub::used == 0);
+}
+
 // an allocation that does not fit beside the idle blocks takes their place
 static void out_of_memory()
 {
@@ -295,7 +319,7 @@ static void threads()
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
-        {"reuse", reuse},   {"last_one", last_one},         {"bounds", bounds},   {"oldest_first", oldest_first}, {"limits", limits}, {"out_of_memory", out_of_memory},
+        {"reuse", reuse},   {"last_one", last_one},         {"bounds", bounds},   {"oldest_first", oldest_first}, {"limits", limits}, {"others", others}, {"out_of_memory", out_of_memory},
         {"waiting_free", waiting_free}, {"no_host_memory", no_host_memory}, {"copies", copies}, {"threads", threads},
     };
     if (argc == 1)
