@@ -313,7 +313,6 @@ struct fh_reconstructor {
     float2 *data = nullptr;
     float *norm = nullptr;
     float2 *ref = nullptr;      // fourier_iter: the reference volume of setup_seed (or null)
-    float4 *pack = nullptr;     // the volume as (re, im, weight, 0) in cubes of 2^3 voxels, for the batched agreement
     float2 *pvol = nullptr;     // gauss_fft projector: the map's transform (phase origin at the corner)
     float *exptab = nullptr, *rtab = nullptr, *syms_d = nullptr;
     float2 *tw = nullptr;
@@ -491,7 +490,6 @@ static void free_volume(fh_reconstructor *h)
 {
     if (h->data) { dfree(h, h->data); h->data = nullptr; }
     if (h->norm) { dfree(h, h->norm); h->norm = nullptr; }
-    if (h->pack) { dfree(h, h->pack); h->pack = nullptr; }
     h->ready = false;
 }
 
@@ -1839,16 +1837,24 @@ int fh_agreement_batch(fh_reconstructor *h, const float *imgs, int n, int box, c
     }
     const InsertConst c = iconst(h);
     const float rmax = agree_rmax(h->P, apix);
-    const float4 *vol = nullptr;
-    // packing moves 28 bytes a voxel, 14 P^3; a slice then reads some 35 P^2 bytes less: worth it from about
-    // 0.4 P slices on (pad 600, 8,000 slices: 0.62 ms for 9.6)
-    if (!seq && (long long)n * h->nsym >= h->P) {
-        if (!h->pack && dmalloc(h, &h->pack, sizeof(float4) * pack_elems(h->P)) != hipSuccess) {
-            (void)hipGetLastError();  // no room: the volume and its weights are read as they are
-            h->pack = nullptr;
+    // The volume as (re, im, weight, 0) in cubes of 2^3 voxels, for this call: packing moves 28 bytes a voxel,
+    // 14 P^3; a slice then reads some 35 P^2 bytes less, which pays from 0.4 P slices on. Taken from P on (pad
+    // 600, 8,000 slices: 0.62 ms for 9.6). It takes 16 bytes a voxel, after all else that the call needs.
+    struct Pack {
+        fh_reconstructor *h;
+        float4 *vol = nullptr;
+        ~Pack()
+        {
+            if (vol) dfree(h, vol);
         }
-        if (h->pack) FH_TRY(h, launch_pack_volume(h->data, h->norm, h->P, h->pack, h->stream));
-        vol = h->pack;
+    } pack{h};
+    if (!seq && (long long)n * h->nsym >= h->P) {
+        if (xfh && (rc = ensure_ximgs(h, chunk, defocus && ctf ? 1 : 0))) return rc;
+        if (dmalloc(h, &pack.vol, sizeof(float4) * pack_elems(h->P)) != hipSuccess) {
+            (void)hipGetLastError();  // no room: the volume and its weights are read as they are
+            pack.vol = nullptr;
+        }
+        if (pack.vol) FH_TRY(h, launch_pack_volume(h->data, h->norm, h->P, pack.vol, h->stream));
     }
     std::vector<float> res(5 * (size_t)std::max(n, 1));
     std::vector<double> acc(8 * (size_t)chunk);
@@ -1878,7 +1884,7 @@ int fh_agreement_batch(fh_reconstructor *h, const float *imgs, int n, int box, c
         // (what e2make3d.py:447-491 gets from determine_slice_agreement called
         // particle by particle), recomputed by a gather instead of mutating V
         FH_TRY(h, launch_agree_batch(h->slices, h->nsym, h->t3d, h->wq, m * h->nsym, c, rmax, sub, h->data, h->norm,
-                                     vol, h->exptab, h->rtab, h->acc8, h->stream));
+                                     pack.vol, h->exptab, h->rtab, h->acc8, h->stream));
         FH_TRY(h, hipMemcpyAsync(acc.data(), h->acc8, sizeof(double) * 8 * m, hipMemcpyDeviceToHost, h->stream));
         FH_TRY(h, hipStreamSynchronize(h->stream));
         for (int i = 0; i < m; i++)
