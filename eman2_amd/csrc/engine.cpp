@@ -578,9 +578,15 @@ static BrickGeom brick_geom(int P, int mode)
     return g;
 }
 
-// list entries a slice can take: at most 5 bricks per brick column along its
-// dominant normal axis (4 shown, see k_bin_cols)
-static long long list_per_slice(const BrickGeom &g) { return 5LL * g.nb * std::max(g.nb, g.nbz); }
+// List entries a slice can take.  Along its dominant normal axis (slopes of at
+// most 1, margins below 0.01, see k_bin_cols) it spans at most the column's two
+// edges, which reach floor(span / edge) + 2 bricks: 4 of the cubes; of the 3 x
+// 3 x 5 bricks 4 along x or y and 3 along z, whose columns are the most.
+static long long list_per_slice(const BrickGeom &g)
+{
+    const long long xy = (long long)((g.bs + g.bsz + 0.01) / g.bs) + 2, z = (long long)((2 * g.bs + 0.01) / g.bsz) + 2;
+    return std::max(xy * g.nb * g.nbz, z * g.nb * g.nb);
+}
 
 // Slices per work item of a batch of nslices slices (at most the tuned value).
 // A work item is one wave's serial chain and ends in one partial brick: with
@@ -610,9 +616,8 @@ static int ensure_bins(fh_reconstructor *h, long long nslices)
     h->geom = g;
     BinBuffers &b = h->bins;
     b.list_cap = list_per_slice(g) * nslices;
-    // smaller batches have fewer items: pairs over K grows with the slices, up to K's rounding
-    const int K = item_slices(h, nslices);
-    b.item_cap = b.list_cap / K * (K < h->tune.slices_per_item ? 5 : 4) / 4 + g.nkeys + 1;
+    // smaller batches have fewer items: pairs over K grows with the slices, up to K's rounding (17 / 16)
+    b.item_cap = b.list_cap / item_slices(h, nslices) * 5 / 4 + g.nkeys + 1;
     FH_TRY(h, dmalloc(h, &b.counts, sizeof(int) * g.nkeys));
     FH_TRY(h, dmalloc(h, &b.offsets, sizeof(int) * (g.nkeys + 1)));
     FH_TRY(h, dmalloc(h, &b.item_off, sizeof(int) * (g.nkeys + 1)));
@@ -627,14 +632,15 @@ static int ensure_bins(fh_reconstructor *h, long long nslices)
 }
 
 // Partial bricks for `items` work items (grown on demand; 8.5 KiB each for
-// gauss_2 and gauss_var).
+// gauss_2, 7.5 for the 6-cell Gaussians), with room for batches that need
+// some more.
 static int ensure_partials(fh_reconstructor *h, long long items)
 {
     BinBuffers &b = h->bins;
     if (items <= b.part_cap) return FH_OK;
     if (b.part) { dfree(h, b.part); b.part = nullptr; }
     b.part_cap = 0;
-    const long long cap = items + items / 4 + 1024;
+    const long long cap = items + items / 16 + 1024;
     FH_TRY(h, dmalloc(h, &b.part, sizeof(float) * h->geom.part_floats * (size_t)cap));
     b.part_cap = cap;
     return FH_OK;
