@@ -598,15 +598,25 @@ static long long list_per_slice(const BrickGeom &g)
 // slices 1.38 -> 0.37 ms; pad 192, 5,000 slices 2.66 -> 1.45 ms; pad 384,
 // 24,000 slices (K = 757) 19.85 -> 19.9 ms; gauss_var at pad 96, 3,000 slices
 // 6.8 -> 3.6 ms, at pad 192, 1,000 slices 8.2 -> 3.3 ms.
+static int item_slices(const BrickGeom &g, int P, bool wide, int cus, int most, long long nslices)
+{
+    // about 0.63 of (P + brick)^2 times the brick's mean width over its volume
+    const double pb2 = (double)(P + 8) * (P + 8) * (2 * g.bs + g.bsz) / (3.0 * g.bs * g.bs * g.bsz);
+    const double per_wave = 0.63 * pb2 * (double)nslices / (16.0 * cus);
+    const double k = (wide ? 6.0 : 8.0) * sqrt(per_wave);
+    return (int)std::min((double)most, std::max(16.0, k));
+}
 static int item_slices(const fh_reconstructor *h, long long nslices)
 {
-    const BrickGeom &g = h->geom;
-    // about 0.63 of (P + brick)^2 times the brick's mean width over its volume
-    const double pb2 = (double)(h->P + 8) * (h->P + 8) * (2 * g.bs + g.bsz) / (3.0 * g.bs * g.bs * g.bsz);
-    const double per_wave = 0.63 * pb2 * (double)nslices / (16.0 * h->cus);
-    const double k = (wide_cells(h->mode) ? 6.0 : 8.0) * sqrt(per_wave);
-    return (int)std::min((double)h->tune.slices_per_item, std::max(16.0, k));
+    return item_slices(h->geom, h->P, wide_cells(h->mode) != 0, h->cus, h->tune.slices_per_item, nslices);
 }
+
+// room of the work item list; smaller batches fit too: pairs over K grows with the slices, up to K's rounding
+// (17 / 16)
+static long long item_room(const BrickGeom &g, long long list, int K) { return list / K * 5 / 4 + g.nkeys + 1; }
+
+// room of the partial bricks for `items` work items: batches that need some more fit too
+static long long partial_room(long long items) { return items + items / 16 + 1024; }
 
 static int ensure_bins(fh_reconstructor *h, long long nslices)
 {
@@ -616,8 +626,7 @@ static int ensure_bins(fh_reconstructor *h, long long nslices)
     h->geom = g;
     BinBuffers &b = h->bins;
     b.list_cap = list_per_slice(g) * nslices;
-    // smaller batches have fewer items: pairs over K grows with the slices, up to K's rounding (17 / 16)
-    b.item_cap = b.list_cap / item_slices(h, nslices) * 5 / 4 + g.nkeys + 1;
+    b.item_cap = item_room(g, b.list_cap, item_slices(h, nslices));
     FH_TRY(h, dmalloc(h, &b.counts, sizeof(int) * g.nkeys));
     FH_TRY(h, dmalloc(h, &b.offsets, sizeof(int) * (g.nkeys + 1)));
     FH_TRY(h, dmalloc(h, &b.item_off, sizeof(int) * (g.nkeys + 1)));
@@ -632,15 +641,14 @@ static int ensure_bins(fh_reconstructor *h, long long nslices)
 }
 
 // Partial bricks for `items` work items (grown on demand; 8.5 KiB each for
-// gauss_2, 7.5 for the 6-cell Gaussians), with room for batches that need
-// some more.
+// gauss_2, 7.5 for the 6-cell Gaussians).
 static int ensure_partials(fh_reconstructor *h, long long items)
 {
     BinBuffers &b = h->bins;
     if (items <= b.part_cap) return FH_OK;
     if (b.part) { dfree(h, b.part); b.part = nullptr; }
     b.part_cap = 0;
-    const long long cap = items + items / 16 + 1024;
+    const long long cap = partial_room(items);
     FH_TRY(h, dmalloc(h, &b.part, sizeof(float) * h->geom.part_floats * (size_t)cap));
     b.part_cap = cap;
     return FH_OK;
@@ -674,7 +682,7 @@ static int inserter_index(const char *m)
 
 // Device bytes of a handle of size P and inserter `mode` (a mode name; unknown
 // names count as gauss_2) after setup, with batches of `chunk` particles.
-long long footprint_bytes_for_mode(int P, int nsym, int chunk, const char *mode_name)
+long long footprint_bytes_for_mode(int P, int nsym, int chunk, const char *mode_name, int corners)
 {
     const int mode = mode_name ? inserter_index(mode_name) : 0;
     if (chunk <= 0) chunk = chunk_for(fh_tuning{1, 1, 0, 1, 0}, P, P);
@@ -683,15 +691,24 @@ long long footprint_bytes_for_mode(int P, int nsym, int chunk, const char *mode_
     const BrickGeom g = brick_geom(P, mode);
     const long long nslices = (long long)chunk * nsym;
     const long long list = list_per_slice(g) * nslices;
-    const long long items = list / 64 + g.nkeys + 1;
-    const long long bins = 4LL * list + 16LL * items + 16LL * g.nkeys + 3LL * (long long)sizeof(SliceRec) * nslices;
-    // partial bricks: about 1.1 (P/bs)^2 (slice, brick) pairs per slice (P^2 times the
-    // mean width of a brick over its volume), one item per 64 pairs of a key plus one
-    // per key the slices reach
+    const int K = g.per_brick ? item_slices(g, P, true, 256, 64, nslices) : 64;
+    const long long bins =
+        4LL * list + 16LL * item_room(g, list, K) + 16LL * g.nkeys + 3LL * (long long)sizeof(SliceRec) * nslices;
+    // partial bricks: about 1.1 (P/bs)^2 (slice, brick) pairs per slice (P^2 times the mean width of a brick over
+    // its volume), one item per K pairs and one per key that the slices reach, about half of the keys (smaller batches
+    // take fewer slices per item, but reach fewer keys); the wide stencils' items span a brick's keys: one per
+    // brick within the pixels' reach
     const double pb2 = (double)P * P * (2 * g.bs + g.bsz) / (3.0 * g.bs * g.bs * g.bsz);
-    const long long part_items = (long long)(1.1 * pb2 * nslices / 64) + g.nkeys / 2;
+    const long long pairs = (long long)(1.1 * pb2 * nslices);
+    long long parts = pairs / K + g.nkeys / 2;
+    if (g.per_brick) {
+        const double r = P / 2 + 3.5 + 0.5 * sqrt((double)(2 * g.bs * g.bs + g.bsz * g.bsz));
+        const double ball = 4.0 / 3.0 * M_PI * r * r * r / (g.bs * g.bs * g.bsz);
+        const long long bricks = corners ? g.nbricks : (long long)std::min((double)g.nbricks, ball);
+        parts = partial_room(pairs / K + std::min(bricks, pairs));
+    }
     const long long inter = (long long)prep_inter_bytes(P, std::min(chunk, PREP_INTER_PARTICLES));
-    return v + sl + inter + bins + 4LL * g.part_floats * part_items;
+    return v + sl + inter + bins + 4LL * g.part_floats * parts;
 }
 
 extern "C" {
@@ -2181,7 +2198,7 @@ int fh_get_symmetries(const char *sym, float *out9, int max_ops)
 
 long long fh_footprint_bytes(int P, int nsym, int chunk)
 {
-    return footprint_bytes_for_mode(P, nsym, chunk, nullptr);
+    return footprint_bytes_for_mode(P, nsym, chunk, nullptr, 0);
 }
 
 }  // extern "C"
