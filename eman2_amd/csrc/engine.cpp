@@ -1849,7 +1849,8 @@ int fh_agreement_batch(fh_reconstructor *h, const float *imgs, int n, int box, c
     const float *xfh = xf6.empty() ? nullptr : xf6.data();
     std::vector<float> df2;
     second_defocus(defocus, ctf, n, df2);
-    const long long xbytes = xfh ? ((defocus && ctf) ? 8LL : 4LL) * h->P * h->P : 0;
+    // a CTF flip before a 2-D resampling stages a P x P image per particle
+    const long long xbytes = xfh && defocus && ctf ? 4LL * h->P * h->P : 0;
     const int chunk = std::max(1, std::min(chunk_for(h->tune, h->P, box, xbytes), std::max(n, 1)));
     if ((rc = ensure_chunk(h, chunk, box))) return rc;
     if (!h->acc8 || h->acc8_cap < chunk) {

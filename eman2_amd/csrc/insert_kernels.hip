@@ -280,8 +280,8 @@ __global__ void __launch_bounds__(256) k_insert_corners(const float2 *__restrict
 // The plain (global-atomic) form over every slice of a batch in one launch:
 // block (xb, q) covers pixels x in [64 xb, 64 xb + 64) of rows y of slice q
 // = p nsym + s, with t3d[q] and weight wq[q] (or the particle's class_ssnr
-// radial weights).  Used for the inserter modes the brick scatter does not
-// take (gauss_var's 6x6x6 stencil).
+// radial weights).  For the wide modes where a batch has more tiles than a grid
+// of k_insert_wide_tiles holds (2^31).
 __global__ void __launch_bounds__(64) k_insert_plain_batch(const float2 *__restrict__ slices, int nsym, int nxb,
                                                            const float *__restrict__ t3d, const float *__restrict__ wq,
                                                            InsertConst c, float2 *data, float *norm,
@@ -302,19 +302,7 @@ __global__ void __launch_bounds__(64) k_insert_plain_batch(const float2 *__restr
     const float *m = t3d + 9 * (size_t)q;
     float xx, yy, zz;
     pixel_coords(x, y, m, rtab_g, H, c.Pf, xx, yy, zz);
-    const float2 dt = slice_value(S, x, y, P, H);
-    if (c.mode >= 2) {
-        insert_wide(c.mode, dt, xx, yy, zz, weight, P, H, exptab, data, norm, c.ref);
-        return;
-    }
-    const int x0 = (int)floorf(xx), y0 = (int)floorf(yy), z0 = (int)floorf(zz);
-    if (x0 < -H - 1 || y0 < -H - 1 || z0 < -H - 1 || x0 > H || y0 > H || z0 > H) return;
-    for (int k = z0; k <= z0 + 1; k++)
-        for (int j = y0; j <= y0 + 1; j++)
-            for (int i = x0; i <= x0 + 1; i++) {
-                const float gg = corner_weight(c.mode, i, j, k, xx, yy, zz, c.h, weight, exptab);
-                add_complex_atomic(data, norm, P, H, i, j, k, dt.x * gg, dt.y * gg, gg);
-            }
+    insert_wide(c.mode, slice_value(S, x, y, P, H), xx, yy, zz, weight, P, H, exptab, data, norm, c.ref);
 }
 
 // The wide modes with LDS accumulation: a workgroup takes an 8 x 8 tile of
@@ -677,14 +665,13 @@ hipError_t launch_insert_plain_batch(const float2 *slices, int nslices, int nsym
                                      const float *rw, hipStream_t s)
 {
     if (nslices <= 0) return hipSuccess;
-    if (c.mode >= 2) {
-        const int ntx = (c.H + 1 + WT_TILE - 1) / WT_TILE, nty = (c.P + WT_TILE - 1) / WT_TILE;
-        const long long blocks = (long long)ntx * nty * nslices;
-        if (blocks < INT32_MAX) {
-            hipLaunchKernelGGL(k_insert_wide_tiles, dim3((unsigned)blocks), dim3(256), sizeof(float) * 3 * WT_CELLS, s,
-                               slices, nsym, ntx, nty, t3d, wq, c, data, norm, exptab, rtab, rw);
-            return hipGetLastError();
-        }
+    if (c.mode < 2) return hipErrorInvalidValue;
+    const int ntx = (c.H + 1 + WT_TILE - 1) / WT_TILE, nty = (c.P + WT_TILE - 1) / WT_TILE;
+    const long long blocks = (long long)ntx * nty * nslices;
+    if (blocks < INT32_MAX) {
+        hipLaunchKernelGGL(k_insert_wide_tiles, dim3((unsigned)blocks), dim3(256), sizeof(float) * 3 * WT_CELLS, s,
+                           slices, nsym, ntx, nty, t3d, wq, c, data, norm, exptab, rtab, rw);
+        return hipGetLastError();
     }
     const int nxb = (c.H + 1 + 63) / 64;
     hipLaunchKernelGGL(k_insert_plain_batch, dim3(nxb * nslices, c.P), dim3(64), 0, s, slices, nsym, nxb, t3d, wq, c,
