@@ -345,7 +345,7 @@ struct fh_reconstructor {
     hipEvent_t ev[6] = {};
     // blocks, streams, pinned staging and copy threads shared with other handles
     HostPool::Ref pool = HostPool::get();
-    char *pin = nullptr;                              // staging ring
+    char *pin = nullptr;                              // staging ring of uploads
     hipEvent_t pin_ev[HostPool::PIN_SLOTS] = {};      // the last copy through each slot
 };
 
@@ -394,12 +394,11 @@ static size_t stage_chunk(size_t bytes)
     return std::min(HostPool::PIN_SLOT, std::max<size_t>(512u << 10, (bytes / 4 + 4095) & ~(size_t)4095));
 }
 
-// the staging ring and its events (recorded once, so that a first wait on
-// them returns at once)
-static hipError_t ensure_pinned(fh_reconstructor *h)
+// the events of a ring's slots (recorded once, so that a first wait on them
+// returns at once)
+static hipError_t ensure_pin_events(fh_reconstructor *h)
 {
     hipError_t e;
-    if (!h->pin && (e = h->pool->pinned(&h->pin)) != hipSuccess) return e;
     for (auto &ev : h->pin_ev)
         if (!ev) {
             if ((e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
@@ -408,21 +407,15 @@ static hipError_t ensure_pinned(fh_reconstructor *h)
     return hipSuccess;
 }
 
-static hipError_t d2h_staged(fh_reconstructor *h, void *dst, const void *src, size_t bytes)
+static hipError_t d2h_ring(fh_reconstructor *h, char *ring, char *d, const char *s, size_t bytes)
 {
     hipError_t e;
-    if (bytes < STAGE_MIN) {
-        if ((e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream)) != hipSuccess) return e;
-        return hipStreamSynchronize(h->stream);
-    }
-    if ((e = ensure_pinned(h)) != hipSuccess) return e;
-    const char *s = static_cast<const char *>(src);
-    char *d = static_cast<char *>(dst);
+    if ((e = ensure_pin_events(h)) != hipSuccess) return e;
     const size_t chunk = stage_chunk(bytes), n = (bytes + chunk - 1) / chunk, ahead = HostPool::PIN_SLOTS - 1;
     for (size_t c = 0; c < n + ahead; c++) {
         if (c < n) {  // the DMA of chunk c into its slot (free: chunk c - 4 was copied out)
             const size_t off = c * chunk, len = std::min(chunk, bytes - off), k = c % HostPool::PIN_SLOTS;
-            if ((e = hipMemcpyAsync(h->pin + k * HostPool::PIN_SLOT, s + off, len, hipMemcpyDeviceToHost, h->stream)) !=
+            if ((e = hipMemcpyAsync(ring + k * HostPool::PIN_SLOT, s + off, len, hipMemcpyDeviceToHost, h->stream)) !=
                 hipSuccess)
                 return e;
             if ((e = hipEventRecord(h->pin_ev[k], h->stream)) != hipSuccess) return e;
@@ -430,20 +423,38 @@ static hipError_t d2h_staged(fh_reconstructor *h, void *dst, const void *src, si
         if (c >= ahead && c - ahead < n) {  // chunk c - 3 out of its slot while the next ones are in flight
             const size_t q = c - ahead, off = q * chunk, len = std::min(chunk, bytes - off), k = q % HostPool::PIN_SLOTS;
             if ((e = hipEventSynchronize(h->pin_ev[k])) != hipSuccess) return e;
-            h->pool->copies.copy(d + off, h->pin + k * HostPool::PIN_SLOT, len);
+            h->pool->copies.copy(d + off, ring + k * HostPool::PIN_SLOT, len);
         }
     }
     return hipSuccess;
 }
 
+// Complete when it returns, so the ring is borrowed for the copy: as many
+// rings as copies run at once, not as handles live.
+static hipError_t d2h_staged(fh_reconstructor *h, void *dst, const void *src, size_t bytes)
+{
+    hipError_t e;
+    char *ring = bytes < STAGE_MIN ? nullptr : h->pin ? h->pin : h->pool->pinned(bytes);
+    if (!ring) {
+        if ((e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream)) != hipSuccess) return e;
+        return hipStreamSynchronize(h->stream);
+    }
+    e = d2h_ring(h, ring, static_cast<char *>(dst), static_cast<const char *>(src), bytes);
+    if (e != hipSuccess) (void)hipStreamSynchronize(h->stream);
+    if (ring != h->pin) h->pool->give_pinned(ring);
+    return e;
+}
+
 // The mirror image: host threads copy chunk c into its slot (once the DMA
 // that last read the slot is done) while the DMA of the chunks before runs.
-// Queued on the handle's stream, so kernels queued after it see the data.
+// Queued on the handle's stream, so kernels queued after it see the data; the
+// handle keeps its ring, whose last chunks may be on their way.
 static hipError_t h2d_staged(fh_reconstructor *h, void *dst, const void *src, size_t bytes)
 {
     hipError_t e;
-    if (bytes < (16ull << 20)) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream);
-    if ((e = ensure_pinned(h)) != hipSuccess) return e;
+    if (bytes >= (16ull << 20) && !h->pin) h->pin = h->pool->pinned(bytes);
+    if (bytes < (16ull << 20) || !h->pin) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream);
+    if ((e = ensure_pin_events(h)) != hipSuccess) return e;
     const char *s = static_cast<const char *>(src);
     char *d = static_cast<char *>(dst);
     const size_t chunk = stage_chunk(bytes), n = (bytes + chunk - 1) / chunk;

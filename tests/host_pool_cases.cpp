@@ -66,8 +66,8 @@ static void last_one()
     for (int i = 0; i < 30; i++) {
         hipStream_t s;
         CHECK(p->stream(0, &s) == hipSuccess);
-        char *h;
-        CHECK(p->pinned(&h) == hipSuccess);
+        char *h = p->pinned(GB);
+        CHECK(h);
         p->free(0, get(*p, (i + 1) * 100 * MB));
         p->give_stream(0, s);
         p->give_pinned(h);
@@ -88,7 +88,7 @@ static void bounds()
     std::vector<char *> h(10);
     for (int i = 0; i < 40; i++) v.push_back(get(*p, GB + i * 300 * MB));
     for (auto &x : s) CHECK(p->stream(0, &x) == hipSuccess);
-    for (auto &x : h) CHECK(p->pinned(&x) == hipSuccess);
+    for (auto &x : h) CHECK((x = p->pinned(GB)));
     for (void *x : v) p->free(0, x);
     for (auto x : s) p->give_stream(0, x);
     for (auto x : h) p->give_pinned(x);
@@ -208,7 +208,7 @@ static void waiting_free()
         void *b = get(*p, 100 * MB);
         hipStream_t s;
         char *h;
-        CHECK(p->stream(0, &s) == hipSuccess && p->pinned(&h) == hipSuccess);
+        CHECK(p->stream(0, &s) == hipSuccess && (h = p->pinned(GB)));
         p->give_stream(0, s);
         p->give_pinned(h);
         p->free(0, b);
@@ -229,6 +229,32 @@ static void waiting_free()
     CHECK(later);
 }
 
+// a pool's first small copies take no ring, large ones do; one that is there is taken by all
+static void rings()
+{
+    auto p = HostPool::get();
+    for (size_t i = 0; i < HostPool::SMALL_COPIES; i++) CHECK(!p->pinned(4 * MB));
+    char *a = p->pinned(4 * MB), *b = p->pinned(4 * MB);
+    CHECK(a && b && a != b);
+    p->give_pinned(a);
+    CHECK(p->pinned(4 * MB) == a);
+    p->give_pinned(a);
+    p->give_pinned(b);
+    p.reset();
+    CHECK(stub::hosts.empty());
+    p = HostPool::get();
+    CHECK(!p->pinned(HostPool::PIN_SLOT - 1));
+    char *c = p->pinned(HostPool::PIN_SLOT);
+    CHECK(c);
+    p->give_pinned(c);
+    CHECK(p->pinned(4 * MB) == c);
+    p->give_pinned(c);
+    stub::no_hosts = true;  // no pinned memory to be had
+    char *d = p->pinned(GB);
+    CHECK(d == c && !p->pinned(GB));
+    p->give_pinned(d);
+}
+
 // without host memory nothing is thrown: what cannot be noted is given back, copies are made by the caller
 static void no_host_memory()
 {
@@ -239,8 +265,8 @@ static void no_host_memory()
     for (int i = 0; i < 8; i++) v.push_back(get(*p, (i + 1) * MB));
     std::vector<hipStream_t> s(3);
     for (auto &x : s) CHECK(p->stream(0, &x) == hipSuccess);
-    char *h;
-    CHECK(p->pinned(&h) == hipSuccess);
+    char *h = p->pinned(GB);
+    CHECK(h);
     no_memory = true;
     bool thrown = false;
     try {
@@ -319,7 +345,7 @@ static void threads()
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
-        {"reuse", reuse},   {"last_one", last_one},         {"bounds", bounds},   {"oldest_first", oldest_first}, {"limits", limits}, {"others", others}, {"out_of_memory", out_of_memory},
+        {"reuse", reuse},   {"last_one", last_one},         {"bounds", bounds},   {"oldest_first", oldest_first}, {"limits", limits}, {"rings", rings}, {"others", others}, {"out_of_memory", out_of_memory},
         {"waiting_free", waiting_free}, {"no_host_memory", no_host_memory}, {"copies", copies}, {"threads", threads},
     };
     if (argc == 1)

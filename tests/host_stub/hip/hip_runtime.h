@@ -21,6 +21,7 @@ inline std::map<char *, size_t> blocks;                       // live device blo
 inline std::set<void *> hosts, streams;
 inline std::set<char *> hold;  // hipFree of these waits until they are taken out
 inline int mallocs = 0, frees = 0, waiting = 0;
+inline bool no_hosts = false;  // no pinned memory
 inline char *next = reinterpret_cast<char *>(1ull << 40);
 }  // namespace stub
 
@@ -66,6 +67,7 @@ inline hipError_t hipMemGetInfo(size_t *free, size_t *total)
 
 inline hipError_t hipHostMalloc(void **p, size_t n, unsigned)
 {
+    if (stub::no_hosts) return hipErrorOutOfMemory;
     *p = malloc(n);
     std::lock_guard<std::mutex> lk(stub::mu);
     stub::hosts.insert(*p);
