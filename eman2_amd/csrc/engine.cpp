@@ -382,11 +382,12 @@ static void dfree(fh_reconstructor *h, void *p)
 
 // Copies between the device and caller (pageable) memory run through a ring
 // of pinned slots, the DMA of some chunks beside the host copy of another by
-// several threads.  A pageable copy of the runtime takes longer from some
-// tens of KB on: 1 MB to the host 0.45 ms against 0.15, 4 MB 1.7 against
-// 0.25 (first touch of the target's pages included); below that it is as
-// quick as the staging.  340 MB: 8.8 ms through two 64 MB buffers and threads
-// started per chunk.
+// several threads.  The runtime's own copy takes longer from some tens of KB
+// on: 0.2 + 0.1 MB (two copies) 0.20 ms against 0.10 into fresh pages, 2.8 +
+// 1.4 MB 1.16 against 0.95, 8.1 + 4.1 MB 3.4 against 2.3, and into pages that
+// were there 0.14 against 0.05, 0.26 against 0.24, 0.75 against 0.44; only
+// around 0.5 to 1 MB into pages that were there it is the shorter one (1.0 +
+// 0.5 MB: 0.10 against 0.13, into fresh pages 0.43 against 0.41).
 constexpr size_t STAGE_MIN = 64u << 10;
 static size_t stage_chunk(size_t bytes)
 {
@@ -982,6 +983,27 @@ int fh_clear(fh_reconstructor *h)
     return FH_OK;
 }
 
+// The resampling of few particles is a pass of its own, a thread per pixel:
+// read by the prep's first pass it waits in the few workgroups that this has,
+// on the runtime plan (one particle at pad 384: 49 us, 32 apart, 90 and 69
+// with a flip; 16: 50 and 43; 128: 135 and 160).  Equal at about 32 particles
+// of pad 256 and 8 of 600.
+static bool resample_apart(const fh_reconstructor *h, int n) { return (long long)n * h->P <= 6144; }
+
+// n particles (box B, edge means or null) resampled by xfd into slices, by way of tmp if apart
+static hipError_t prep_resampled(fh_reconstructor *h, int n, int B, const float *imgs, const float *means,
+                                 const float *xfd, float *tmp)
+{
+    const int P = h->P;
+    if (!resample_apart(h, n))
+        return launch_prep2d_xform(imgs, n, B, P, means, xfd, h->slices, h->inter, h->inter_n, h->scale, h->plan, h->tw,
+                                   h->stream);
+    const hipError_t e = launch_xform2d(imgs, n, B, P, means, xfd, tmp, h->stream);
+    if (e != hipSuccess) return e;
+    return launch_prep2d(tmp, n, P, P, nullptr, h->slices, h->inter, h->inter_n, nullptr, nullptr, CtfConst{}, h->scale,
+                         h->plan, h->tw, h->stream);
+}
+
 // prep kernels of n particles (box B) into h->slices; dfd: device defocus or null
 static hipError_t prep_kernels(fh_reconstructor *h, int n, int B, const float *dev_imgs, const float *dfd,
                                const CtfConst &cc, const float *xfd = nullptr, const float *dfd2 = nullptr)
@@ -992,17 +1014,14 @@ static hipError_t prep_kernels(fh_reconstructor *h, int n, int B, const float *d
         // the reference's order (e2make3dpar.py:698-716): the padded image is
         // flipped first -- FFT, CTF_SIGN (times the second sign), inverse FFT,
         // through the slices' memory -- and preprocess_slice then resamples the
-        // flipped image with the 2-D part, read by the prep without flip
+        // flipped image with the 2-D part, for the prep without flip
         const int P = h->P;
         if ((e = launch_flip2d(dev_imgs, n, B, P, h->means, h->slices, h->inter, h->inter_n, dfd, dfd2, cc,
                                1.0f / ((float)P * (float)P), h->ximgs, h->plan, h->tw, h->stream)) != hipSuccess)
             return e;
-        return launch_prep2d_xform(h->ximgs, n, P, P, nullptr, xfd, h->slices, h->inter, h->inter_n, h->scale, h->plan,
-                                   h->tw, h->stream);
+        return prep_resampled(h, n, P, h->ximgs, nullptr, xfd, h->ximgs2);
     }
-    if (xfd)
-        return launch_prep2d_xform(dev_imgs, n, B, h->P, h->means, xfd, h->slices, h->inter, h->inter_n, h->scale,
-                                   h->plan, h->tw, h->stream);
+    if (xfd) return prep_resampled(h, n, B, dev_imgs, h->means, xfd, h->ximgs);
     return launch_prep2d(dev_imgs, n, B, h->P, h->means, h->slices, h->inter, h->inter_n, dfd, dfd2, cc, h->scale,
                          h->plan, h->tw, h->stream);
 }
@@ -1027,6 +1046,12 @@ static int ensure_ximgs(fh_reconstructor *h, int n, int stagings)
     return rc;
 }
 
+// the same for a prep of n particles with 2-D transforms
+static int ensure_resample(fh_reconstructor *h, int n, bool flip)
+{
+    return ensure_ximgs(h, n, (flip ? 1 : 0) + (resample_apart(h, n) ? 1 : 0));
+}
+
 // prep of n particles already in h->imgs (box B) into h->slices; xf_host:
 // their inverse 2-D transforms (n x 6) or null when all are identities
 // defocus2_host: the second defocus of the two-sign flip (or null)
@@ -1046,7 +1071,7 @@ static int prep_chunk(fh_reconstructor *h, int n, int B, const float *dev_imgs, 
     }
     const float *xfd = nullptr;
     if (xf_host) {
-        int rc = ensure_ximgs(h, n, dfd ? 1 : 0);
+        int rc = ensure_resample(h, n, dfd != nullptr);
         if (rc) return rc;
         FH_TRY(h, hipMemcpyAsync(h->xfd, xf_host, sizeof(float) * 6 * n, hipMemcpyHostToDevice, h->stream));
         xfd = h->xfd;
@@ -1062,11 +1087,10 @@ static int prep_single_raw(fh_reconstructor *h, const float *xf6)
 {
     const int P = h->P;
     if (xf6) {
-        int rc = ensure_ximgs(h, 1, 0);
+        int rc = ensure_resample(h, 1, false);
         if (rc) return rc;
         FH_TRY(h, hipMemcpyAsync(h->xfd, xf6, sizeof(float) * 6, hipMemcpyHostToDevice, h->stream));
-        FH_TRY(h, launch_prep2d_xform(h->imgs, 1, P, P, nullptr, h->xfd, h->slices, h->inter, h->inter_n, h->scale,
-                                      h->plan, h->tw, h->stream));
+        FH_TRY(h, prep_resampled(h, 1, P, h->imgs, nullptr, h->xfd, h->ximgs));
         return FH_OK;
     }
     FH_TRY(h, launch_prep2d(h->imgs, 1, P, P, nullptr, h->slices, h->inter, h->inter_n, nullptr, nullptr, CtfConst{},
@@ -1087,7 +1111,6 @@ static int insert_batch_graph(fh_reconstructor *h, const float *imgs, int n, int
 {
     int rc = ensure_partials(h, h->bins.item_cap);
     if (rc) return rc;
-    if (xf_host && (rc = ensure_ximgs(h, chunk, defocus && ctf ? 1 : 0))) return rc;
     const InsertConst c = iconst(h);
     fh_stats st{};
     const int wpb = h->tune.waves_per_block;
@@ -1097,6 +1120,7 @@ static int insert_batch_graph(fh_reconstructor *h, const float *imgs, int n, int
     for (int c0 = 0; c0 < n; c0 += chunk) {
         const int m = std::min(chunk, n - c0);
         const float *dimgs = imgs + (size_t)c0 * box * box;
+        if (xf_host && (rc = ensure_resample(h, m, defocus && ctf))) return rc;
         FH_TRY(h, hipMemcpyAsync(h->rots, &rot9[9 * (size_t)c0], sizeof(float) * 9 * m, hipMemcpyHostToDevice, h->stream));
         FH_TRY(h, hipMemcpyAsync(h->wts, weights + c0, sizeof(float) * m, hipMemcpyHostToDevice, h->stream));
         if (rw_host)
@@ -1884,7 +1908,8 @@ int fh_agreement_batch(fh_reconstructor *h, const float *imgs, int n, int box, c
         }
     } pack{h};
     if (!seq && (long long)n * h->nsym >= h->P) {
-        if (xfh && (rc = ensure_ximgs(h, chunk, defocus && ctf ? 1 : 0))) return rc;
+        for (int m : {chunk, n % chunk})
+            if (xfh && m > 0 && (rc = ensure_resample(h, m, defocus && ctf))) return rc;
         if (dmalloc(h, &pack.vol, sizeof(float4) * pack_elems(h->P)) != hipSuccess) {
             (void)hipGetLastError();  // no room: the volume and its weights are read as they are
             pack.vol = nullptr;

@@ -56,7 +56,7 @@ __global__ void k_compose(const float *__restrict__ rots, const float *__restric
     wq[q] = weights[p];
 }
 
-// The "xform" processor's resampling (xform_sample) of n particles into P x P images.
+// The "xform" processor's resampling (xform_sample) of n particles (edge means or null) into P x P images.
 __global__ void __launch_bounds__(256) k_xform2d(const float *__restrict__ imgs, int B, int P, int off,
                                                  const float *__restrict__ means, const float *__restrict__ xf,
                                                  float *__restrict__ out)
@@ -66,7 +66,7 @@ __global__ void __launch_bounds__(256) k_xform2d(const float *__restrict__ imgs,
     if (idx >= P * P) return;
     const int i = idx % P, j = idx / P;
     out[(size_t)p * P * P + idx] =
-        xform_sample(imgs + (size_t)p * B * B, B, P, off, means[p], xf + 6 * (size_t)p, i, j);
+        xform_sample(imgs + (size_t)p * B * B, B, P, off, means ? means[p] : 0.f, xf + 6 * (size_t)p, i, j);
 }
 
 hipError_t launch_xform2d(const float *imgs, int n, int B, int P, const float *means, const float *xf, float *out,
