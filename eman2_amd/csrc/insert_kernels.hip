@@ -6,8 +6,10 @@
 // hypot3sq (libEM/util.cpp:788-800, util.h:816-819) and
 // EMData::add_complex_at_fast (libEM/emdata_core.h:368-413).  The float
 // arithmetic of coordinates and weights is evaluated in the reference's
-// order with contraction off, so every contribution is bit-identical to the
-// reference's; only the order of the FP32 sums differs.
+// order with contraction off, so a weight is the reference's bit for bit; the
+// brick scatters fuse a value's last product into its FP32 sum, and the order
+// of the sums differs.  The 6-cell Gaussians multiply value and weight first
+// and take gauss_var's width by Newton steps (k_scatter_gauss6).
 //
 //  k_insert_corners  one launch per (slice, symmetry op), one thread per pixel
 //                    and corner, global atomics per contribution (the plain
@@ -21,7 +23,7 @@
 //                    a stencil origin take turns, elected by an LDS tag).
 //                    Each item writes its partial brick to HBM.
 //  k_reduce_items    the items of a brick summed into its first one, where
-//                    the batch has more than about two per brick.
+//                    the batch has an item per brick of the grid or more.
 //  k_merge_partials  one thread per half-volume voxel sums the partial
 //                    bricks of its unfolded source cells under the Hermitian
 //                    fold of add_complex_at_fast and adds them with plain
@@ -1110,18 +1112,19 @@ __device__ __forceinline__ unsigned pack_index(unsigned x, unsigned y, unsigned 
 // double sums per particle accumulated with float64 atomics into acc[p][8].
 // vol: the volume as float4 (re, im, weight, 0) per voxel, or null, then data
 // and norm are read.  n3: the low-resolution band is 9 < x^2 + y^2 < n3.
-// Bound: VALU (0.24 instructions per SIMD and clock at pad 600), then the
-// volume's cache lines.  8,000
-// slices at pad 600: 36.5 ms before, 23.8 now.  What it took: the voxels read
-// before the patch is staged and at most 80 registers (3 workgroups of 8 waves
-// per CU; 34 ms with 2), the packed volume in 2^3 cubes (0.60 G instead of
-// 0.92 G line misses; data and weights read apart: 33.4 ms), offsets in groups
-// of four so that their LDS reads overlap, 32 x 32 tiles (halo 1.27 instead of
-// 1.41).  1,500 particles of d2 at pad 192: 7.1 -> 5.6 ms, the other planes'
-// gather by full waves (with the volume as it is 5.7).  The whole call 5.8 ms
-// with their sums in double; 5.9 with float atomics, whose order showed in the
-// results; 7.6 plane by plane without atomics, the waves half empty (300
-// particles of d7: 7.0, 7.7 and 13.6).
+// Bound: latency.  At pad 600 0.24 VALU instructions per SIMD and clock, 0.48
+// of the published vector rate (k_scatter_gauss6 reaches 0.70), the LDS busy
+// 38 %, 5.2 waves per SIMD resident: a gather is a chain of patch read, table
+// read and sum.  With symmetry 0.14 at 2.6 waves.  8,000 slices at pad 600:
+// 36.5 ms before, 23.7 now.  What it took: the voxels read before the patch is
+// staged and at most 80 registers (3 workgroups of 8 waves per CU; 34 ms with
+// 2), the packed volume in 2^3 cubes (0.60 G instead of 0.92 G line misses;
+// data and weights read apart: 33.4 ms), offsets in groups of four so that
+// their LDS reads overlap, 32 x 32 tiles (halo 1.27 instead of 1.41).  1,500
+// particles of d2 at pad 192: 7.1 -> 5.5 ms, the other planes' gather by full
+// waves.  The whole call 5.8 ms with their sums in double; 5.9 with float
+// atomics, whose order showed in the results; 7.6 plane by plane without
+// atomics, the waves half empty (300 particles of d7: 7.0, 7.7 and 13.6).
 template <int MODE, bool SYM, bool PACKED>
 __global__ void __launch_bounds__(AgreeTile<SYM ? 16 : 32>::THREADS) __attribute__((amdgpu_waves_per_eu(SYM ? 5 : 6)))
     k_agree_batch(const float2 *__restrict__ slices, int nsym, const float *__restrict__ t3d, const float *__restrict__ wq,
