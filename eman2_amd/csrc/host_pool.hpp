@@ -130,7 +130,7 @@ class HostPool {
 public:
     using Ref = std::shared_ptr<HostPool>;
     static constexpr size_t KEEP_DEVICE = 8ull << 30, KEEP_STREAMS = 16, KEEP_PINNED = 4;
-    static constexpr size_t SMALL_COPIES = 8;      // of less than a slot, before the pool's first ring
+    static constexpr size_t SMALL_BYTES = 64u << 20;  // in copies of less than a slot, before the pool's first ring
     static constexpr size_t LARGE = 32ull << 20;  // from here on a block is kept by what the device has left
     static constexpr size_t PIN_SLOTS = 4, PIN_SLOT = 16u << 20;  // a staging ring: 4 slots of 16 MB
 
@@ -296,10 +296,11 @@ public:
         (void)hipStreamDestroy(s);
     }
 
-    // A staging ring for a copy of `bytes`, or null where the runtime's own copy is the better one: the ring's
-    // memory and the copy threads take 1 to 2 ms to set up and take down, as much as some eight small copies
-    // gain from them, and a pool of one short-lived handle makes two (a volume of pad 96 from create to
-    // destroy: 1.2 ms, 3.3 with a ring for every pool).
+    // A staging ring for a copy of `bytes`, or null where the runtime's own copy is the better one.  The first
+    // ring's memory and the copy threads take 2 to 3 ms to set up, fault in and take down, what copies of below
+    // a slot gain from them over some 64 MB (0.03 to 0.09 ms per MB); the pool of a short-lived handle makes
+    // fewer (a volume of pad 96 from create to destroy: 1.2 ms, 3.3 with a ring for every pool).  No more than
+    // the kept rings for such copies: more of several threads would be set up and taken down each time.
     char *pinned(size_t bytes) noexcept
     {
         {
@@ -309,11 +310,17 @@ public:
                 pinned_.pop_back();
                 return p;
             }
-            if (bytes < PIN_SLOT && ++small_ <= SMALL_COPIES) return nullptr;
+            if (bytes < PIN_SLOT) {
+                small_ = std::min(small_ + bytes, SMALL_BYTES);
+                if (small_ < SMALL_BYTES || rings_ >= KEEP_PINNED) return nullptr;
+            }
+            rings_++;
         }
         void *p = nullptr;
         if (hipHostMalloc(&p, PIN_SLOTS * PIN_SLOT, hipHostMallocDefault) == hipSuccess) return static_cast<char *>(p);
         (void)hipGetLastError();
+        std::lock_guard<std::mutex> lk(mu_);
+        rings_--;
         return nullptr;
     }
 
@@ -325,6 +332,7 @@ public:
                 pinned_.push_back(p);
                 return;
             }
+            rings_--;
         }
         (void)hipHostFree(p);
     }
@@ -385,7 +393,8 @@ private:
     std::map<const void *, std::pair<int, long long>> limits_;  // by owner: device, bytes
     std::vector<std::pair<int, hipStream_t>> streams_;
     std::vector<char *> pinned_;
-    size_t small_ = 0;  // copies that found no ring
+    size_t rings_ = 0;  // in use and idle
+    size_t small_ = 0;  // bytes of small copies that found no ring
 };
 
 }  // namespace fh

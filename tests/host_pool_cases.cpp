@@ -229,17 +229,27 @@ static void waiting_free()
     CHECK(later);
 }
 
-// a pool's first small copies take no ring, large ones do; one that is there is taken by all
+// a pool's first small copies take no ring, large ones do; one that is there is taken by all; small copies
+// take no more rings than are kept
 static void rings()
 {
     auto p = HostPool::get();
-    for (size_t i = 0; i < HostPool::SMALL_COPIES; i++) CHECK(!p->pinned(4 * MB));
+    for (size_t i = 0; i + 1 < HostPool::SMALL_BYTES / (4 * MB); i++) CHECK(!p->pinned(4 * MB));
     char *a = p->pinned(4 * MB), *b = p->pinned(4 * MB);
     CHECK(a && b && a != b);
     p->give_pinned(a);
     CHECK(p->pinned(4 * MB) == a);
+    std::vector<char *> more;
+    for (size_t i = 2; i < HostPool::KEEP_PINNED; i++) more.push_back(p->pinned(4 * MB));
+    CHECK(!p->pinned(4 * MB));
+    more.push_back(p->pinned(HostPool::PIN_SLOT));
+    for (char *c : more) {
+        CHECK(c);
+        p->give_pinned(c);
+    }
     p->give_pinned(a);
     p->give_pinned(b);
+    CHECK(stub::hosts.size() == HostPool::KEEP_PINNED);
     p.reset();
     CHECK(stub::hosts.empty());
     p = HostPool::get();
