@@ -1,5 +1,5 @@
-"""Copies to the host through the staging ring, which a pool sets up after its
-first small copies: with a handle that has made them, volumes come back byte
+"""Copies to the host through the staging ring, which a pool sets up for a
+copy of 16 MB or after its first small ones: with a handle that has made one, volumes come back byte
 for byte at sizes around the thresholds (64 KB, the 512 KB smallest chunk, 16
 MB slots and a ring's four), from one thread and from several at once."""
 import threading
@@ -13,10 +13,9 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture
 def warm():
     from eman2_amd import Reconstructors
-    r = Reconstructors.get("fourier_hip", dict(size=(64, 64, 64)))
+    r = Reconstructors.get("fourier_hip", dict(size=(192, 192, 192)))
     r.setup()
-    for _ in range(10):
-        r.get_state()
+    r.get_state()                              # 28 MB and 14 MB
     return r
 
 
